@@ -33,6 +33,10 @@ DEVICE_SOURCES = [
     ("reduce.hip", ["-ffp-contract=off"]),
     ("unary.hip", ["-ffp-contract=off"]),
     ("gemm.hip", []),
+    ("gemm_tile_f32.hip", []),
+    ("gemm_tile_f64.hip", []),
+    ("gemm_tile_c64.hip", []),
+    ("gemm_tile_c128.hip", []),
     ("ozaki.hip", []),
     ("blas.hip", []),
 ]

@@ -1,5 +1,6 @@
-// GEMM on gfx950: FP64 MFMA DGEMM / ZGEMM, SIMT fallback for f32 and integers,
-// and the matmul entry point with rstsr's batch-broadcast rules.
+// GEMM on gfx950: the matmul entry point with rstsr's batch-broadcast rules, the dispatch to the
+// matrix-core tile kernel (gemm_tile.hpp: f32, f64, c64, c128) or the split GEMM (ozaki.hip), and
+// a SIMT kernel for integers.
 //
 // Replaces DeviceMatMulAPI for DeviceFaer (rstsr-core/src/device_faer/matmul.rs:
 // 19-239 -> faer) and the naive kernels of rstsr-native-impl/src/cpu_serial/
@@ -7,14 +8,6 @@
 // column stride) pairs directly, so no packing copy is made for any strided
 // operand (the OpenBLAS device packs non-BLAS layouts, crates-device/
 // rstsr-openblas/src/matmul_impl.rs:92-113; here the LDS tile load absorbs it).
-//
-// DGEMM tiling: 256 threads = 4 waves in a 2x2 grid; each wave owns a
-// (16*WM) x (16*WN) patch of C built from v_mfma_f64_16x16x4_f64 tiles. A and
-// B stage through LDS in BK=16 slices with a one-slice register prefetch, so
-// global loads of slice k+1 overlap the MFMAs of slice k. Global loads walk the
-// operand's unit-stride axis (template flags), so both row- and column-major
-// operands read coalesced. ZGEMM uses the same kernel with separate real and
-// imaginary LDS planes and four real MFMAs per complex tile (4M form).
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -32,12 +25,6 @@
 namespace rstsr {
 namespace hip {
 
-typedef double dbl4 __attribute__((ext_vector_type(4)));
-typedef double dbl2 __attribute__((ext_vector_type(2)));
-
-constexpr int GBK = 16;  // K slice held in LDS
-constexpr int GPAD = 4;  // LDS row padding (doubles)
-
 template <class T>
 struct GemmArgs {
     int64_t M, N, K;
@@ -51,268 +38,8 @@ struct GemmArgs {
     int beta_zero;
     uint32_t tiles_m, tiles_n;
     uint32_t batch0;  // first batch index of this launch
-    int tri;          // symmetric product: only the tiles with tm >= tn
     BatchDesc bd;
 };
-
-template <class T>
-struct CplxOf : std::false_type {};
-template <>
-struct CplxOf<c128> : std::true_type {};
-
-__device__ __forceinline__ double re_of(double x) { return x; }
-__device__ __forceinline__ double im_of(double) { return 0.0; }
-__device__ __forceinline__ double re_of(c128 x) { return x.re; }
-__device__ __forceinline__ double im_of(c128 x) { return x.im; }
-
-
-// Operands of one C tile's problem.
-template <class T>
-struct TileArgs {
-    int64_t M, N, K;
-    const T* A;
-    int64_t rsa, csa;
-    const T* B;
-    int64_t rsb, csb;
-    T* C;
-    int64_t rsc, csc;
-};
-
-// Block tile configuration: WVM x WVN waves, each owning FM x FN 16x16 output
-// tiles, so a block covers BM x BN = (16 WVM FM) x (16 WVN FN).
-// OCC: waves per SIMD the register budget is set for (the launch bound's second argument).
-template <int WVM_, int WVN_, int FM_, int FN_, int OCC_ = 2>
-struct MCfg {
-    static constexpr int WVM = WVM_, WVN = WVN_, FM = FM_, FN = FN_;
-    static constexpr int NT = 64 * WVM * WVN, BM = 16 * WVM * FM, BN = 16 * WVN * FN;
-    static constexpr int OCC = OCC_;
-};
-
-// LDS planes of one block (re/im planes for complex). Real types double-buffer
-// the K slices (one barrier per slice); complex tiles keep one buffer so that
-// two blocks still fit in a CU's LDS.
-template <class T, class CF>
-struct MfmaSmem {
-    static constexpr int NP = CplxOf<T>::value ? 2 : 1;
-    static constexpr int NB = CplxOf<T>::value ? 1 : 2;
-    double As[NB][NP][GBK][CF::BM + GPAD];
-    double Bs[NB][NP][GBK][CF::BN + GPAD];
-};
-
-// One BM x BN C tile: C = alpha * A B + beta * C (beta_zero: C not read).
-// A_MC: A's unit-stride axis is m (else k); B_KC: B's is k (else n). Each
-// thread loads VW consecutive elements along that axis per slot (VEC: two
-// doubles in one 16-byte load, which needs a +1 stride and 16-byte alignment).
-template <class T, class CF, bool A_MC, bool B_KC, bool VEC>
-__device__ __forceinline__ void mfma_tile(const TileArgs<T>& g, uint32_t tm, uint32_t tn, T alpha, T beta,
-                                          int beta_zero, MfmaSmem<T, CF>& sm) {
-    constexpr bool CX = CplxOf<T>::value;
-    constexpr int NP = MfmaSmem<T, CF>::NP;
-    constexpr int NT = CF::NT, BM = CF::BM, BN = CF::BN, FM = CF::FM, FN = CF::FN;
-    constexpr int VW = VEC ? 2 : 1;
-    static_assert(!VEC || !CX, "vector loads are for real operands");
-    // A slots: along m (A_MC) rows of BM/VW threads, KRA k-rows per pass; else
-    // along k rows of GBK/VW threads, RPA m-rows per pass. B likewise.
-    constexpr int TPA = A_MC ? BM / VW : GBK / VW, PPA = NT / TPA, LA = (A_MC ? GBK : BM) / PPA;
-    constexpr int TPB = B_KC ? GBK / VW : BN / VW, PPB = NT / TPB, LB = (B_KC ? BN : GBK) / PPB;
-    static_assert(NT % TPA == 0 && NT % TPB == 0 && LA >= 1 && LB >= 1 && (A_MC ? GBK : BM) % PPA == 0 &&
-                      (B_KC ? BN : GBK) % PPB == 0,
-                  "loader shape");
-    auto& As = sm.As;
-    auto& Bs = sm.Bs;
-    const T* A = g.A;
-    const T* B = g.B;
-    T* C = g.C;
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    // wave -> (row group, column group): waves w and w + 4 share a SIMD, so the column group is
-    // rotated by w / 4 to give each SIMD waves of different column groups as well as rows (an edge
-    // tile's padding then idles every SIMD alike)
-    const int wm = wave / CF::WVN, wn = (wave % CF::WVN + wave / 4) % CF::WVN;
-    const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
-
-    dbl4 acc[NP][FM][FN];
-#pragma unroll
-    for (int p = 0; p < NP; ++p)
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) acc[p][i][j] = dbl4{0.0, 0.0, 0.0, 0.0};
-
-    // slot i of this thread covers A(mm0 + i*dam + v*[A_MC], ka0 + i*dak + v*[!A_MC]), v < VW
-    constexpr int dam = A_MC ? 0 : PPA, dak = A_MC ? PPA : 0;
-    constexpr int dbk = B_KC ? 0 : PPB, dbn = B_KC ? PPB : 0;
-    const int mm0 = A_MC ? (tid % TPA) * VW : tid / TPA, ka0 = A_MC ? tid / TPA : (tid % TPA) * VW;
-    const int kb0 = B_KC ? (tid % TPB) * VW : tid / TPB, nn0 = B_KC ? tid / TPB : (tid % TPB) * VW;
-    const int64_t sa_i = dam * g.rsa + dak * g.csa, sb_i = dbk * g.rsb + dbn * g.csb;
-    const int64_t sa_v = A_MC ? g.rsa : g.csa, sb_v = B_KC ? g.rsb : g.csb;
-    const T* pa = A + (m0 + mm0) * g.rsa + ka0 * g.csa;
-    const T* pb = B + kb0 * g.rsb + (n0 + nn0) * g.csb;
-    // interior tiles skip the bounds tests except in a partial last K slice
-    const bool interior = m0 + BM <= g.M && n0 + BN <= g.N;
-
-    T ra[LA][VW], rb[LB][VW];
-    auto load_slice = [&](int64_t k0) {
-        const int64_t oa = k0 * g.csa, ob = k0 * g.rsb;
-        if (interior && k0 + GBK <= g.K) {
-#pragma unroll
-            for (int i = 0; i < LA; ++i) {
-                const T* p = pa + oa + i * sa_i;
-                if constexpr (VEC) {
-                    const dbl2 w = *(const dbl2*)p;
-                    ra[i][0] = w[0];
-                    ra[i][VW - 1] = w[1];
-                } else {
-                    ra[i][0] = *p;
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < LB; ++i) {
-                const T* p = pb + ob + i * sb_i;
-                if constexpr (VEC) {
-                    const dbl2 w = *(const dbl2*)p;
-                    rb[i][0] = w[0];
-                    rb[i][VW - 1] = w[1];
-                } else {
-                    rb[i][0] = *p;
-                }
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < LA; ++i)
-#pragma unroll
-                for (int v = 0; v < VW; ++v) {
-                    const bool ok = m0 + mm0 + i * dam + (A_MC ? v : 0) < g.M && k0 + ka0 + i * dak + (A_MC ? 0 : v) < g.K;
-                    ra[i][v] = ok ? pa[oa + i * sa_i + v * sa_v] : T{};
-                }
-#pragma unroll
-            for (int i = 0; i < LB; ++i)
-#pragma unroll
-                for (int v = 0; v < VW; ++v) {
-                    const bool ok = k0 + kb0 + i * dbk + (B_KC ? v : 0) < g.K && n0 + nn0 + i * dbn + (B_KC ? 0 : v) < g.N;
-                    rb[i][v] = ok ? pb[ob + i * sb_i + v * sb_v] : T{};
-                }
-        }
-    };
-    auto store_slice = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < LA; ++i)
-#pragma unroll
-            for (int v = 0; v < VW; ++v) {
-                const int kk = ka0 + i * dak + (A_MC ? 0 : v), mm = mm0 + i * dam + (A_MC ? v : 0);
-                As[buf][0][kk][mm] = re_of(ra[i][v]);
-                if constexpr (CX) As[buf][NP - 1][kk][mm] = im_of(ra[i][v]);
-            }
-#pragma unroll
-        for (int i = 0; i < LB; ++i)
-#pragma unroll
-            for (int v = 0; v < VW; ++v) {
-                const int kk = kb0 + i * dbk + (B_KC ? v : 0), nn = nn0 + i * dbn + (B_KC ? 0 : v);
-                Bs[buf][0][kk][nn] = re_of(rb[i][v]);
-                if constexpr (CX) Bs[buf][NP - 1][kk][nn] = im_of(rb[i][v]);
-            }
-    };
-
-    // 16 x 16 fragments of this wave that hold any row < M and column < N (the wave index is
-    // uniform, read through a scalar register so the tests below are scalar branches): edge
-    // tiles skip the MFMAs of fragments wholly in the padding
-    const int wv = __builtin_amdgcn_readfirstlane(wave);
-    const int64_t rows_left = g.M - (m0 + (wv / CF::WVN) * 16 * FM),
-                  cols_left = g.N - (n0 + ((wv % CF::WVN + wv / 4) % CF::WVN) * 16 * FN);
-    const int fmv = rows_left <= 0 ? 0 : (int)std::min<int64_t>(FM, (rows_left + 15) / 16);
-    const int fnv = cols_left <= 0 ? 0 : (int)std::min<int64_t>(FN, (cols_left + 15) / 16);
-
-    load_slice(0);
-    store_slice(0);
-    __syncthreads();
-    const int fr = lane & 15, fk = lane >> 4;
-    int buf = 0;
-    for (int64_t k0 = 0; k0 < g.K; k0 += GBK) {
-        const bool more = k0 + GBK < g.K;
-        if (more) load_slice(k0 + GBK);
-#pragma unroll
-        for (int kk = 0; kk < GBK; kk += 4) {
-            double fa[NP][FM], fb[NP][FN];
-#pragma unroll
-            for (int i = 0; i < FM; ++i) {
-                fa[0][i] = As[buf][0][kk + fk][wm * 16 * FM + i * 16 + fr];
-                if constexpr (CX) fa[NP - 1][i] = As[buf][NP - 1][kk + fk][wm * 16 * FM + i * 16 + fr];
-            }
-#pragma unroll
-            for (int j = 0; j < FN; ++j) {
-                fb[0][j] = Bs[buf][0][kk + fk][wn * 16 * FN + j * 16 + fr];
-                if constexpr (CX) fb[NP - 1][j] = Bs[buf][NP - 1][kk + fk][wn * 16 * FN + j * 16 + fr];
-            }
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j) {
-                    if (i >= fmv || j >= fnv) continue;
-                    if constexpr (!CX) {
-                        acc[0][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[0][i], fb[0][j], acc[0][i][j], 0, 0, 0);
-                    } else {
-                        // re += ar*br - ai*bi ; im += ar*bi + ai*br
-                        acc[0][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[0][i], fb[0][j], acc[0][i][j], 0, 0, 0);
-                        acc[0][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(-fa[1][i], fb[1][j], acc[0][i][j], 0, 0, 0);
-                        acc[1][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[0][i], fb[1][j], acc[1][i][j], 0, 0, 0);
-                        acc[1][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[1][i], fb[0][j], acc[1][i][j], 0, 0, 0);
-                    }
-                }
-        }
-        if constexpr (MfmaSmem<T, CF>::NB == 2) {
-            // the other buffer was last read before the previous barrier
-            if (more) store_slice(buf ^ 1);
-            __syncthreads();
-            buf ^= 1;
-        } else {
-            __syncthreads();
-            if (more) {
-                store_slice(0);
-                __syncthreads();
-            }
-        }
-    }
-    // epilogue: v_mfma_f64_16x16x4f64 leaves register r of lane l at row 4*r + l/16,
-    // column l%16 of its 16x16 tile
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                int64_t gm = m0 + wm * 16 * FM + i * 16 + 4 * r + (lane >> 4);
-                int64_t gn = n0 + wn * 16 * FN + j * 16 + (lane & 15);
-                if (gm < g.M && gn < g.N) {
-                    T* cp = C + gm * g.rsc + gn * g.csc;
-                    if constexpr (!CX) {
-                        double v = alpha * acc[0][i][j][r];
-                        if (!beta_zero) v += beta * (*cp);
-                        *cp = v;
-                    } else {
-                        double xr = acc[0][i][j][r], xi = acc[1][i][j][r];
-                        c128 v{alpha.re * xr - alpha.im * xi, alpha.re * xi + alpha.im * xr};
-                        if (!beta_zero) {
-                            c128 o = *cp;
-                            v.re += beta.re * o.re - beta.im * o.im;
-                            v.im += beta.re * o.im + beta.im * o.re;
-                        }
-                        *cp = v;
-                    }
-                }
-            }
-}
-
-// Index t of the lower triangle (diag = 0: i >= j, t = i(i+1)/2 + j; diag = 1:
-// i > j, t = i(i-1)/2 + j) -> (i, j). The floating root is corrected exactly.
-__device__ __forceinline__ void tri_coords(uint32_t t, int diag, uint32_t& i, uint32_t& j) {
-    auto first = [&](uint64_t r) { return diag ? r * (r - 1) / 2 : r * (r + 1) / 2; };
-    uint64_t r = (uint64_t)((diag ? 1.0 + sqrt(1.0 + 8.0 * t) : sqrt(1.0 + 8.0 * t) - 1.0) * 0.5);
-    while (r > 0 && first(r) > t) --r;
-    while (first(r + 1) <= t) ++r;
-    i = (uint32_t)r;
-    j = (uint32_t)(t - first(r));
-}
 
 // Symmetric product (A = B^T, same buffer): copy the transpose of every 64 x 64
 // tile on and below the diagonal onto its mirror, through LDS so both the reads
@@ -341,84 +68,7 @@ __global__ void __launch_bounds__(256) k_mirror(GemmArgs<T> g) {
     }
 }
 
-// Strided-batched GEMM: one C tile per block, batch index from blockIdx.y.
-// run_if (nullable): the whole grid exits unless *run_if != 0 (device-side
-// selection between alternative paths without a host round trip).
-template <class T, class CF, bool A_MC, bool B_KC, bool VEC>
-__global__ void __launch_bounds__(CF::NT, CF::OCC) k_gemm_mfma(GemmArgs<T> g, const int* run_if) {
-    if (run_if && *run_if == 0) return;
-    __shared__ MfmaSmem<T, CF> sm;
-    uint32_t tm, tn;
-    if (g.tri) tri_coords(xcd_remap8(blockIdx.x, g.tiles_m * (g.tiles_m + 1) / 2), 0, tm, tn);
-    else tile_coords<8>(blockIdx.x, g.tiles_m, g.tiles_n, tm, tn);
-    int64_t boa, bob, boc;
-    batch_offsets(g.bd, g.batch0 + blockIdx.y, boa, bob, boc);
-    TileArgs<T> t{g.M, g.N, g.K, g.a + boa, g.rsa, g.csa, g.b + bob, g.rsb, g.csb, g.c + boc, g.rsc, g.csc};
-    mfma_tile<T, CF, A_MC, B_KC, VEC>(t, tm, tn, g.alpha, g.beta, g.beta_zero, sm);
-}
-
-// Grouped (uneven) GEMMs in one persistent launch. Problem g owns tiles
-// [prefix[g], prefix[g+1]); blocks stride over all tiles. flags bit0: A
-// m-contiguous, bit1: B k-contiguous, bit2: 16-byte loads (selects the loader).
-template <class T>
-struct GroupProblem {
-    TileArgs<T> t;
-    uint32_t tiles_n;
-    uint32_t flags;
-};
-
-// VM: bit f set for each loader form f (GroupProblem::flags) the launch holds; a kernel with fewer
-// forms holds fewer inlined tile loops, so it needs fewer registers
-template <class T, class CF, uint32_t VM = 31>
-__global__ void __launch_bounds__(CF::NT, CF::OCC) k_gemm_grouped(const GroupProblem<T>* __restrict__ probs, int count,
-                                                                  const uint32_t* __restrict__ prefix, uint32_t total,
-                                                                  T alpha, T beta, int beta_zero,
-                                                                  const int* __restrict__ run_if,
-                                                                  uint32_t* __restrict__ queue) {
-    if (run_if && *run_if == 0) return;
-    __shared__ MfmaSmem<T, CF> sm;
-    __shared__ uint32_t next_tile;
-    constexpr bool RV = !CplxOf<T>::value;  // vector loads exist for real operands
-    // tiles handed out in order: block b starts with tile b, then takes the next unclaimed one
-    // from the queue counter (zero at launch), claimed while its current tile computes
-    for (uint32_t tile = blockIdx.x; tile < total;) {
-        uint32_t claimed = 0;
-        if (threadIdx.x == 0) claimed = atomicAdd(queue, 1u) + gridDim.x;
-        // problem of this tile: last g with prefix[g] <= tile
-        int lo = 0, hi = count - 1;
-        while (lo < hi) {
-            int mid = (lo + hi + 1) >> 1;
-            if (prefix[mid] <= tile) lo = mid;
-            else hi = mid - 1;
-        }
-        const GroupProblem<T> gp = probs[lo];
-        const uint32_t local = tile - prefix[lo];
-        const uint32_t tm = local / gp.tiles_n, tn = local - (local / gp.tiles_n) * gp.tiles_n;
-        switch (gp.flags & 7) {
-            case 3:
-                if constexpr ((VM & 8) != 0) mfma_tile<T, CF, true, true, false>(gp.t, tm, tn, alpha, beta, beta_zero, sm);
-                break;
-            case 1:
-                if constexpr ((VM & 2) != 0) mfma_tile<T, CF, true, false, false>(gp.t, tm, tn, alpha, beta, beta_zero, sm);
-                break;
-            case 2:
-                if constexpr ((VM & 4) != 0) mfma_tile<T, CF, false, true, false>(gp.t, tm, tn, alpha, beta, beta_zero, sm);
-                break;
-            case 4:
-                if constexpr (RV && (VM & 16) != 0) mfma_tile<T, CF, false, false, RV>(gp.t, tm, tn, alpha, beta, beta_zero, sm);
-                break;
-            default:
-                if constexpr ((VM & 1) != 0) mfma_tile<T, CF, false, false, false>(gp.t, tm, tn, alpha, beta, beta_zero, sm);
-                break;
-        }
-        if (threadIdx.x == 0) next_tile = claimed;
-        __syncthreads();  // LDS reuse by the next tile; next_tile visible
-        tile = next_tile;
-        __syncthreads();  // every thread has read next_tile before it is written again
-    }
-}
-
-/* ---------------- SIMT fallback: f32, i32, i64, c64 ---------------- */
+/* ---------------- SIMT kernel: i32, i64 ---------------- */
 
 template <class T>
 __device__ __forceinline__ T g_mul(T a, T b) {
@@ -475,106 +125,15 @@ __global__ void __launch_bounds__(256) k_gemm_simt(GemmArgs<T> g) {
 
 /* ---------------- host side ---------------- */
 
-/* ---------------- tile configurations and the autotuner ---------------- */
-
-// MFMA tile configurations: (WM, WN) -> block tile (32*WM) x (32*WN).
-// Candidate tile configurations, in the autotuner's candidate order.
-using D0 = MCfg<4, 2, 2, 4>;  // f64 128 x 128, 8 waves of 32 x 64
-using D1 = MCfg<4, 4, 2, 2>;  // f64 128 x 128, 16 waves of 32 x 32
-using D2 = MCfg<2, 2, 4, 4>;  // f64 128 x 128, 4 waves of 64 x 64
-using D3 = MCfg<2, 2, 2, 2>;  // f64 64 x 64, 4 waves of 32 x 32 (small outputs)
-using D4 = MCfg<4, 2, 2, 2, 4>;  // f64 128 x 64, 8 waves of 32 x 32, two blocks per CU (grouped only)
-using Z0 = MCfg<2, 2, 2, 4>;  // c128 64 x 128, 4 waves of 32 x 64
-using Z1 = MCfg<2, 2, 2, 2>;  // c128 64 x 64
-using Z2 = MCfg<2, 4, 2, 2>;  // c128 64 x 128, 8 waves of 32 x 32
-constexpr int NCAND_D = 4, NCAND_Z = 3;
-
-// The autotuner (tune_select, api.cpp) times every candidate configuration once
-// per problem class (sizes bucketed to powers of two, layout flags, batch bucket)
-// on the real call and keeps the fastest. Timing runs only when C is write-only
-// (beta == 0) and the stream is not being captured; otherwise the cached choice
-// or the size heuristic is used. RSTSR_HIP_TUNE_CACHE=<file> persists choices.
-static int bucket(int64_t x) {
-    int b = 0;
-    while ((1ll << b) < x) ++b;
-    return b;
-}
-
-// run(c) performs the whole call with configuration c. Returns the chosen index.
-template <class F>
-static int tuned_run(rstsr_hip_ctx* ctx, const std::string& key, int ncand, int heuristic, bool can_time, F&& run) {
-    return tune_select(ctx, key, ncand, heuristic, can_time, std::function<void(int)>(run));
-}
-
-template <class T, class CF>
-static void launch_mfma_cfg(rstsr_hip_ctx* ctx, GemmArgs<T> g, uint32_t nb, bool amc, bool bkc, bool vec,
-                            const int* run_if) {
-    g.tiles_m = ceil_div_u32(g.M, CF::BM);
-    g.tiles_n = ceil_div_u32(g.N, CF::BN);
-    uint64_t nt = (uint64_t)g.tiles_m * g.tiles_n;
-    if (g.tri) {
-        if (CF::BM != CF::BN || g.M != g.N) RSTSR_RAISE(RuntimeError, "symmetric product needs square tiles");
-        nt = (uint64_t)g.tiles_m * (g.tiles_m + 1) / 2;
-    }
-    if (nt >= (1ull << 31)) RSTSR_RAISE(UnImplemented, "GEMM grid too large");
-    dim3 grid((uint32_t)nt, nb), blk(CF::NT);
-    auto go = [&](auto a_mc, auto b_kc, auto v) {
-        hipLaunchKernelGGL((k_gemm_mfma<T, CF, decltype(a_mc)::value, decltype(b_kc)::value, decltype(v)::value>), grid,
-                           blk, 0, ctx->stream, g, run_if);
-    };
-    using F = std::false_type;
-    using Tr = std::true_type;
-    if constexpr (!CplxOf<T>::value) {
-        if (vec) {
-            if (amc && bkc) go(Tr{}, Tr{}, Tr{});
-            else if (amc) go(Tr{}, F{}, Tr{});
-            else if (bkc) go(F{}, Tr{}, Tr{});
-            else go(F{}, F{}, Tr{});
-            check_launch("gemm");
-            return;
-        }
-    }
-    if (amc && bkc) go(Tr{}, Tr{}, F{});
-    else if (amc) go(Tr{}, F{}, F{});
-    else if (bkc) go(F{}, Tr{}, F{});
-    else go(F{}, F{}, F{});
-    check_launch("gemm");
-}
-
+// Copy the lower triangle of nb batches (from g.batch0) onto the upper one.
 template <class T>
-static void launch_mfma_any(rstsr_hip_ctx* ctx, int c, const GemmArgs<T>& g, uint32_t nb, bool amc, bool bkc,
-                            bool vec, const int* run_if) {
-    if constexpr (std::is_same<T, double>::value) {
-        switch (c) {
-            case 0: return launch_mfma_cfg<T, D0>(ctx, g, nb, amc, bkc, vec, run_if);
-            case 1: return launch_mfma_cfg<T, D1>(ctx, g, nb, amc, bkc, vec, run_if);
-            case 2: return launch_mfma_cfg<T, D2>(ctx, g, nb, amc, bkc, vec, run_if);
-            default: return launch_mfma_cfg<T, D3>(ctx, g, nb, amc, bkc, vec, run_if);
-        }
-    } else {
-        switch (c) {
-            case 0: return launch_mfma_cfg<T, Z0>(ctx, g, nb, amc, bkc, vec, run_if);
-            case 1: return launch_mfma_cfg<T, Z1>(ctx, g, nb, amc, bkc, vec, run_if);
-            default: return launch_mfma_cfg<T, Z2>(ctx, g, nb, amc, bkc, vec, run_if);
-        }
-    }
-}
-
-template <class T>
-static int heuristic_cfg(int64_t m, int64_t n) {
-    int64_t s = std::min(m, n);
-    if constexpr (std::is_same<T, double>::value) return s >= 128 ? 0 : 3;
-    else return s >= 128 ? 0 : 1;
-}
-
-// Two-double loads along an operand's unit-stride axis: the stride along it is
-// +1, the other matrix stride and every batch stride are even, and the base is
-// 16-byte aligned, so every tile-aligned element pair is one aligned 16-byte word.
-static bool pair_loads_ok(const void* p, int64_t unit, int64_t other, const int64_t* bs, int nbd) {
-    if (unit != 1 || other % 2 != 0 || ((uintptr_t)p & 15) != 0) return false;
-    for (int d = 0; d < nbd; ++d)
-        if (bs[d] % 2 != 0) return false;
-    return true;
+static void mirror_batches(rstsr_hip_ctx* ctx, const GemmArgs<T>& g, uint32_t nb) {
+    const uint64_t t64 = ceil_div_u32(g.M, 64);
+    const uint64_t nm = t64 * (t64 + 1) / 2;
+    if (nm >= (1ull << 31)) RSTSR_RAISE(UnImplemented, "symmetric product too large");
+    if (nm == 0) return;
+    hipLaunchKernelGGL(k_mirror<T>, dim3((uint32_t)nm, nb), dim3(256), 0, ctx->stream, g);
+    check_launch("gemm mirror");
 }
 
 template <class T>
@@ -596,52 +155,24 @@ static void launch_gemm_t(rstsr_hip_ctx* ctx, const GemmProblem& P, T alpha, T b
     g.alpha = alpha;
     g.beta = beta;
     g.beta_zero = beta_zero ? 1 : 0;
-    g.tri = 0;
     g.bd = P.bd;
-    const uint64_t YMAX = 65535;
-    constexpr bool MF = std::is_same<T, double>::value || std::is_same<T, c128>::value;
-    if constexpr (MF) {
-        constexpr bool CX = std::is_same<T, c128>::value;
-        const int ncand = CX ? NCAND_Z : NCAND_D;
-        bool amc = std::llabs(P.rsa) == 1 && std::llabs(P.csa) != 1;
-        bool bkc = std::llabs(P.rsb) == 1 && std::llabs(P.csb) != 1;
-        const bool vec = !CX && pair_loads_ok(P.a, amc ? P.rsa : P.csa, amc ? P.csa : P.rsa, P.bd.sa, P.bd.nbd) &&
-                         pair_loads_ok(P.b, bkc ? P.rsb : P.csb, bkc ? P.csb : P.rsb, P.bd.sb, P.bd.nbd);
+    if constexpr (!std::is_integral<T>::value) {
         // SYRK shortcut (device_faer/matmul.rs:38-48): beta = 0 and A is B's transpose
         // in the same buffer, so C is symmetric. Only the tiles on and below the
         // diagonal are multiplied; the rest is mirrored. For real types C[i][j] and
         // C[j][i] sum the same products in the same K order, so the mirror equals the
         // full product bit for bit; for complex the imaginary part's two products
         // swap order, and the mirror makes the result exactly symmetric.
-        bool syrk = beta_zero && run_if == nullptr && P.a == P.b && P.M == P.N && P.rsa == P.csb && P.csa == P.rsb;
-        for (int d = 0; d < P.bd.nbd && syrk; ++d) syrk = P.bd.sa[d] == P.bd.sb[d];
-        // square candidates only (complex: the 64 x 64 tile)
-        const int ncand_s = syrk ? (CX ? 1 : ncand) : ncand;
-        auto cand = [&](int c) { return syrk && CX ? 1 : c; };
-        auto run = [&](int c) {
-            for (uint64_t b0 = 0; b0 < P.nbatch; b0 += YMAX) {
-                GemmArgs<T> gg = g;
-                gg.batch0 = (uint32_t)b0;
-                gg.tri = syrk ? 1 : 0;
-                uint32_t nb = (uint32_t)std::min<uint64_t>(YMAX, P.nbatch - b0);
-                launch_mfma_any<T>(ctx, cand(c), gg, nb, amc, bkc, vec, run_if);
-                if (syrk) {
-                    const uint64_t t64 = ceil_div_u32(P.M, 64);
-                    const uint64_t nm = t64 * (t64 + 1) / 2;
-                    if (nm >= (1ull << 31)) RSTSR_RAISE(UnImplemented, "symmetric product too large");
-                    if (nm > 0) {
-                        hipLaunchKernelGGL(k_mirror<T>, dim3((uint32_t)nm, nb), dim3(256), 0, ctx->stream, gg);
-                        check_launch("gemm mirror");
-                    }
-                }
-            }
+        auto mirror = [&](uint64_t b0, uint32_t nb) {
+            g.batch0 = (uint32_t)b0;
+            mirror_batches<T>(ctx, g, nb);
         };
-        char key[160];
-        std::snprintf(key, sizeof(key), "gemm:%s:m%d:n%d:k%d:b%d:f%d", CX ? "z" : "d", bucket(P.M), bucket(P.N),
-                      bucket(P.K), bucket((int64_t)P.nbatch),
-                      (amc ? 1 : 0) | (bkc ? 2 : 0) | (vec ? 4 : 0) | (syrk ? 8 : 0));
-        tuned_run(ctx, key, ncand_s, syrk && CX ? 0 : heuristic_cfg<T>(P.M, P.N), beta_zero && run_if == nullptr, run);
+        if constexpr (std::is_same<T, float>::value) tile_gemm_f32(ctx, P, alpha, beta, beta_zero, mirror);
+        else if constexpr (std::is_same<T, c64>::value) tile_gemm_c64(ctx, P, alpha, beta, beta_zero, mirror);
+        else if constexpr (std::is_same<T, double>::value) tile_gemm_f64(ctx, P, alpha, beta, beta_zero, run_if, mirror);
+        else tile_gemm_c128(ctx, P, alpha, beta, beta_zero, run_if, mirror);
     } else {
+        const uint64_t YMAX = 65535;
         for (uint64_t b0 = 0; b0 < P.nbatch; b0 += YMAX) {
             uint32_t nb = (uint32_t)std::min<uint64_t>(YMAX, P.nbatch - b0);
             g.batch0 = (uint32_t)b0;
@@ -660,111 +191,6 @@ void plain_dgemm(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, double 
     launch_gemm_t<double>(ctx, P, alpha, beta, beta_zero, run_if);
 }
 
-
-/* ---------------- grouped GEMM ---------------- */
-
-template <class T, class CF>
-static void launch_grouped_cfg(rstsr_hip_ctx* ctx, const std::vector<TileArgs<T>>& probs, T alpha, T beta,
-                               bool beta_zero, const int* run_if = nullptr) {
-    std::vector<GroupProblem<T>> gp(probs.size());
-    std::vector<uint32_t> prefix(probs.size() + 1, 0);
-    // Tiles are handed out in problem order to blocks that stride over them: longest K
-    // (the time of one tile) first, so that short tiles fill the end of the launch
-    // instead of a few long ones trailing it. Each problem writes only its own C, so the
-    // order changes no result.
-    std::vector<size_t> order(probs.size());
-    for (size_t i = 0; i < order.size(); ++i) order[i] = i;
-    std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return probs[x].K > probs[y].K; });
-    uint64_t total = 0;
-    uint32_t forms = 0;  // bit f: some problem loads with form f
-    for (size_t i = 0; i < probs.size(); ++i) {
-        const auto& t = probs[order[i]];
-        uint32_t tm = ceil_div_u32(t.M, CF::BM), tn = ceil_div_u32(t.N, CF::BN);
-        gp[i].t = t;
-        gp[i].tiles_n = tn;
-        bool amc = std::llabs(t.rsa) == 1 && std::llabs(t.csa) != 1;
-        bool bkc = std::llabs(t.rsb) == 1 && std::llabs(t.csb) != 1;
-        bool vec = !CplxOf<T>::value && !amc && !bkc && pair_loads_ok(t.A, t.csa, t.rsa, nullptr, 0) &&
-                   pair_loads_ok(t.B, t.csb, t.rsb, nullptr, 0);
-        gp[i].flags = vec ? 4u : ((amc ? 1u : 0u) | (bkc ? 2u : 0u));
-        forms |= 1u << gp[i].flags;
-        prefix[i] = (uint32_t)total;
-        total += (uint64_t)tm * tn;
-    }
-    prefix[probs.size()] = (uint32_t)total;
-    if (total == 0) return;
-    if (total >= (1ull << 31)) RSTSR_RAISE(UnImplemented, "grouped GEMM has too many tiles");
-    const size_t poff = (gp.size() * sizeof(GroupProblem<T>) + 255) & ~(size_t)255;
-    const size_t qoff = poff + prefix.size() * sizeof(uint32_t);  // the tile queue counter
-    const size_t bytes = qoff + sizeof(uint32_t);
-    char* meta = (char*)aux_buffer(ctx, bytes + 256);
-    char* host = (char*)meta_stage(ctx, bytes, "grouped GEMM");
-    std::memcpy(host, gp.data(), gp.size() * sizeof(GroupProblem<T>));
-    std::memcpy(host + poff, prefix.data(), prefix.size() * sizeof(uint32_t));
-    const uint32_t zero = 0;
-    std::memcpy(host + qoff, &zero, sizeof(zero));
-    meta_upload(ctx, meta, bytes);
-    auto launch = [&](auto vm) {
-        constexpr uint32_t VM = decltype(vm)::value;
-        // persistent grid: as many blocks as can be resident at once. The launch bound sets waves
-        // per SIMD, not blocks per CU, so the count comes from the occupancy query: a block beyond
-        // it would start only once the queue is empty and then run its first tile (one of the
-        // longest) alone.
-        static const int per_cu = [] {
-            int v = 0;
-            HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, k_gemm_grouped<T, CF, VM>, CF::NT, 0));
-            return std::max(v, 1);
-        }();
-        uint32_t grid = (uint32_t)std::min<uint64_t>(total, (uint64_t)std::max(ctx->num_cu, 1) * per_cu);
-        hipLaunchKernelGGL((k_gemm_grouped<T, CF, VM>), dim3(grid), dim3(CF::NT), 0, ctx->stream,
-                           (const GroupProblem<T>*)meta, (int)gp.size(), (const uint32_t*)(meta + poff),
-                           (uint32_t)total, alpha, beta, beta_zero ? 1 : 0, run_if, (uint32_t*)(meta + qoff));
-        check_launch("grouped gemm");
-    };
-    // every problem row-major in both operands (forms 0 and 4): the kernel with those two only
-    if ((forms & ~17u) == 0) launch(std::integral_constant<uint32_t, 17>{});
-    else launch(std::integral_constant<uint32_t, 31>{});
-}
-
-template <class T>
-static void grouped_t(rstsr_hip_ctx* ctx, const std::vector<TileArgs<T>>& probs, T alpha, T beta, bool beta_zero) {
-    if (probs.empty()) return;
-    constexpr bool CX = std::is_same<T, c128>::value;
-    double mean = 0;
-    for (auto& p : probs) mean += (double)std::min(p.M, p.N);
-    mean /= (double)probs.size();
-    int64_t tot_mnk = 0;
-    for (auto& p : probs) tot_mnk += p.M * p.N * p.K;
-    auto run = [&](int c) {
-        if constexpr (CX) {
-            if (c == 0) launch_grouped_cfg<T, Z2>(ctx, probs, alpha, beta, beta_zero);
-            else launch_grouped_cfg<T, Z1>(ctx, probs, alpha, beta, beta_zero);
-        } else {
-            if (c == 0) launch_grouped_cfg<T, D0>(ctx, probs, alpha, beta, beta_zero);
-            else if (c == 1) launch_grouped_cfg<T, D1>(ctx, probs, alpha, beta, beta_zero);
-            else if (c == 2) launch_grouped_cfg<T, D3>(ctx, probs, alpha, beta, beta_zero);
-            else launch_grouped_cfg<T, D4>(ctx, probs, alpha, beta, beta_zero);
-        }
-    };
-    char key[160];
-    std::snprintf(key, sizeof(key), "grouped:%s:n%d:mean%d:work%d", CX ? "z" : "d", bucket((int64_t)probs.size()),
-                  bucket((int64_t)mean), bucket(tot_mnk));
-    tuned_run(ctx, key, CX ? 2 : 4, mean >= 128 ? (CX ? 0 : 1) : (CX ? 1 : 2), beta_zero, run);
-}
-
-void plain_grouped_f64(rstsr_hip_ctx* ctx, const std::vector<GemmProblem>& probs, double alpha, double beta,
-                       bool beta_zero, const int* run_if) {
-    std::vector<TileArgs<double>> ta;
-    ta.reserve(probs.size());
-    for (auto& P : probs)
-        ta.push_back(TileArgs<double>{P.M, P.N, P.K, (const double*)P.a, P.rsa, P.csa, (const double*)P.b, P.rsb, P.csb,
-                                      (double*)P.c, P.rsc, P.csc});
-    if (ta.empty()) return;
-    // unconditional: the tuned configuration; conditional (a fallback inside a captured
-    // sequence): the fixed one, since the autotuner cannot time a launch that may not run
-    if (run_if) launch_grouped_cfg<double, D1>(ctx, ta, alpha, beta, beta_zero, run_if);
-    else grouped_t<double>(ctx, ta, alpha, beta, beta_zero);
-}
 
 // Zero-fill C (k == 0 with beta == 0: crates-device/rstsr-openblas/src/matmul_impl.rs:78-81).
 template <class T>
@@ -1241,16 +667,10 @@ int rstsr_hip_gemm_grouped(rstsr_hip_ctx_t* ctx, rstsr_dtype_t t, rstsr_gemm_mod
                 T al, be;
                 std::memcpy(&al, alpha, sizeof(T));
                 std::memcpy(&be, beta, sizeof(T));
-                std::vector<TileArgs<T>> ta;
-                for (auto& P : probs) {
-                    if (P.K == 0) {
-                        rest.push_back(P);
-                        continue;
-                    }
-                    ta.push_back(TileArgs<T>{P.M, P.N, P.K, (const T*)P.a, P.rsa, P.csa, (const T*)P.b, P.rsb, P.csb,
-                                             (T*)P.c, P.rsc, P.csc});
-                }
-                grouped_t<T>(ctx, ta, al, be, is_zero_scalar(t, beta));
+                std::vector<GemmProblem> gp;
+                for (auto& P : probs) (P.K == 0 ? rest : gp).push_back(P);
+                if constexpr (std::is_same<T, double>::value) tile_grouped_f64(ctx, gp, al, be, is_zero_scalar(t, beta), nullptr);
+                else tile_grouped_c128(ctx, gp, al, be, is_zero_scalar(t, beta), nullptr);
             };
             if (t == RSTSR_F64) go(double{});
             else go(c128{});

@@ -1,6 +1,7 @@
 // Shared GEMM problem description (gemm.hip, ozaki.hip).
 #pragma once
 
+#include <functional>
 #include <vector>
 
 #include "common.hpp"
@@ -49,6 +50,17 @@ __device__ __forceinline__ void tile_coords(uint32_t id, uint32_t tiles_m, uint3
     tn = r / gsz;
 }
 
+// Index t of the lower triangle (diag = 0: i >= j, t = i(i+1)/2 + j; diag = 1:
+// i > j, t = i(i-1)/2 + j) -> (i, j). The floating root is corrected exactly.
+__device__ __forceinline__ void tri_coords(uint32_t t, int diag, uint32_t& i, uint32_t& j) {
+    auto first = [&](uint64_t r) { return diag ? r * (r - 1) / 2 : r * (r + 1) / 2; };
+    uint64_t r = (uint64_t)((diag ? 1.0 + sqrt(1.0 + 8.0 * t) : sqrt(1.0 + 8.0 * t) - 1.0) * 0.5);
+    while (r > 0 && first(r) > t) --r;
+    while (first(r + 1) <= t) ++r;
+    i = (uint32_t)r;
+    j = (uint32_t)(t - first(r));
+}
+
 // Device offsets of batch `bi` (innermost batch axis first).
 __device__ __forceinline__ void batch_offsets(const BatchDesc& bd, uint32_t bi, int64_t& oa, int64_t& ob, int64_t& oc) {
     oa = ob = oc = 0;
@@ -76,6 +88,23 @@ inline void batch_offsets_host(const BatchDesc& bd, uint64_t bi, int64_t& oa, in
     }
 }
 
+// Copies the lower triangle onto the upper one for batches [b0, b0 + nb) of a symmetric product.
+using MirrorFn = std::function<void(uint64_t b0, uint32_t nb)>;
+// GEMM of one element type on the matrix cores (gemm_tile_*.hip). run_if (device, nullable): the
+// kernels exit unless *run_if != 0.
+void tile_gemm_f32(rstsr_hip_ctx* ctx, const GemmProblem& P, float alpha, float beta, bool beta_zero,
+                   const MirrorFn& mirror);
+void tile_gemm_c64(rstsr_hip_ctx* ctx, const GemmProblem& P, c64 alpha, c64 beta, bool beta_zero, const MirrorFn& mirror);
+void tile_gemm_f64(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, double beta, bool beta_zero,
+                   const int* run_if, const MirrorFn& mirror);
+void tile_gemm_c128(rstsr_hip_ctx* ctx, const GemmProblem& P, c128 alpha, c128 beta, bool beta_zero,
+                    const int* run_if, const MirrorFn& mirror);
+// Grouped (uneven) GEMMs in one persistent launch: problems without batches, with M, N, K > 0 and
+// outputs that do not overlap. The tile shape is the tuner's, or with run_if a fixed one.
+void tile_grouped_f64(rstsr_hip_ctx* ctx, const std::vector<GemmProblem>& probs, double alpha, double beta,
+                      bool beta_zero, const int* run_if);
+void tile_grouped_c128(rstsr_hip_ctx* ctx, const std::vector<GemmProblem>& probs, c128 alpha, c128 beta,
+                       bool beta_zero, const int* run_if);
 // Ozaki-II split GEMM for f64 (ozaki.hip). Falls back to the plain kernel for
 // non-finite inputs.
 void ozaki_gemm_f64(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, double beta, bool beta_zero);
@@ -87,10 +116,6 @@ void plain_dgemm(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, double 
 // Outputs must not overlap.
 void ozaki_grouped_f64(rstsr_hip_ctx* ctx, const std::vector<GemmProblem>& probs, double alpha, double beta,
                        bool beta_zero);
-// Plain grouped FP64 GEMM in one persistent launch (gemm.hip): the autotuned tile
-// shape, or with run_if (as for plain_dgemm) a fixed one.
-void plain_grouped_f64(rstsr_hip_ctx* ctx, const std::vector<GemmProblem>& probs, double alpha, double beta,
-                       bool beta_zero, const int* run_if);
 
 }  // namespace hip
 }  // namespace rstsr

@@ -1872,7 +1872,7 @@ void ozaki_grouped_f64(rstsr_hip_ctx* ctx, const std::vector<GemmProblem>& probs
             if (split_pays(P)) ozaki_gemm_f64(ctx, P, alpha, beta, beta_zero);
             else plain.push_back(P);
         }
-        plain_grouped_f64(ctx, plain, alpha, beta, beta_zero, nullptr);
+        tile_grouped_f64(ctx, plain, alpha, beta, beta_zero, nullptr);
         return;
     }
     // a K longer than one INT8 launch can sum goes through the single-problem path
@@ -1989,7 +1989,7 @@ void ozaki_grouped_f64(rstsr_hip_ctx* ctx, const std::vector<GemmProblem>& probs
                        eA, fB, A8, B8, (int64_t)sA, (int64_t)sB, su.ms, flag);
     check_launch("grouped ozaki split");
     // non-finite inputs anywhere in the group: the plain grouped kernel computes every product
-    plain_grouped_f64(ctx, probs, alpha, beta, beta_zero, flag);
+    tile_grouped_f64(ctx, probs, alpha, beta, beta_zero, flag);
     hipLaunchKernelGGL((k_gi8gemm<I8Sq, I8_ROW4G>), dim3((uint32_t)tg, (uint32_t)n), dim3(I8Sq::NT), 0, ctx->stream,
                        dprobs, count,
                        dpre + 2 * (count + 1), (uint32_t)tg, A8, B8, R, (int64_t)sA, (int64_t)sB, (int64_t)sR, su.ms,
