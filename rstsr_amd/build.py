@@ -33,6 +33,7 @@ DEVICE_SOURCES = [
     ("reduce.hip", ["-ffp-contract=off"]),
     ("unary.hip", ["-ffp-contract=off"]),
     ("gemm.hip", []),
+    ("gemv.hip", []),
     ("gemm_tile_f32.hip", []),
     ("gemm_tile_f64.hip", []),
     ("gemm_tile_c64.hip", []),

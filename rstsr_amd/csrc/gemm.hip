@@ -431,6 +431,7 @@ void run_gemm(rstsr_hip_ctx* ctx, rstsr_dtype_t t, rstsr_gemm_mode_t mode, const
                 return;
             }
         }
+        if (gemv(ctx, t, P, alpha, beta, bz)) return;
         launch_gemm_t<T>(ctx, P, al, be, bz);
     };
     switch (t) {

@@ -99,7 +99,9 @@ void tile_gemm_f64(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, doubl
                    const int* run_if, const MirrorFn& mirror);
 void tile_gemm_c128(rstsr_hip_ctx* ctx, const GemmProblem& P, c128 alpha, c128 beta, bool beta_zero,
                     const int* run_if, const MirrorFn& mirror);
-// Grouped (uneven) GEMMs in one persistent launch: problems without batches, with M, N, K > 0 and
+// Products with one row or one column (gemv.hip); false when the problem is not one it takes.
+bool gemv(rstsr_hip_ctx* ctx, rstsr_dtype_t t, const GemmProblem& P, const void* alpha, const void* beta, bool beta_zero);
+// Grouped (uneven) GEMMs, one launch per operand form: problems without batches, with M, N, K > 0 and
 // outputs that do not overlap. The tile shape is the tuner's, or with run_if a fixed one.
 void tile_grouped_f64(rstsr_hip_ctx* ctx, const std::vector<GemmProblem>& probs, double alpha, double beta,
                       bool beta_zero, const int* run_if);
