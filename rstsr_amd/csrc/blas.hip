@@ -16,7 +16,7 @@
 // use.
 #include "common.hpp"
 #include "registry.hpp"
-#include "gemm.hpp"
+#include "gemm_tile.hpp"
 
 #include <cstring>
 #include <type_traits>
@@ -70,67 +70,258 @@ __global__ void __launch_bounds__(256) k_sym_expand(T* __restrict__ dst, const T
     }
 }
 
-// complex-aware arithmetic of the triangular solve
 template <class T>
 __device__ __forceinline__ T t_mul(T a, T b) {
     if constexpr (std::is_same<T, c128>::value || std::is_same<T, c64>::value)
         return T{a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
     else return a * b;
 }
+
+// Quotients by one divisor, as accurate as divisions and without their branches: both parts are
+// scaled to [1/2, 1), q = a r is corrected by its exact remainder (r = 1/d), and the exponents are put
+// back; v_div_fixup gives zeros, infinities and NaN their IEEE results.
+template <class R>
+struct Recip {
+    R d, m, r;
+    int e;
+    __device__ static R mant(R x) {
+        if constexpr (sizeof(R) == 8) return __builtin_amdgcn_frexp_mant(x);
+        else return __builtin_amdgcn_frexp_mantf(x);
+    }
+    __device__ static int expo(R x) {
+        if constexpr (sizeof(R) == 8) return __builtin_amdgcn_frexp_exp(x);
+        else return __builtin_amdgcn_frexp_expf(x);
+    }
+    __device__ static Recip of(R d) {
+        const R m = mant(d);
+        return {d, m, (R)1 / m, expo(d)};
+    }
+    __device__ __forceinline__ R quot(R a) const {
+        const R am = mant(a);
+        R q = am * r;
+        q = fma(fma(-m, q, am), r, q);
+        q = ldexp(q, expo(a) - e);
+        if constexpr (sizeof(R) == 8) return __builtin_amdgcn_div_fixup(q, d, a);
+        else return __builtin_amdgcn_div_fixupf(q, d, a);
+    }
+};
+// The divisor of one row of the solve. Complex: a conj(b) / |b|^2 with b scaled by its larger part
+// (no overflow for moderate b).
 template <class T>
-__device__ __forceinline__ T t_sub(T a, T b) {
-    if constexpr (std::is_same<T, c128>::value || std::is_same<T, c64>::value) return T{a.re - b.re, a.im - b.im};
-    else return a - b;
+struct Divisor {
+    Recip<T> s;
+    __device__ static Divisor of(T b) { return {Recip<T>::of(b)}; }
+    __device__ __forceinline__ T quot(T a) const { return s.quot(a); }
+};
+template <class T, class R>
+struct DivisorC {
+    R br, bi;
+    Recip<R> d, s;
+    __device__ static DivisorC of(T b) {
+        const R m = fmax(fabs(b.re), fabs(b.im)), br = b.re / m, bi = b.im / m;
+        return {br, bi, Recip<R>::of(br * br + bi * bi), Recip<R>::of(m)};
+    }
+    __device__ __forceinline__ T quot(T a) const {
+        return T{s.quot(d.quot(a.re * br + a.im * bi)), s.quot(d.quot(a.im * br - a.re * bi))};
+    }
+};
+template <>
+struct Divisor<c64> : DivisorC<c64, float> {
+    __device__ static Divisor of(c64 b) { return {DivisorC<c64, float>::of(b)}; }
+};
+template <>
+struct Divisor<c128> : DivisorC<c128, double> {
+    __device__ static Divisor of(c128 b) { return {DivisorC<c128, double>::of(b)}; }
+};
+
+// v of lanes 16 g .. 16 g + 15 in every group of 16 lanes
+__device__ __forceinline__ uint32_t bcast_row(uint32_t v, int g) {
+    const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);  // lower halves, upper halves
+    const uint32_t w = g < 2 ? h[0] : h[1];
+    const auto r = __builtin_amdgcn_permlane16_swap(w, w, false, false);  // even rows, odd rows
+    return g % 2 == 0 ? r[0] : r[1];
 }
 template <class T>
-__device__ __forceinline__ T t_div(T a, T b) {
-    if constexpr (std::is_same<T, c128>::value || std::is_same<T, c64>::value) {
-        // a conj(b) / |b|^2 with |b|^2 scaled by the larger part of b (no overflow for moderate b)
-        const auto s = fmax(fabs(b.re), fabs(b.im));
-        const auto br = b.re / s, bi = b.im / s, d = br * br + bi * bi;
-        return T{(a.re * br + a.im * bi) / d / s, (a.im * br - a.re * bi) / d / s};
-    } else {
-        return a / b;
-    }
+__device__ __forceinline__ T bcast_rows(T v, int g) {
+    uint32_t w[sizeof(T) / 4];
+    __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+    for (size_t i = 0; i < sizeof(T) / 4; ++i) w[i] = bcast_row(w[i], g);
+    __builtin_memcpy(&v, w, sizeof(T));
+    return v;
 }
 
-constexpr int TRSM_NB = 64;  // rows of a diagonal block solved in LDS
+// Barrier for data that waves exchange through LDS: unlike __syncthreads it leaves global loads and
+// stores in flight.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// One diagonal block of the triangular solve, in place: X (kb x r, strides xrs / xcs) :=
-// T^-1 X for the kb x kb triangle T (strides trs / tcs; lower or upper; unit: diagonal taken
-// as one and not read). One thread per column of X (64 per block); T and the block's 64
-// columns staged in LDS, each column by forward (lower) or backward substitution.
+constexpr int TRSM_NB = 256;                 // rows solved by one launch
+constexpr int TRSM_F = TRSM_NB / 16;         // 16-row fragments of them
+constexpr int TRSM_NW = 8;                   // waves per block
+constexpr int TRSM_FPW = TRSM_F / TRSM_NW;   // fragments per wave
+
+// Triangular solve of up to 256 rows, in place: X (kb x r, strides xrs / xcs) := T^-1 X for the
+// lower triangle T (kb x kb, strides trs / tcs; an upper one comes with its rows, columns and X's
+// rows reversed, that is negative strides; unit: diagonal taken as one and not read).
+//
+// What bounds it: the chain over the rows (a column's x[i] needs every x before it), so all of it
+// runs in one launch and each step is kept short. A block owns 16 columns of X, which are
+// independent of all others: r / 16 blocks without any exchange. X stays in the matrix cores'
+// accumulators, fragment f (rows 16 f ..) in wave f % 8. Step j: the wave that owns fragment j
+// subtracts block j - 1's share from it (four MFMAs), solves its 16 rows by substitution in the
+// accumulators' own layout and publishes x through LDS; after one barrier the waves subtract
+// T(f, j) x from their fragments below, with the blocks of T loaded a step ahead.
+// Measured: 256 rows x 1600 columns f64 29-37 us; 2000 rows 0.52 ms in all, eight such launches and
+// the updates between them by the GEMM (3.5 ms with 64-row blocks, one thread per column).
 template <class T>
-__global__ void __launch_bounds__(TRSM_NB) k_trsm_diag(const T* __restrict__ Tm, int64_t trs, int64_t tcs, int lower,
-                                                      int unit, int kb, T* __restrict__ X, int64_t xrs, int64_t xcs,
-                                                      int64_t r) {
-    __shared__ T Ts[TRSM_NB][TRSM_NB + 1];
-    __shared__ T Xs[TRSM_NB][TRSM_NB];
-    const int j = threadIdx.x;
-    const int64_t col = (int64_t)blockIdx.x * TRSM_NB + j;
-    for (int e = j; e < kb * kb; e += TRSM_NB) {
-        const int i = e / kb, k = e - i * kb;
-        // only the stored triangle is read, and a unit diagonal not at all
-        const bool in = (lower ? k <= i : k >= i) && !(unit && k == i);
-        Ts[i][k] = in ? Tm[(int64_t)i * trs + (int64_t)k * tcs] : T{};
+__global__ void __launch_bounds__(64 * TRSM_NW) k_trsm_block(const T* __restrict__ Tm, int64_t trs, int64_t tcs, int unit,
+                                                            int kb, T* __restrict__ X, int64_t xrs, int64_t xcs,
+                                                            int64_t r) {
+    using R = typename ElemOf<T>::R;
+    using MM = Mma<R>;
+    constexpr bool CX = ElemOf<T>::CX;
+    constexpr int NP = CX ? 2 : 1;
+    __shared__ T diag[TRSM_F][16][16];  // [block][column c][row r > c]
+    __shared__ Divisor<T> divs[TRSM_NB];
+    __shared__ T xs[2][16][16];         // x of the current block: [parity][row][column]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = lane & 15, q = lane >> 4;
+    const int64_t col = (int64_t)blockIdx.x * 16 + n;
+    const int nf = (kb + 15) / 16;
+    // rows past kb: x = 0, divisor one
+    constexpr int DL = TRSM_F * 256 / (64 * TRSM_NW);  // diagonal elements per thread, all in flight at once
+    T dl[DL];
+#pragma unroll
+    for (int u = 0; u < DL; ++u) {
+        const int e = u * 64 * TRSM_NW + threadIdx.x, f = e >> 8, i = e >> 4 & 15, c = e & 15, row = 16 * f + i;
+        dl[u] = i > c && row < kb ? Tm[(int64_t)row * trs + (int64_t)(16 * f + c) * tcs] : T{};
     }
-    for (int i = 0; i < kb; ++i) Xs[i][j] = col < r ? X[(int64_t)i * xrs + col * xcs] : T{};
-    __syncthreads();
-    if (col >= r) return;
-    if (lower) {
-        for (int i = 0; i < kb; ++i) {
-            T acc = Xs[i][j];
-            for (int k = 0; k < i; ++k) acc = t_sub(acc, t_mul(Ts[i][k], Xs[k][j]));
-            Xs[i][j] = unit ? acc : t_div(acc, Ts[i][i]);
-        }
-    } else {
-        for (int i = kb - 1; i >= 0; --i) {
-            T acc = Xs[i][j];
-            for (int k = i + 1; k < kb; ++k) acc = t_sub(acc, t_mul(Ts[i][k], Xs[k][j]));
-            Xs[i][j] = unit ? acc : t_div(acc, Ts[i][i]);
-        }
+    for (int i = threadIdx.x; i < nf * 16; i += 64 * TRSM_NW) {
+        T d{};
+        if constexpr (CX) d.re = 1;
+        else d = 1;
+        if (!unit && i < kb) d = Tm[(int64_t)i * (trs + tcs)];
+        divs[i] = Divisor<T>::of(d);
     }
-    for (int i = 0; i < kb; ++i) X[(int64_t)i * xrs + col * xcs] = Xs[i][j];
+    typename MM::Acc acc[TRSM_FPW][NP];
+#pragma unroll
+    for (int i = 0; i < TRSM_FPW; ++i)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int row = 16 * (i * TRSM_NW + wave) + MM::row(k, lane);
+            const T v = row < kb && col < r ? X[(int64_t)row * xrs + col * xcs] : T{};
+            if constexpr (CX) {
+                acc[i][0][k] = v.re;
+                acc[i][NP - 1][k] = v.im;
+            } else {
+                acc[i][0][k] = v;
+            }
+        }
+    // T(f, j) of this lane: row n of the fragment, positions 4 q + e of block j
+    auto load_t = [&](T (&t)[4], int f, int j) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int row = 16 * f + n;
+            t[e] = f > j && row < kb ? Tm[(int64_t)row * trs + (int64_t)(16 * j + 4 * q + e) * tcs] : T{};
+        }
+    };
+    auto subtract = [&](typename MM::Acc (&a)[NP], const T (&t)[4], const T (&x)[4]) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if constexpr (CX) {
+                a[0] = MM::mma(-t[e].re, x[e].re, a[0]);
+                a[0] = MM::mma(t[e].im, x[e].im, a[0]);
+                a[NP - 1] = MM::mma(-t[e].re, x[e].im, a[NP - 1]);
+                a[NP - 1] = MM::mma(-t[e].im, x[e].re, a[NP - 1]);
+            } else {
+                a[0] = MM::mma(-t[e], x[e], a[0]);
+            }
+        }
+    };
+    // substitution of fragment f (this wave's accumulators): x replaces it and goes to xs[f & 1]. Lane
+    // (n, q) holds rows MM::row(k, lane) of column n; each quotient is formed in the lanes that hold its
+    // row and handed to the column's other lanes by two lane swaps. The divisors and columns of the
+    // diagonal block do not depend on x: they are read a step ahead.
+    auto solve = [&](typename MM::Acc (&a)[NP], int f) __attribute__((always_inline)) {
+        T b[4], d[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if constexpr (CX) b[k] = T{a[0][k], a[NP - 1][k]};
+            else b[k] = a[0][k];
+            d[k] = diag[f][0][MM::row(k, lane)];
+        }
+        Divisor<T> dv = divs[16 * f];
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            constexpr bool RS = sizeof(R) == 8;  // row 4 k + q (else 4 q + k) is in lanes q, register k
+            const int k0 = RS ? c / 4 : c % 4, g = RS ? c % 4 : c / 4;
+            const Divisor<T> dc = dv;
+            T e[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) e[k] = d[k];
+            if (c < 15) {
+                dv = divs[16 * f + c + 1];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) d[k] = diag[f][c + 1][MM::row(k, lane)];
+            }
+            const T xc = dc.quot(b[k0]);
+            if (q == g) b[k0] = xc;
+            const T xb = bcast_rows(xc, g);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (RS && k < k0) continue;  // rows above c only
+                T v = b[k];
+                if constexpr (CX) {
+                    v.re = fma(e[k].im, xb.im, fma(-e[k].re, xb.re, v.re));
+                    v.im = fma(-e[k].im, xb.re, fma(-e[k].re, xb.im, v.im));
+                } else {
+                    v = fma(-e[k], xb, v);
+                }
+                if (MM::row(k, lane) > c) b[k] = v;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) xs[f & 1][MM::row(k, lane)][n] = b[k];
+    };
+    T t[TRSM_FPW][4];
+#pragma unroll
+    for (int i = 0; i < TRSM_FPW; ++i) load_t(t[i], i * TRSM_NW + wave, 0);
+#pragma unroll
+    for (int u = 0; u < DL; ++u) {
+        const int e = u * 64 * TRSM_NW + threadIdx.x;
+        diag[e >> 8][e & 15][e >> 4 & 15] = dl[u];
+    }
+    __syncthreads();  // diagonal blocks and divisors staged
+    if (wave == 0) solve(acc[0], 0);
+    lds_barrier();
+    for (int j = 0; j < nf; ++j) {
+        // x of block j is in xs[j & 1], T(., j) in t
+        T x[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = xs[j & 1][4 * q + e][n];
+        const int own = (j + 1) % TRSM_NW == wave && j + 1 < nf ? (j + 1) / TRSM_NW : -1;
+#pragma unroll
+        for (int i = 0; i < TRSM_FPW; ++i)
+            if (i == own) {
+                subtract(acc[i], t[i], x);
+                solve(acc[i], j + 1);
+            }
+#pragma unroll
+        for (int i = 0; i < TRSM_FPW; ++i)
+            if (i != own && i * TRSM_NW + wave > j && i * TRSM_NW + wave < nf) subtract(acc[i], t[i], x);
+        // the wave that solves last from here on stores block j
+        if (wave == j % TRSM_NW && col < r) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int row = 16 * j + 4 * q + e;
+                if (row < kb) X[(int64_t)row * xrs + col * xcs] = x[e];
+            }
+        }
+        // the next solver is another wave, whose loads run while this step's solver works
+#pragma unroll
+        for (int i = 0; i < TRSM_FPW; ++i) load_t(t[i], i * TRSM_NW + wave, j + 1);
+        lds_barrier();
+    }
 }
 
 // X (rows x cols, strides rs / cs) *= alpha, or := 0 when zero (BLAS: B is not read)
@@ -326,7 +517,7 @@ static void driver_syhemm(rstsr_hip_ctx* ctx, rstsr_dtype_t t, rstsr_gemm_mode_t
 // a transposition swaps T's strides and its triangle; a conjugated A (trans C or CN) is copied
 // conjugated into scratch first. T Y = Z is solved recursively: halves of the rows, the
 // trailing half updated by the GEMM (alpha -1, beta 1) with K the leading half's size, down to
-// 64-row diagonal blocks solved in LDS (k_trsm_diag).
+// 256-row diagonal blocks solved in one launch each (k_trsm_block).
 static void driver_trsm(rstsr_hip_ctx* ctx, rstsr_dtype_t t, rstsr_gemm_mode_t mode, int order, int side, int uplo,
                         int transa, int diag, size_t m, size_t n, const void* alpha, const void* a, size_t lda, void* b,
                         size_t ldb) {
@@ -391,9 +582,11 @@ static void driver_trsm(rstsr_hip_ctx* ctx, rstsr_dtype_t t, rstsr_gemm_mode_t m
         auto solve = [&](auto&& self, int64_t lo, int64_t hi) -> void {
             const int64_t len = hi - lo;
             if (len <= TRSM_NB) {
-                hipLaunchKernelGGL(k_trsm_diag<T>, dim3((uint32_t)((r + TRSM_NB - 1) / TRSM_NB)), dim3(TRSM_NB), 0,
-                                   ctx->stream, Tm + lo * trs + lo * tcs, trs, tcs, lower ? 1 : 0,
-                                   diag == DIAG_U ? 1 : 0, (int)len, Y + lo * yrs, yrs, ycs, r);
+                // an upper triangle is a lower one with every row order reversed
+                const int64_t at = lower ? lo : hi - 1, sg = lower ? 1 : -1;
+                hipLaunchKernelGGL(k_trsm_block<T>, dim3((uint32_t)((r + 15) / 16)), dim3(64 * TRSM_NW), 0, ctx->stream,
+                                   Tm + at * (trs + tcs), sg * trs, sg * tcs, diag == DIAG_U ? 1 : 0, (int)len,
+                                   Y + at * yrs, sg * yrs, ycs, r);
                 check_launch("trsm diagonal block");
                 return;
             }
