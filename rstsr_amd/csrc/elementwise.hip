@@ -184,8 +184,9 @@ __device__ __forceinline__ TC cast_to(TA a) {
 }
 
 /* =============================== bodies =============================== */
-// A body loads operand A and B at element offsets and stores C; kernels only do
-// index arithmetic. TA/TB = None marks an absent operand.
+// A body loads operand A and B at element offsets and stores C (st), or gives C's value for a
+// packed store (val, of type TO); kernels only do index arithmetic. TA/TB = None marks an absent
+// operand.
 
 template <int OP, class T, bool AS, bool BS>
 struct BinBody {
@@ -197,13 +198,14 @@ struct BinBody {
     T sa, sb;
     static constexpr int OPS = (AS ? 0 : 1) | (BS ? 0 : 2);
     static constexpr size_t OUT_SIZE = sizeof(T);
-    static constexpr bool NT_JOINT = false;
     template <bool NT = false>
     __device__ __forceinline__ T la(int64_t o) const { return AS ? sa : ld<NT>(a + o); }
     template <bool NT = false>
     __device__ __forceinline__ T lb(int64_t o) const { return BS ? sb : ld<NT>(b + o); }
     template <bool NT = false>
     __device__ __forceinline__ void st(int64_t o, T x, T y) const { sto<NT>(c + o, apply_op<OP, T>(x, y)); }
+    using TO = T;
+    __device__ __forceinline__ T val(T x, T y) const { return apply_op<OP, T>(x, y); }
 };
 
 // c = a op b with one operand complex (C) and the other its real type; AS / BS: host scalar.
@@ -218,15 +220,18 @@ struct MixBody {
     TBv sb;
     static constexpr int OPS = (AS ? 0 : 1) | (BS ? 0 : 2);
     static constexpr size_t OUT_SIZE = sizeof(C);
-    static constexpr bool NT_JOINT = false;
     template <bool NT = false>
     __device__ __forceinline__ TAv la(int64_t o) const { return AS ? sa : ld<NT>(a + o); }
     template <bool NT = false>
     __device__ __forceinline__ TBv lb(int64_t o) const { return BS ? sb : ld<NT>(b + o); }
     template <bool NT = false>
     __device__ __forceinline__ void st(int64_t o, TAv x, TBv y) const {
-        if constexpr (std::is_same<TAv, C>::value) sto<NT>(c + o, mix_cr<OP, C>(x, y));
-        else sto<NT>(c + o, mix_rc<OP, C>(x, y));
+        sto<NT>(c + o, val(x, y));
+    }
+    using TO = C;
+    __device__ __forceinline__ C val(TAv x, TBv y) const {
+        if constexpr (std::is_same<TAv, C>::value) return mix_cr<OP, C>(x, y);
+        else return mix_rc<OP, C>(x, y);
     }
 };
 
@@ -238,13 +243,14 @@ struct CastBody {
     const TAv* a;
     static constexpr int OPS = 1;
     static constexpr size_t OUT_SIZE = sizeof(TCv);
-    static constexpr bool NT_JOINT = false;
     template <bool NT = false>
     __device__ __forceinline__ TAv la(int64_t o) const { return ld<NT>(a + o); }
     template <bool NT = false>
     __device__ __forceinline__ None lb(int64_t) const { return None{}; }
     template <bool NT = false>
     __device__ __forceinline__ void st(int64_t o, TAv x, None) const { sto<NT>(c + o, cast_to<TCv, TAv>(x)); }
+    using TO = TCv;
+    __device__ __forceinline__ TCv val(TAv x, None) const { return cast_to<TCv, TAv>(x); }
 };
 
 template <class T>
@@ -255,13 +261,14 @@ struct FillBody {
     T v;
     static constexpr int OPS = 0;
     static constexpr size_t OUT_SIZE = sizeof(T);
-    static constexpr bool NT_JOINT = false;
     template <bool NT = false>
     __device__ __forceinline__ None la(int64_t) const { return None{}; }
     template <bool NT = false>
     __device__ __forceinline__ None lb(int64_t) const { return None{}; }
     template <bool NT = false>
     __device__ __forceinline__ void st(int64_t o, None, None) const { sto<NT>(c + o, v); }
+    using TO = T;
+    __device__ __forceinline__ T val(None, None) const { return v; }
 };
 
 // ExtNum::ext_abs_diff / ext_abs (rstsr-dtype-traits/src/ext_num.rs:72-214) in the element
@@ -305,7 +312,6 @@ struct CloseBody {
     int equal_nan;
     static constexpr int OPS = 3;
     static constexpr size_t OUT_SIZE = 0;
-    static constexpr bool NT_JOINT = false;
     template <bool NT = false>
     __device__ __forceinline__ T la(int64_t o) const { return ld<NT>(a + o); }
     template <bool NT = false>

@@ -11,9 +11,11 @@
 //   2. if an input's unit-stride axis differs from the output's, run the
 //      LDS-tiled kernel: tiles read along the input's unit axis and written
 //      along the output's unit axis (both sides coalesced);
-//   3. else if the innermost extent is long, run the row kernel (one block per
+//   3. else if the output is contiguous, run the flat kernel (packs of consecutive
+//      elements, index math once per pack and only for operands that are not);
+//   4. else if the innermost extent is long, run the row kernel (one block per
 //      row chunk, index math once per block);
-//   4. else the generic kernel (per-element fast-division unravel).
+//   5. else the generic kernel (per-element fast-division unravel).
 #pragma once
 #include "common.hpp"
 #include "registry.hpp"
@@ -87,6 +89,130 @@ __global__ void __launch_bounds__(EW_BLOCK) k_ew_generic(Body body, EwPlan p, ui
     }
 }
 
+// N consecutive elements as words of up to 16 bytes; the address needs the element's alignment only.
+template <bool NT, class T, int N>
+__device__ __forceinline__ void store_pack(T* p, const T (&v)[N]) {
+    constexpr int B = sizeof(T) * N, W = B % 16 == 0 ? 4 : (B % 8 == 0 ? 2 : 1);
+    typedef uint32_t Word __attribute__((ext_vector_type(W), aligned(sizeof(T) < 4 ? sizeof(T) : 4)));
+    if constexpr (B % 4 != 0) {
+#pragma unroll
+        for (int e = 0; e < N; ++e) p[e] = v[e];
+    } else {
+#pragma unroll
+        for (int i = 0; i < B / (4 * W); ++i) {
+            Word w;
+            __builtin_memcpy(&w, (const char*)v + i * 4 * W, 4 * W);
+            if constexpr (NT) __builtin_nontemporal_store(w, (Word*)p + i);
+            else ((Word*)p)[i] = w;
+        }
+    }
+}
+
+// flat: the output is contiguous, so each thread takes U packs of VEC consecutive elements and
+// stores each as one word. Operands laid out like the output (bit k of `same`) load the same way;
+// others are broadcast or contiguous along dim 0 (stride 0 or 1): their row (dims 1 ..) is
+// unravelled once per pack, and once more for a pack that crosses into the next row. Bound by HBM (or the last-level cache): what it saves over the generic kernel is
+// the index math per element and three quarters of the load and store instructions of 4-byte types.
+// NTM as below. Measurements at untiled_kind.
+template <class Body, int VEC, int U, int NTM>
+__global__ void __launch_bounds__(EW_BLOCK) k_ew_flat(Body body, EwPlan p, uint32_t total, int same) {
+    using TA = typename Body::TA;
+    using TB = typename Body::TB;
+    constexpr uint32_t STEP = EW_BLOCK * VEC;
+    const uint32_t base = (blockIdx.x * (EW_BLOCK * U) + threadIdx.x) * VEC;
+    const uint32_t n0 = p.shape[0];
+    TA va[U][VEC];
+    TB vb[U][VEC];
+    // elements i .. i + cnt - 1 of operand k into v
+    auto fetch = [&](auto load, int k, uint32_t i, uint32_t cnt, auto& v) {
+        if (same >> k & 1) {
+            if (cnt == VEC) {
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) v[e] = load(p.off[k] + (int64_t)i + e);
+            } else {
+                for (uint32_t e = 0; e < cnt; ++e) v[e] = load(p.off[k] + (int64_t)i + e);
+            }
+            return;
+        }
+        auto at = [&](uint32_t row) {
+            int64_t o = p.off[k];
+#pragma unroll
+            for (int d = 1; d < MAXD; ++d) {
+                if (d >= p.nd) break;
+                const uint32_t q = fdiv(row, p.fd[d]);
+                o += (int64_t)(row - q * p.shape[d]) * p.st[k][d];
+                row = q;
+            }
+            return o;
+        };
+        const int64_t s0 = p.st[k][0];
+        const uint32_t row = fdiv(i, p.fd[0]), r = i - row * n0;
+        if (cnt == VEC && n0 >= VEC) {
+            // inside one row, or across the end of one into the next
+            const int64_t o = at(row);
+            if (n0 % VEC == 0 || __all(r + VEC <= n0)) {
+                if (s0 == 0) {
+                    const auto x = load(o);
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) v[e] = x;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) v[e] = load(o + r + e);
+                }
+                return;
+            }
+            const int64_t o1 = r + VEC > n0 ? at(row + 1) : o;
+            if (s0 == 0) {
+                const auto x = load(o), x1 = load(o1);
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) v[e] = r + e < n0 ? x : x1;
+            } else {
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) v[e] = load(r + e < n0 ? o + r + e : o1 + (r + e - n0));
+            }
+            return;
+        }
+#pragma unroll
+        for (int e = 0; e < VEC; ++e)
+            if ((uint32_t)e < cnt) {
+                const uint32_t w = fdiv(i + e, p.fd[0]);
+                v[e] = load(at(w) + (int64_t)(i + e - w * n0) * s0);
+            }
+    };
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const uint32_t i = base + u * STEP;
+        if (i >= total) continue;
+        const uint32_t cnt = min((uint32_t)VEC, total - i);
+        if constexpr ((Body::OPS & 1) != 0)
+            fetch([&](int64_t o) { return body.template la<(NTM & 1) != 0>(o); }, 1, i, cnt, va[u]);
+        if constexpr ((Body::OPS & 2) != 0)
+            fetch([&](int64_t o) { return body.template lb<(NTM & 2) != 0>(o); }, 2, i, cnt, vb[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const uint32_t i = base + u * STEP;
+        if (i >= total) continue;
+        // an operand that is a scalar comes from the body
+        auto xa = [&](int e) {
+            if constexpr ((Body::OPS & 1) != 0) return va[u][e];
+            else return body.la(0);
+        };
+        auto xb = [&](int e) {
+            if constexpr ((Body::OPS & 2) != 0) return vb[u][e];
+            else return body.lb(0);
+        };
+        if (i + VEC <= total) {
+            typename Body::TO o[VEC];
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) o[e] = body.val(xa(e), xb(e));
+            store_pack<(NTM & 4) != 0>(body.c + p.off[0] + i, o);
+        } else {
+            for (uint32_t e = 0; i + e < total; ++e) body.st(p.off[0] + (int64_t)i + e, xa(e), xb(e));
+        }
+    }
+}
+
 // rows: dim 0 is a long row; blockIdx -> (row, chunk); unravel once per block.
 // NTM: bit0 / bit1 streaming loads of A / B (operands read once), bit2 streaming
 // stores (large outputs).
@@ -129,7 +255,8 @@ __global__ void __launch_bounds__(EW_BLOCK) k_ew_rows(Body body, EwPlan p, uint3
 // offset is one product instead of an unravel over every axis.
 // NTM: bit0 / bit1 streaming loads of the staged A / B in full tiles, bit2
 // streaming stores.
-template <class Body, int TI, int TC, int STAGE, bool ONE, int NTM>
+// EDGE: tiles may end past the matrix; without it the code for such tiles is left out.
+template <class Body, int TI, int TC, int STAGE, bool ONE, int NTM, bool EDGE>
 __global__ void __launch_bounds__(EW_BLOCK) k_ew_tiled(Body body, EwPlan p, int di, int od, uint32_t nti,
                                                        uint32_t ntc, FastDiv fti, FastDiv ftc, int xmap) {
     using TA = typename Body::TA;
@@ -141,11 +268,11 @@ __global__ void __launch_bounds__(EW_BLOCK) k_ew_tiled(Body body, EwPlan p, int 
     __shared__ TA lds_a[SA ? TC : 1][SA ? TI + 1 : 1];
     __shared__ TB lds_b[SB ? TC : 1][SB ? TI + 1 : 1];
 
-    // tile order (autotuned per problem class): 0 output-axis tiles fastest,
-    // 1 the same in one contiguous range per XCD, 2 input-axis tiles fastest
-    uint32_t b = xmap == 1 ? xcd_chunk(blockIdx.x, gridDim.x) : blockIdx.x;
+    // tile order (autotuned per problem class): bit 1 input-axis tiles fastest (else output-axis
+    // ones), bit 0 one contiguous range of the order per XCD
+    uint32_t b = xmap & 1 ? xcd_chunk(blockIdx.x, gridDim.x) : blockIdx.x;
     uint32_t tc, ti, outer;
-    if (xmap == 2) {
+    if (xmap & 2) {
         uint32_t q1 = fdiv(b, fti);
         ti = b - q1 * nti;
         outer = fdiv(q1, ftc);
@@ -183,7 +310,7 @@ __global__ void __launch_bounds__(EW_BLOCK) k_ew_tiled(Body body, EwPlan p, int 
     const int64_t sc_c = p.st[0][0], sc_i = p.st[0][di];
     const int64_t sa_c = p.st[1][0], sa_i = p.st[1][di];
     const int64_t sb_c = p.st[2][0], sb_i = p.st[2][di];
-    const bool full = (i0 + TI <= Ni) && (c0 + TC <= Nc);
+    const bool full = !EDGE || ((i0 + TI <= Ni) && (c0 + TC <= Nc));
     const int tid = threadIdx.x;
 
     if constexpr (SA || SB) {
@@ -193,20 +320,46 @@ __global__ void __launch_bounds__(EW_BLOCK) k_ew_tiled(Body body, EwPlan p, int 
         const int64_t pb = ob + (int64_t)(i0 + ii) * sb_i + (int64_t)(c0 + cb) * sb_c, db = (int64_t)ROWS1 * sb_c;
         if (full) {
             // offsets advance by a uniform stride: one 64-bit add per load
-            int64_t ua = pa, ub = pb;
+            auto rows = [&](auto k0, auto k1, auto ntm) {
+                constexpr int H = decltype(ntm)::value;
+                int64_t ua = pa + decltype(k0)::value * da, ub = pb + decltype(k0)::value * db;
 #pragma unroll
-            for (int k = 0; k < PER1; ++k) {
-                if constexpr (SA) lds_a[k * ROWS1 + cb][ii] = body.template la<(NTM & 1) != 0>(ua);
-                if constexpr (SB) lds_b[k * ROWS1 + cb][ii] = body.template lb<(NTM & 2) != 0>(ub);
-                ua += da;
-                ub += db;
-            }
+                for (int k = decltype(k0)::value; k < decltype(k1)::value; ++k) {
+                    if constexpr (SA) lds_a[k * ROWS1 + cb][ii] = body.template la<(H & 1) != 0>(ua);
+                    if constexpr (SB) lds_b[k * ROWS1 + cb][ii] = body.template lb<(H & 2) != 0>(ub);
+                    ua += da;
+                    ub += db;
+                }
+            };
+            // of the streamed rows one in eight is loaded without the hint: those lines live on in the
+            // last-level cache, where a stream of all rows would push itself out, and a later pass over
+            // the same operand finds them (f64 [1024, 256, 256] multiply, three 512 MB inputs in turn:
+            // none 192 us, 1 in 16 186, 1 in 8 181, 1 in 4 194: no longer in the cache together)
+            constexpr int KEEP = PER1 >= 8 ? PER1 / 8 : 0;
+            rows(std::integral_constant<int, 0>{}, std::integral_constant<int, PER1 - KEEP>{},
+                 std::integral_constant<int, NTM>{});
+            if constexpr (KEEP > 0)
+                rows(std::integral_constant<int, PER1 - KEEP>{}, std::integral_constant<int, PER1>{},
+                     std::integral_constant<int, 0>{});
         } else {
+            // edge tile: positions past the end repeat the last one (never stored), so that the loads
+            // need no branch and are in flight together, four at a time
+            const int64_t i = min(i0 + ii, Ni - 1);
+            const int64_t ua = oa + i * sa_i, ub = ob + i * sb_i;
+            constexpr int P = PER1 % 4 == 0 ? 4 : PER1;
+            for (int k0 = 0; k0 < PER1; k0 += P) {
+                TA xa[SA ? P : 1];
+                TB xb[SB ? P : 1];
 #pragma unroll
-            for (int k = 0; k < PER1; ++k) {
-                if (i0 + ii < Ni && c0 + k * ROWS1 + cb < Nc) {
-                    if constexpr (SA) lds_a[k * ROWS1 + cb][ii] = body.la(pa + k * da);
-                    if constexpr (SB) lds_b[k * ROWS1 + cb][ii] = body.lb(pb + k * db);
+                for (int k = 0; k < P; ++k) {
+                    const int64_t c = min(c0 + (k0 + k) * ROWS1 + cb, Nc - 1);
+                    if constexpr (SA) xa[k] = body.template la<(NTM & 1) != 0>(ua + c * sa_c);
+                    if constexpr (SB) xb[k] = body.template lb<(NTM & 2) != 0>(ub + c * sb_c);
+                }
+#pragma unroll
+                for (int k = 0; k < P; ++k) {
+                    if constexpr (SA) lds_a[(k0 + k) * ROWS1 + cb][ii] = xa[k];
+                    if constexpr (SB) lds_b[(k0 + k) * ROWS1 + cb][ii] = xb[k];
                 }
             }
         }
@@ -217,7 +370,7 @@ __global__ void __launch_bounds__(EW_BLOCK) k_ew_tiled(Body body, EwPlan p, int 
     const int64_t pc = oc + (int64_t)(c0 + cc) * sc_c + (int64_t)(i0 + ib) * sc_i, dc2 = (int64_t)ROWS2 * sc_i;
     const int64_t qa = oa + (int64_t)(c0 + cc) * sa_c + (int64_t)(i0 + ib) * sa_i, da2 = (int64_t)ROWS2 * sa_i;
     const int64_t qb = ob + (int64_t)(c0 + cc) * sb_c + (int64_t)(i0 + ib) * sb_i, db2 = (int64_t)ROWS2 * sb_i;
-    const bool col_ok = c0 + cc < Nc;
+    const bool col_ok = !EDGE || c0 + cc < Nc;
     auto run = [&](auto hoist_b) {
         constexpr bool HB = decltype(hoist_b)::value;
         TB yb{};
@@ -328,13 +481,35 @@ static EwPlan to_plan(const Dims& d) {
     return p;
 }
 
-enum class EwKind { Generic, Rows, Tiled };
+enum class EwKind { Generic, Rows, Flat, Tiled };
 
 struct EwChoice {
     EwKind kind = EwKind::Generic;
     int di = -1;
     int stage = 0;  // bit0 A, bit1 B
 };
+
+// Whether operand k's strides are those of a contiguous array over the dims in their order.
+static bool is_flat(const Dims& d, int k) {
+    int64_t n = 1;
+    for (int i = 0; i < d.nd; ++i) {
+        if (d.st[i][k] != n) return false;
+        n *= (int64_t)d.shape[i];
+    }
+    return true;
+}
+
+// A contiguous output whose operands (bits of `ops`: A, B) are contiguous or broadcast along dim 0
+// takes the flat kernel. Measured (us, 16-byte packs against the generic / row kernel): f32 [50021,
+// 233] - [50021, 1] 16.6 against 24.1, exp of 47 MB 14.9 against 16.1, [400000, 256] - [400000, 1]
+// 149 against 229; f64 [8192, 256] + [256] 6.9 against 7.4.
+static EwKind untiled_kind(const Dims& d, int ops) {
+    bool flat = is_flat(d, 0);
+    for (int k = 1; k <= 2; ++k)
+        if (ops >> (k - 1) & 1) flat = flat && (d.st[0][k] == 0 || d.st[0][k] == 1);
+    if (flat) return EwKind::Flat;
+    return d.shape[0] >= (uint64_t)(EW_BLOCK * EW_VEC) ? EwKind::Rows : EwKind::Generic;
+}
 
 // has_a / has_b: operand present as an array (not scalar / absent)
 static EwChoice choose(const Dims& d, bool has_a, bool has_b) {
@@ -367,44 +542,27 @@ static EwChoice choose(const Dims& d, bool has_a, bool has_b) {
         }
         return ch;
     }
-    if (d.shape[0] >= (uint64_t)(EW_BLOCK * EW_VEC)) ch.kind = EwKind::Rows;
+    ch.kind = untiled_kind(d, (has_a ? 1 : 0) | (has_b ? 2 : 0));
     return ch;
 }
 
 // Outputs at least this large are written with streaming stores: they cannot
 // stay in the 256 MB last-level cache for a following kernel anyway.
 constexpr uint64_t EW_NT_STORE_MIN = 128ull << 20;
+// The flat kernel's streaming hints: below, its operands were often written just before and lie in
+// the last-level cache, which hinted loads do not use (131 MB: 37 us without, 48 with hints; 410 MB:
+// 152 and 149, exp 132 and 124).
+constexpr uint64_t EW_NT_FLAT_MIN = 256ull << 20;
 // Tiled launches moving at least this many bytes have their tile order tuned.
 constexpr uint64_t EW_TUNE_MIN = 32ull << 20;
-
-// Call f(std::integral_constant<int, v>) for the runtime value v in [0, 8),
-// instantiating only masks whose load bits are operands the body has.
-template <int OPS, class F>
-static void with_ntm(int v, F&& f) {
-    auto one = [&](auto c) {
-        constexpr int V = decltype(c)::value;
-        if constexpr (((V & 3) & ~OPS) == 0) f(c);
-    };
-    switch (v & 7) {
-        case 0: one(std::integral_constant<int, 0>{}); break;
-        case 1: one(std::integral_constant<int, 1>{}); break;
-        case 2: one(std::integral_constant<int, 2>{}); break;
-        case 3: one(std::integral_constant<int, 3>{}); break;
-        case 4: one(std::integral_constant<int, 4>{}); break;
-        case 5: one(std::integral_constant<int, 5>{}); break;
-        case 6: one(std::integral_constant<int, 6>{}); break;
-        default: one(std::integral_constant<int, 7>{}); break;
-    }
-}
 
 // Launch `body` over the plan, splitting the outermost axis so that every
 // launch indexes fewer than 2^31 elements with 32-bit arithmetic.
 // TILED = false: the LDS-tiled kernel is not instantiated for this body, and a
 // tiled choice runs the generic kernel instead.
 // Streaming hints (compile-time kernel variants): loads of operands read once,
-// stores of outputs of at least EW_NT_STORE_MIN bytes. Bodies with NT_JOINT
-// take both hints or neither (fewer variants).
-// NTV = false: only the plain (hint-free) variant of the row kernel is instantiated, for bodies
+// stores of outputs of at least EW_NT_STORE_MIN bytes.
+// NTV = false: only the plain (hint-free) variant of the flat kernel is instantiated, for bodies
 // off the hot path.
 template <class Body, bool TILED = true, bool NTV = true>
 static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch, bool can_time = false) {
@@ -412,6 +570,9 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
     if (!TILED && ch.kind == EwKind::Tiled) ch.kind = EwKind::Generic;
     if (OPS == 0 && ch.kind == EwKind::Tiled) ch.kind = EwKind::Generic;
     if (d.nd < 0) return;
+    // a piece cut out of a contiguous output need not be contiguous any more; no output, no packs
+    if (ch.kind == EwKind::Flat && (d.nd < 1 || Body::OUT_SIZE == 0 || !is_flat(d, 0)))
+        ch.kind = d.nd >= 1 && d.shape[0] >= (uint64_t)(EW_BLOCK * EW_VEC) ? EwKind::Rows : EwKind::Generic;
     if (d.nd == 0) {
         d.nd = 1;
         d.shape.push_back(1);
@@ -457,8 +618,7 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
             if (d.shape[i] > 1 && d.st[i][k] == 0) once[k] = false;
     const bool big = Body::OUT_SIZE > 0 && all * Body::OUT_SIZE >= EW_NT_STORE_MIN;
     int lmask = ((OPS & 1) && once[1] ? 1 : 0) | ((OPS & 2) && once[2] ? 2 : 0);
-    int rows_ntm = lmask | (big ? 4 : 0);
-    if (Body::NT_JOINT) rows_ntm = (lmask == OPS && big) ? (OPS | 4) : 0;
+    const int flat_ntm = lmask != 0 && all * Body::OUT_SIZE >= EW_NT_FLAT_MIN ? (lmask | 4) : 0;
 
     uint64_t inner = 1;
     for (int i = 0; i + 1 < d.nd; ++i) inner *= d.shape[i];
@@ -481,24 +641,36 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
             uint64_t nrows = total / dd.shape[0];
             uint64_t nb = nrows * nchunk;
             if (nb >= LIM) RSTSR_RAISE(UnImplemented, "grid too large");
+            hipLaunchKernelGGL((k_ew_rows<Body, 0>), dim3((uint32_t)nb), dim3(EW_BLOCK), 0, ctx->stream, body, p, nchunk,
+                               FastDiv(nchunk));
+        } else if (ch.kind == EwKind::Flat) {
+          if constexpr (Body::OUT_SIZE > 0) {
+            constexpr size_t EA = sizeof(typename Body::TA), EB = sizeof(typename Body::TB);
+            constexpr size_t ES = std::max({(OPS & 1) ? EA : (size_t)1, (OPS & 2) ? EB : (size_t)1, Body::OUT_SIZE});
+            // two packs per thread for two operands: one leaves the second operand's index math and
+            // load latency uncovered (27 us against 17 above), four cost occupancy
+            constexpr int VEC = ES >= 16 ? 1 : (ES >= 8 ? 2 : 4), U = OPS == 3 ? 2 : 1;
+            const int same = (is_flat(dd, 1) ? 2 : 0) | (is_flat(dd, 2) ? 4 : 0);
+            const uint32_t nb = ceil_div_u32(total, (uint64_t)EW_BLOCK * U * VEC);
             auto go = [&](auto ntm) {
-                hipLaunchKernelGGL((k_ew_rows<Body, decltype(ntm)::value>), dim3((uint32_t)nb), dim3(EW_BLOCK), 0,
-                                   ctx->stream, body, p, nchunk, FastDiv(nchunk));
+                hipLaunchKernelGGL((k_ew_flat<Body, VEC, U, decltype(ntm)::value>), dim3(nb), dim3(EW_BLOCK), 0, ctx->stream,
+                                   body, p, (uint32_t)total, same);
             };
-            if constexpr (!NTV) {
+            if constexpr (!NTV || OPS == 0) {
                 go(std::integral_constant<int, 0>{});
-            } else if constexpr (Body::NT_JOINT) {
-                if (rows_ntm) go(std::integral_constant<int, OPS | 4>{});
-                else go(std::integral_constant<int, 0>{});
             } else {
-                with_ntm<OPS>(rows_ntm, go);
+                if (flat_ntm == 0) go(std::integral_constant<int, 0>{});
+                else if (flat_ntm == (OPS | 4)) go(std::integral_constant<int, OPS | 4>{});
+                else if (flat_ntm == 5) go(std::integral_constant<int, (OPS & 1) | 4>{});
+                else go(std::integral_constant<int, (OPS & 2) | 4>{});
             }
+          }
         } else if constexpr (TILED && OPS != 0) {
-            // tiles: 64x64 for 8-byte elements, 128 (input axis) x 64 for 4-byte and smaller, 32x32 for 16-byte
+            // tiles: 64x64 for 8-byte elements, 128 (input axis) x 64 for 4-byte and smaller, 32x64 for 16-byte
             constexpr size_t ES = sizeof(typename Body::TA) > sizeof(typename Body::TB) ? sizeof(typename Body::TA)
                                                                                           : sizeof(typename Body::TB);
             constexpr int TI = ES > 8 ? 32 : (ES > 4 ? 64 : 128);
-            constexpr int TC = ES > 8 ? 32 : 64;
+            constexpr int TC = 64;
             uint32_t ntc = ceil_div_u32(dd.shape[0], TC);
             uint32_t nti = ceil_div_u32(dd.shape[ch.di], TI);
             uint64_t nouter = total / (dd.shape[0] * dd.shape[ch.di]);
@@ -508,27 +680,46 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
             for (int k = 1; k < dd.nd; ++k)
                 if (k != ch.di) od = k;
 
-            int xmap = 0;
-            auto go = [&](auto stage, auto one, auto ntm) {
+            // Tile orders (xmap) and streaming hints (bit 0: staged loads, bit 1: stores). Rows whose
+            // tile segments start and end inside 128-byte lines share those lines with neighbouring
+            // tiles: hints would fetch or write them twice, so such launches choose among fewer hints,
+            // with orders that keep neighbours on one XCD.
+            int xmap = 0, hint = 0;
+            const bool edge = dd.shape[0] % TC != 0 || dd.shape[ch.di] % TI != 0;
+            auto go = [&](auto stage, auto one, auto ntm, auto eg) {
                 hipLaunchKernelGGL((k_ew_tiled<Body, TI, TC, decltype(stage)::value, decltype(one)::value,
-                                               decltype(ntm)::value>),
+                                               decltype(ntm)::value, decltype(eg)::value>),
                                    dim3((uint32_t)nb), dim3(EW_BLOCK), 0, ctx->stream, body, p, ch.di, od, nti, ntc,
                                    FastDiv(nti), FastDiv(ntc), xmap);
             };
-            // ONE (at most three axes): streaming variants, staged loads all-or-none; more axes: plain
+            // ONE (at most three axes): streaming variants, staged loads all-or-none, stores in launches
+            // of whole tiles only; more axes: plain
             auto by_nt = [&](auto stage) {
                 constexpr int S = decltype(stage)::value;
+                using Y = std::true_type;
+                using N = std::false_type;
                 if (dd.nd <= 3) {
                     const bool lo = ((S & 1) == 0 || once[1]) && ((S & 2) == 0 || once[2]);
-                    using Y = std::true_type;
-                    switch ((lo ? 1 : 0) | (big ? 2 : 0)) {
-                        case 0: go(stage, Y{}, std::integral_constant<int, 0>{}); break;
-                        case 1: go(stage, Y{}, std::integral_constant<int, S>{}); break;
-                        case 2: go(stage, Y{}, std::integral_constant<int, 4>{}); break;
-                        default: go(stage, Y{}, std::integral_constant<int, S | 4>{}); break;
+                    const int h = lo ? hint : hint & 2;
+                    if (edge) {
+                        if constexpr (Body::OUT_SIZE > 8) {
+                            if (h == 3) {
+                                go(stage, Y{}, std::integral_constant<int, S | 4>{}, Y{});
+                                return;
+                            }
+                        }
+                        if (h & 1) go(stage, Y{}, std::integral_constant<int, S>{}, Y{});
+                        else go(stage, Y{}, std::integral_constant<int, 0>{}, Y{});
+                        return;
+                    }
+                    switch (h) {
+                        case 0: go(stage, Y{}, std::integral_constant<int, 0>{}, N{}); break;
+                        case 1: go(stage, Y{}, std::integral_constant<int, S>{}, N{}); break;
+                        case 2: go(stage, Y{}, std::integral_constant<int, 4>{}, N{}); break;
+                        default: go(stage, Y{}, std::integral_constant<int, S | 4>{}, N{}); break;
                     }
                 } else {
-                    go(stage, std::false_type{}, std::integral_constant<int, 0>{});
+                    go(stage, N{}, std::integral_constant<int, 0>{}, Y{});
                 }
             };
             // choose() tiles along an input's unit axis, so that input is always staged:
@@ -546,23 +737,50 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
                     }
                 }
             };
-            // The fastest tile order depends on how the shapes and strides meet the
+            // whole lines: the output's rows along dim 0 and the staged inputs' rows along the input axis
+            auto lines = [&](int k, int unit, size_t es) {
+                bool ok = dd.off[k] * (int64_t)es % 128 == 0 && dd.shape[unit] * es % 128 == 0;
+                for (int i = 0; i < dd.nd; ++i)
+                    if (i != unit) ok = ok && dd.st[i][k] * (int64_t)es % 128 == 0;
+                return ok;
+            };
+            bool whole = !edge && lines(0, 0, Body::OUT_SIZE);
+            if (ch.stage & 1) whole = whole && lines(1, ch.di, sizeof(typename Body::TA));
+            if (ch.stage & 2) whole = whole && lines(2, ch.di, sizeof(typename Body::TB));
+            // candidates {order, hints}. Rows cut inside lines, inputs in turn: f32 [333, 509, 255] <- its
+            // reverse (345 MB) 85 to 89 us with CUT, 130 and more with stores hinted; 16-byte elements
+            // (half as many rows per line) the other way round, c128 [31, 900, 700] <- its last two axes
+            // swapped (625 MB) 111 to 116 us hinted, 125 with CUT.
+            struct Cand {
+                int xmap, hint;
+            };
+            static constexpr Cand WHOLE[] = {{0, 3}, {1, 3}, {2, 3}, {3, 3}};
+            static constexpr Cand CUT[] = {{3, 0}, {3, 1}, {1, 1}, {1, 0}};
+            static constexpr Cand CUT16[] = {{1, 3}, {0, 3}, {2, 3}, {3, 3}};
+            constexpr bool WIDE = Body::OUT_SIZE > 8;
+            const Cand* cands = whole ? WHOLE : (WIDE ? CUT16 : CUT);
+            auto use = [&](int c) {
+                xmap = cands[c].xmap;
+                hint = cands[c].hint;
+                if ((whole || WIDE) && !big) hint &= 1;  // outputs that the last-level cache can hold are not streamed
+                launch();
+            };
+            // The fastest order depends on how the shapes and strides meet the
             // HBM channel interleave (measured: either order can win by 5-10 %), so it
             // is tuned per problem class on launches of at least EW_TUNE_MIN bytes.
             const uint64_t bytes = total * (sizeof(typename Body::TA) + Body::OUT_SIZE);
             if (can_time && per >= nlast && bytes >= EW_TUNE_MIN) {
-                std::string key = "ew|" + std::to_string(sizeof(typename Body::TA)) + "|" +
+                std::string key = std::string(whole ? "ew|" : "ew|c|") + std::to_string(sizeof(typename Body::TA)) + "|" +
                                   std::to_string(Body::OUT_SIZE) + "|" + std::to_string(ch.stage) + "|" +
                                   std::to_string(ntc) + "|" + std::to_string(nti) + "|" + std::to_string(nouter) +
                                   "|" + std::to_string(dd.st[0][1] + dd.st[0][2]) + "|" +
                                   std::to_string(dd.st[ch.di][0]);
-                tune_select(ctx, key, 3, 0, true, [&](int c) {
-                    xmap = c;
-                    launch();
+                tune_select(ctx, key, 4, 0, true, [&](int c) {
+                    use(c);
                     check_launch("elementwise");
                 });
             } else {
-                launch();
+                use(0);
             }
         }
         check_launch("elementwise");

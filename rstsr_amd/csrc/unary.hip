@@ -316,13 +316,14 @@ struct UnBody {
     const TAv* a;
     static constexpr int OPS = 1;
     static constexpr size_t OUT_SIZE = sizeof(TCv);
-    static constexpr bool NT_JOINT = true;
     template <bool NT = false>
     __device__ __forceinline__ TAv la(int64_t o) const { return ld<NT>(a + o); }
     template <bool NT = false>
     __device__ __forceinline__ None lb(int64_t) const { return None{}; }
     template <bool NT = false>
     __device__ __forceinline__ void st(int64_t o, TAv x, None) const { sto<NT>(c + o, un_apply<OP, TCv, TAv>(x)); }
+    using TO = TCv;
+    __device__ __forceinline__ TCv val(TAv x, None) const { return un_apply<OP, TCv, TAv>(x); }
 };
 
 // integer -> f64 conversion (DTypeIntoFloatAPI::into_float = `as f64`)
@@ -334,13 +335,14 @@ struct ToF64Body {
     const TAv* a;
     static constexpr int OPS = 1;
     static constexpr size_t OUT_SIZE = sizeof(double);
-    static constexpr bool NT_JOINT = true;
     template <bool NT = false>
     __device__ __forceinline__ TAv la(int64_t o) const { return ld<NT>(a + o); }
     template <bool NT = false>
     __device__ __forceinline__ None lb(int64_t) const { return None{}; }
     template <bool NT = false>
     __device__ __forceinline__ void st(int64_t o, TAv x, None) const { sto<NT>(c + o, (double)x); }
+    using TO = double;
+    __device__ __forceinline__ double val(TAv x, None) const { return (double)x; }
 };
 
 /* =============================== host side =============================== */
