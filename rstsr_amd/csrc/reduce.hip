@@ -18,11 +18,11 @@
 //    total order, so the result does not depend on how work is split.
 //
 // Kernels (host planning in reduce_plan):
-//  - row: one 64-lane wave per (output, split); lanes stride a unit-stride
-//    reduced axis (coalesced 512 B per load wave), wave shuffles combine;
-//  - col: one thread per (output, split) with outputs along the input's
-//    unit-stride kept axis (coalesced across lanes), sequential over the
-//    reduced range;
+//  - row: a group of 16 or 64 lanes per (output, split), by the row's length; lanes
+//    stride a unit-stride reduced axis with 16-byte loads, group shuffles combine;
+//  - col: lanes along the outputs on the input's unit-stride kept axis
+//    (coalesced), sequential over a part of the reduced range; few parts are the
+//    waves of one block, many the blocks along grid y;
 //  - finalize: combine the split partials of each output in fixed order.
 // Built with -ffp-contract=off so that TwoSum is not fused or reassociated.
 #include <array>
@@ -368,6 +368,7 @@ struct RedPlan {
     // row kernel segmentation of the reduced space: units = rows(rest) x nseg0
     uint32_t seg0 = 1, nseg0 = 1;
     uint64_t units = 1, upw = 1;  // units per split
+    int ks = 1;                   // column kernel: waves per block that share the reduced range
     int stream = 0;               // every input element is read once: streaming loads
 };
 
@@ -412,26 +413,46 @@ __host__ __device__ constexpr int col_unroll(int lane_bytes) {
 }
 __host__ __device__ constexpr int col_waves_per_cu(int lane_bytes) { return col_unroll(lane_bytes) > 4 ? 4 : 8; }
 
-// VEC consecutive elements loaded as one aligned access
+// VEC consecutive elements
 template <class T, int VEC>
 struct alignas(sizeof(T) * VEC) Pack {
     T v[VEC];
 };
 
-// One wave per (output, split) over rows of the unit-stride reduced axis; each
-// lane loads VEC consecutive elements per access (16-byte loads when the host
-// proved alignment), four accesses in flight per iteration.
-template <class A, class T, int VEC>
+// A pack at an address of its element's alignment: one 16-byte load whatever the row's alignment.
+template <class T, int VEC, bool NT>
+__device__ __forceinline__ Pack<T, VEC> ld_pack(const T* p) {
+    Pack<T, VEC> r;
+    if constexpr (VEC == 1) {
+        r.v[0] = ld<NT>(p);
+    } else {
+        constexpr int W = sizeof(T) * VEC / 4;
+        typedef uint32_t Word __attribute__((ext_vector_type(W), aligned(4)));
+        Word w;
+        if constexpr (NT) w = __builtin_nontemporal_load((const Word*)p);
+        else w = *(const Word*)p;
+        __builtin_memcpy(&r, &w, sizeof(r));
+    }
+    return r;
+}
+
+// A group of G = 16 or 64 lanes per (output, split) over rows of the unit-stride reduced axis; each lane loads
+// VEC consecutive elements per access, four accesses in flight (also in a short or last part of a
+// row: addresses past the end repeat the last pack, whose elements are not counted twice).
+// G: short rows leave most of a 64-lane wave without an element and pay the shuffle tree per row, so
+// they share a wave. Bound by HBM for long rows; for short ones by the loads in flight and the tree
+// (50021 rows of 233 f32: max 21 us and sum 31 us with a wave per row, 11 and 14 us with 16 lanes).
+template <class A, class T, int VEC, int G>
 __global__ void __launch_bounds__(RB) k_red_row(const T* __restrict__ a, typename A::Out* out,
                                                 typename A::S* part, RedPlan p) {
     using S = typename A::S;
     using vt = Pack<T, VEC>;
-    const uint32_t wave = blockIdx.x * (RB / 64) + (threadIdx.x >> 6);
-    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t grp = blockIdx.x * (RB / G) + threadIdx.x / G;
+    const uint32_t lane = threadIdx.x % G;
     const uint64_t nwork = (uint64_t)p.M * p.nsplit;
-    if (wave >= nwork) return;  // whole wave exits together; no block barrier below
-    const uint32_t o = fdiv(wave, p.fsplit);
-    const uint32_t sp = wave - o * p.nsplit;
+    if (grp >= nwork) return;  // whole group exits together; no block barrier below
+    const uint32_t o = fdiv(grp, p.fsplit);
+    const uint32_t sp = grp - o * p.nsplit;
     int64_t oin, oout;
     kept_offsets(p, o, oin, oout);
     S acc = A::init();
@@ -440,17 +461,12 @@ __global__ void __launch_bounds__(RB) k_red_row(const T* __restrict__ a, typenam
     const int64_t s0 = p.rin[0];
     const uint64_t l0 = (uint64_t)p.rlog[0];
     const uint32_t L0 = (uint32_t)p.rshape[0];
-    constexpr uint32_t W = 64 * VEC;  // elements per wave access
+    constexpr uint32_t W = G * VEC;  // elements per group access
     auto sweep = [&](auto nt) {
         constexpr bool NT = decltype(nt)::value;
         auto get = [&](const T* base, uint32_t e) -> vt {
-            if constexpr (VEC == 1) {
-                vt x;
-                x.v[0] = ld<NT>(base + (int64_t)e * s0);
-                return x;
-            } else {
-                return ld<NT>((const vt*)(base + e));  // s0 == 1 on this path
-            }
+            if constexpr (VEC == 1) return ld_pack<T, 1, NT>(base + (int64_t)e * s0);
+            else return ld_pack<T, VEC, NT>(base + e);  // s0 == 1 on this path
         };
         for (uint64_t u = u0; u < u1; ++u) {
             uint64_t row = u / p.nseg0;
@@ -460,46 +476,43 @@ __global__ void __launch_bounds__(RB) k_red_row(const T* __restrict__ a, typenam
             row_offsets(p, row, roff, rli);
             const T* base = a + oin + roff;
             uint32_t e = seg * p.seg0 + lane * VEC;
-            uint32_t eend = min(L0, (seg + 1) * p.seg0);
-            if constexpr (is_arg<A>()) {
-                // positions increase with the logical index inside a row (l0 > 0)
-                T bv{};
-                uint32_t be = ~0u;
-                for (; e + 3 * W < eend; e += 4 * W) {
-                    vt x0 = get(base, e), x1 = get(base, e + W), x2 = get(base, e + 2 * W), x3 = get(base, e + 3 * W);
-#pragma unroll
-                    for (int v = 0; v < VEC; ++v) A::scan(x0.v[v], e + v, bv, be);
-#pragma unroll
-                    for (int v = 0; v < VEC; ++v) A::scan(x1.v[v], e + W + v, bv, be);
-#pragma unroll
-                    for (int v = 0; v < VEC; ++v) A::scan(x2.v[v], e + 2 * W + v, bv, be);
-#pragma unroll
-                    for (int v = 0; v < VEC; ++v) A::scan(x3.v[v], e + 3 * W + v, bv, be);
-                }
-                for (; e < eend; e += W) {
-                    vt x = get(base, e);
-#pragma unroll
-                    for (int v = 0; v < VEC; ++v) A::scan(x.v[v], e + v, bv, be);
-                }
-                if (be != ~0u) A::add(acc, bv, rli + (uint64_t)be * l0);
-                continue;
-            }
-            for (; e + 3 * W < eend; e += 4 * W) {
+            const uint32_t eend = min(L0, (seg + 1) * p.seg0);
+            // argmin/argmax: positions increase with the logical index inside a row (l0 > 0)
+            T bv{};
+            uint32_t be = ~0u;
+            auto take = [&](T x, uint32_t at) {
+                if constexpr (is_arg<A>()) A::scan(x, at, bv, be);
+                else A::add(acc, x, rli + (uint64_t)at * l0);
+            };
+            for (; e + 3 * W + VEC <= eend; e += 4 * W) {
                 vt x0 = get(base, e), x1 = get(base, e + W), x2 = get(base, e + 2 * W), x3 = get(base, e + 3 * W);
 #pragma unroll
-                for (int v = 0; v < VEC; ++v) A::add(acc, x0.v[v], rli + (uint64_t)(e + v) * l0);
+                for (int v = 0; v < VEC; ++v) take(x0.v[v], e + v);
 #pragma unroll
-                for (int v = 0; v < VEC; ++v) A::add(acc, x1.v[v], rli + (uint64_t)(e + W + v) * l0);
+                for (int v = 0; v < VEC; ++v) take(x1.v[v], e + W + v);
 #pragma unroll
-                for (int v = 0; v < VEC; ++v) A::add(acc, x2.v[v], rli + (uint64_t)(e + 2 * W + v) * l0);
+                for (int v = 0; v < VEC; ++v) take(x2.v[v], e + 2 * W + v);
 #pragma unroll
-                for (int v = 0; v < VEC; ++v) A::add(acc, x3.v[v], rli + (uint64_t)(e + 3 * W + v) * l0);
+                for (int v = 0; v < VEC; ++v) take(x3.v[v], e + 3 * W + v);
             }
-            for (; e < eend; e += W) {
-                vt x = get(base, e);
+            if (e + VEC <= eend) {
+                const uint32_t last = eend - VEC;
+                vt x[3];
 #pragma unroll
-                for (int v = 0; v < VEC; ++v) A::add(acc, x.v[v], rli + (uint64_t)(e + v) * l0);
+                for (int q = 0; q < 3; ++q) x[q] = get(base, min(e + q * W, last));
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+                    if (e + q * W <= last)
+#pragma unroll
+                        for (int v = 0; v < VEC; ++v) take(x[q].v[v], e + q * W + v);
             }
+            // the elements after the last whole pack
+            if constexpr (VEC > 1) {
+                const uint32_t rest = eend / VEC * VEC + lane;
+                if (rest < eend) take(base[rest], rest);
+            }
+            if constexpr (is_arg<A>())
+                if (be != ~0u) A::add(acc, bv, rli + (uint64_t)be * l0);
         }
     };
     // streaming loads pay off for 8-byte and wider elements; narrower ones (also as
@@ -507,7 +520,7 @@ __global__ void __launch_bounds__(RB) k_red_row(const T* __restrict__ a, typenam
     if (sizeof(T) >= 8 && p.stream) sweep(std::true_type{});
     else sweep(std::false_type{});
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
+    for (int m = G / 2; m >= 1; m >>= 1) {
         S other = A::shfl(acc, m);
         // lower lane's partial precedes the higher lane's
         acc = (lane & m) ? A::combine(other, acc) : A::combine(acc, other);
@@ -518,28 +531,32 @@ __global__ void __launch_bounds__(RB) k_red_row(const T* __restrict__ a, typenam
     }
 }
 
-// VEC adjacent outputs per thread along the unit-stride kept axis (VEC * sizeof(T)
-// = 16 B vector loads when the host proved alignment), sequential over the reduced range.
-template <class A, class T, int VEC>
-__global__ void __launch_bounds__(RB) k_red_col(const T* __restrict__ a, typename A::Out* out,
+// VEC adjacent outputs per thread along the unit-stride kept axis, sequential over a part of the
+// reduced range. KS = 1: four waves side by side, parts along blockIdx.y, partials combined by
+// k_red_fin. KS = 16: the waves of a block share its 64 VEC outputs, a part each, combined in order
+// through LDS, so that a reduction with few parts needs no second launch ([64, 128, 256] f64 over
+// axis 1: 16.2 -> 7.7 us in all; for many parts splitting inside the block measured 2 % slower).
+template <class A, class T, int VEC, int KS>
+__global__ void __launch_bounds__(KS == 1 ? RB : 64 * KS) k_red_col(const T* __restrict__ a, typename A::Out* out,
                                                 typename A::S* part, RedPlan p) {
     using S = typename A::S;
     using vt = Pack<T, VEC>;
     constexpr int COLU = col_unroll((int)(sizeof(T) * VEC));
-    const uint64_t t = (uint64_t)blockIdx.x * RB + threadIdx.x;
-    const uint32_t MV = p.M / VEC;
-    if (t >= (uint64_t)MV * p.nsplit) return;
-    const uint32_t sp = (uint32_t)(t / MV);
-    const uint32_t o = (uint32_t)(t - (uint64_t)sp * MV) * VEC;
+    __shared__ S red[KS > 1 ? KS : 1][KS > 1 ? 64 * VEC : 1];
+    const uint32_t lane = threadIdx.x & 63, wave = KS > 1 ? threadIdx.x >> 6 : 0;
+    const uint64_t mv = KS > 1 ? (uint64_t)blockIdx.x * 64 + lane : (uint64_t)blockIdx.x * RB + threadIdx.x;
+    const uint32_t sp = blockIdx.y;
+    const bool active = mv < p.M / VEC;
+    const uint32_t o = active ? (uint32_t)mv * VEC : 0;
     int64_t oin, oout;
     kept_offsets(p, o, oin, oout);
     S acc[VEC];
 #pragma unroll
     for (int v = 0; v < VEC; ++v) acc[v] = A::init();
-    const uint64_t chunk = p.upw;  // reduced elements per split
-    uint64_t r0 = (uint64_t)sp * chunk;
+    const uint64_t chunk = p.upw;  // reduced elements per part
+    uint64_t r0 = ((uint64_t)sp * KS + wave) * chunk;
     uint64_t r1 = min(p.R, r0 + chunk);
-    if (r0 < r1) {
+    if (active && r0 < r1) {
         // unravel the start position over the reduced dims
         uint64_t coord[MAXD];
         int64_t off = 0;
@@ -574,14 +591,14 @@ __global__ void __launch_bounds__(RB) k_red_col(const T* __restrict__ a, typenam
                 for (; j + COLU <= n; j += COLU) {
                     vt x[COLU];
 #pragma unroll
-                    for (int q = 0; q < COLU; ++q) x[q] = ld<NT>((const vt*)(rowp + (int64_t)(j + q) * s0));
+                    for (int q = 0; q < COLU; ++q) x[q] = ld_pack<T, VEC, NT>(rowp + (int64_t)(j + q) * s0);
 #pragma unroll
                     for (int q = 0; q < COLU; ++q)
 #pragma unroll
                         for (int v = 0; v < VEC; ++v) A::scan(x[q].v[v], (uint32_t)(j + q), bv[v], be[v]);
                 }
                 for (; j < n; ++j) {
-                    vt x = ld<NT>((const vt*)(rowp + (int64_t)j * s0));
+                    vt x = ld_pack<T, VEC, NT>(rowp + (int64_t)j * s0);
 #pragma unroll
                     for (int v = 0; v < VEC; ++v) A::scan(x.v[v], (uint32_t)j, bv[v], be[v]);
                 }
@@ -593,14 +610,14 @@ __global__ void __launch_bounds__(RB) k_red_col(const T* __restrict__ a, typenam
             for (; j + COLU <= n; j += COLU) {
                 vt x[COLU];
 #pragma unroll
-                for (int q = 0; q < COLU; ++q) x[q] = ld<NT>((const vt*)(rowp + (int64_t)(j + q) * s0));
+                for (int q = 0; q < COLU; ++q) x[q] = ld_pack<T, VEC, NT>(rowp + (int64_t)(j + q) * s0);
 #pragma unroll
                 for (int q = 0; q < COLU; ++q)
 #pragma unroll
                     for (int v = 0; v < VEC; ++v) A::add(acc[v], x[q].v[v], li + (j + q) * l0);
             }
             for (; j < n; ++j) {
-                vt x = ld<NT>((const vt*)(rowp + (int64_t)j * s0));
+                vt x = ld_pack<T, VEC, NT>(rowp + (int64_t)j * s0);
 #pragma unroll
                 for (int v = 0; v < VEC; ++v) A::add(acc[v], x.v[v], li + j * l0);
             }
@@ -628,6 +645,16 @@ __global__ void __launch_bounds__(RB) k_red_col(const T* __restrict__ a, typenam
             }
         }
     }
+    if constexpr (KS > 1) {
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) red[wave][lane * VEC + v] = acc[v];
+        __syncthreads();
+        if (wave != 0) return;
+#pragma unroll
+        for (int v = 0; v < VEC; ++v)
+            for (int w = 1; w < KS; ++w) acc[v] = A::combine(acc[v], red[w][lane * VEC + v]);
+    }
+    if (!active) return;
 #pragma unroll
     for (int v = 0; v < VEC; ++v) {
         // kept axis 0 has input stride +1 when VEC > 1
@@ -822,10 +849,11 @@ static RedSetup reduce_plan(rstsr_hip_ctx* ctx, const Layout& la, const std::vec
         const uint64_t vec = (uint64_t)col_vec(t);
         const uint64_t wpc = (uint64_t)col_waves_per_cu((int)(esize * vec));
         uint64_t want = std::max<uint64_t>(1, ((uint64_t)std::max(ctx->num_cu, 1) * wpc * 64 * vec) / M);
-        uint64_t nsplit = std::min<uint64_t>(want, std::max<uint64_t>(1, R / 64));
-        nsplit = std::min<uint64_t>(nsplit, 65536);
-        p.upw = (R + nsplit - 1) / nsplit;
-        nsplit = (R + p.upw - 1) / p.upw;
+        // two to sixteen parts of at least four positions: the waves of one block
+        p.ks = want > 1 && want <= 16 && R >= 64 ? 16 : 1;
+        uint64_t nsplit = p.ks > 1 ? 1 : std::min<uint64_t>({want, std::max<uint64_t>(1, R / 64), 65535});
+        p.upw = (R + nsplit * p.ks - 1) / (nsplit * p.ks);
+        nsplit = (R + p.upw * p.ks - 1) / (p.upw * p.ks);
         p.nsplit = (uint32_t)nsplit;
     }
     if ((uint64_t)p.M * p.nsplit >= (1ull << 32)) RSTSR_RAISE(UnImplemented, "reduction grid too large");
@@ -858,37 +886,40 @@ static void run_reduce(rstsr_hip_ctx* ctx, const RedSetup& s, const T* a, typena
             part = (S*)workspace(ctx, need);
         }
     }
-    // 16-byte loads when every address a thread touches is 16-byte aligned
+    // elements of a 16-byte load
     constexpr int V16 = (std::is_arithmetic<T>::value && (sizeof(T) == 8 || sizeof(T) == 4)) ? (int)(16 / sizeof(T)) : 1;
     if (s.kind == RedKind::Row) {
-        uint64_t nwaves = (uint64_t)p.M * p.nsplit;
-        uint32_t nb = ceil_div_u32(nwaves, RB / 64);
-        // rows start 16-byte aligned and run in whole 16-byte words
-        bool vec = V16 > 1 && p.rin[0] == 1 && p.rshape[0] % V16 == 0 && p.seg0 % V16 == 0 &&
-                   (p.in_off % V16) == 0 && ((uintptr_t)a % 16) == 0;
-        for (int d = 0; d < p.nk && vec; ++d) vec = (p.kin[d] % V16) == 0;
-        for (int d = 1; d < p.nr && vec; ++d) vec = (p.rin[d] % V16) == 0;
-        if (vec)
-            hipLaunchKernelGGL((k_red_row<A, T, V16>), dim3(nb), dim3(RB), 0, ctx->stream, a, out, part, p);
-        else
-            hipLaunchKernelGGL((k_red_row<A, T, 1>), dim3(nb), dim3(RB), 0, ctx->stream, a, out, part, p);
+        const uint64_t ngroups = (uint64_t)p.M * p.nsplit;
+        auto go = [&](auto vec, auto g) {
+            constexpr int V = decltype(vec)::value, G = decltype(g)::value;
+            hipLaunchKernelGGL((k_red_row<A, T, V, G>), dim3(ceil_div_u32(ngroups, RB / G)), dim3(RB), 0, ctx->stream, a,
+                               out, part, p);
+        };
+        // short rows: 16 lanes each, unless that leaves the chip short of waves
+        auto by_group = [&](auto vec) {
+            const uint64_t packs = p.rshape[0] / decltype(vec)::value, full = (uint64_t)std::max(ctx->num_cu, 1) * 8;
+            if (packs < 128 && ngroups * 16 >= full * 64) go(vec, std::integral_constant<int, 16>{});
+            else go(vec, std::integral_constant<int, 64>{});
+        };
+        // whole 16-byte packs along the row (any alignment)
+        if (V16 > 1 && p.rin[0] == 1 && p.rshape[0] >= V16) by_group(std::integral_constant<int, V16>{});
+        else by_group(std::integral_constant<int, 1>{});
     } else {
         // column kernel: two outputs per thread for 4-byte elements too (8-byte loads), so a
         // split covers the same number of lanes as for 8-byte elements
         constexpr int VC = V16 > 2 ? 2 : V16;
-        bool vec = VC > 1 && p.nk >= 1 && p.kin[0] == 1 && p.kshape[0] % VC == 0 && p.M % VC == 0 &&
-                   (p.in_off % VC) == 0 && ((uintptr_t)a % (VC * sizeof(T))) == 0;
-        for (int d = 1; d < p.nk && vec; ++d) vec = (p.kin[d] % VC) == 0;
-        for (int d = 0; d < p.nr && vec; ++d) vec = (p.rin[d] % VC) == 0;
-        if (vec) {
-            uint64_t nthr = (uint64_t)(p.M / VC) * p.nsplit;
-            hipLaunchKernelGGL((k_red_col<A, T, VC>), dim3(ceil_div_u32(nthr, RB)), dim3(RB), 0, ctx->stream, a, out,
-                               part, p);
-        } else {
-            uint64_t nthr = (uint64_t)p.M * p.nsplit;
-            hipLaunchKernelGGL((k_red_col<A, T, 1>), dim3(ceil_div_u32(nthr, RB)), dim3(RB), 0, ctx->stream, a, out,
-                               part, p);
-        }
+        const bool vec = VC > 1 && p.nk >= 1 && p.kin[0] == 1 && p.kshape[0] % VC == 0 && p.M % VC == 0;
+        auto go = [&](auto v, auto ks) {
+            constexpr int V = decltype(v)::value, KS = decltype(ks)::value;
+            hipLaunchKernelGGL((k_red_col<A, T, V, KS>), dim3(ceil_div_u32(p.M / V, KS == 1 ? RB : 64), p.nsplit),
+                               dim3(KS == 1 ? RB : 64 * KS), 0, ctx->stream, a, out, part, p);
+        };
+        auto by_ks = [&](auto v) {
+            if (p.ks == 1) go(v, std::integral_constant<int, 1>{});
+            else go(v, std::integral_constant<int, 16>{});
+        };
+        if (vec) by_ks(std::integral_constant<int, VC>{});
+        else by_ks(std::integral_constant<int, 1>{});
     }
     check_launch("reduce");
     if (p.nsplit > 1) {
