@@ -41,33 +41,6 @@ struct GemmArgs {
     BatchDesc bd;
 };
 
-// Symmetric product (A = B^T, same buffer): copy the transpose of every 64 x 64
-// tile on and below the diagonal onto its mirror, through LDS so both the reads
-// and the writes run along C's rows; only elements strictly above the diagonal
-// are written, so C comes out exactly symmetric. Batch from blockIdx.y.
-template <class T>
-__global__ void __launch_bounds__(256) k_mirror(GemmArgs<T> g) {
-    __shared__ T tile[64][65];
-    uint32_t ti, tj;
-    tri_coords(blockIdx.x, 0, ti, tj);
-    int64_t oa, ob, oc;
-    batch_offsets(g.bd, g.batch0 + blockIdx.y, oa, ob, oc);
-    T* C = g.c + oc;
-    const int tid = threadIdx.x, c = tid & 63, r0 = tid >> 6;
-    const int64_t i0 = (int64_t)ti * 64, j0 = (int64_t)tj * 64;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-        const int r = r0 + 4 * k;
-        if (i0 + r < g.M && j0 + c < g.N) tile[r][c] = C[(i0 + r) * g.rsc + (j0 + c) * g.csc];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-        const int r = r0 + 4 * k;  // row j0 + r of the upper tile, column i0 + c
-        if (j0 + r < g.N && i0 + c < g.M && i0 + c > j0 + r) C[(j0 + r) * g.rsc + (i0 + c) * g.csc] = tile[c][r];
-    }
-}
-
 /* ---------------- SIMT kernel: i32, i64 ---------------- */
 
 template <class T>
@@ -125,17 +98,6 @@ __global__ void __launch_bounds__(256) k_gemm_simt(GemmArgs<T> g) {
 
 /* ---------------- host side ---------------- */
 
-// Copy the lower triangle of nb batches (from g.batch0) onto the upper one.
-template <class T>
-static void mirror_batches(rstsr_hip_ctx* ctx, const GemmArgs<T>& g, uint32_t nb) {
-    const uint64_t t64 = ceil_div_u32(g.M, 64);
-    const uint64_t nm = t64 * (t64 + 1) / 2;
-    if (nm >= (1ull << 31)) RSTSR_RAISE(UnImplemented, "symmetric product too large");
-    if (nm == 0) return;
-    hipLaunchKernelGGL(k_mirror<T>, dim3((uint32_t)nm, nb), dim3(256), 0, ctx->stream, g);
-    check_launch("gemm mirror");
-}
-
 template <class T>
 static void launch_gemm_t(rstsr_hip_ctx* ctx, const GemmProblem& P, T alpha, T beta, bool beta_zero,
                           const int* run_if = nullptr) {
@@ -159,18 +121,14 @@ static void launch_gemm_t(rstsr_hip_ctx* ctx, const GemmProblem& P, T alpha, T b
     if constexpr (!std::is_integral<T>::value) {
         // SYRK shortcut (device_faer/matmul.rs:38-48): beta = 0 and A is B's transpose
         // in the same buffer, so C is symmetric. Only the tiles on and below the
-        // diagonal are multiplied; the rest is mirrored. For real types C[i][j] and
+        // diagonal are multiplied, and stored twice. For real types C[i][j] and
         // C[j][i] sum the same products in the same K order, so the mirror equals the
         // full product bit for bit; for complex the imaginary part's two products
         // swap order, and the mirror makes the result exactly symmetric.
-        auto mirror = [&](uint64_t b0, uint32_t nb) {
-            g.batch0 = (uint32_t)b0;
-            mirror_batches<T>(ctx, g, nb);
-        };
-        if constexpr (std::is_same<T, float>::value) tile_gemm_f32(ctx, P, alpha, beta, beta_zero, mirror);
-        else if constexpr (std::is_same<T, c64>::value) tile_gemm_c64(ctx, P, alpha, beta, beta_zero, mirror);
-        else if constexpr (std::is_same<T, double>::value) tile_gemm_f64(ctx, P, alpha, beta, beta_zero, run_if, mirror);
-        else tile_gemm_c128(ctx, P, alpha, beta, beta_zero, run_if, mirror);
+        if constexpr (std::is_same<T, float>::value) tile_gemm_f32(ctx, P, alpha, beta, beta_zero);
+        else if constexpr (std::is_same<T, c64>::value) tile_gemm_c64(ctx, P, alpha, beta, beta_zero);
+        else if constexpr (std::is_same<T, double>::value) tile_gemm_f64(ctx, P, alpha, beta, beta_zero, run_if);
+        else tile_gemm_c128(ctx, P, alpha, beta, beta_zero, run_if);
     } else {
         const uint64_t YMAX = 65535;
         for (uint64_t b0 = 0; b0 < P.nbatch; b0 += YMAX) {

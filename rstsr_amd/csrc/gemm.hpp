@@ -88,17 +88,14 @@ inline void batch_offsets_host(const BatchDesc& bd, uint64_t bi, int64_t& oa, in
     }
 }
 
-// Copies the lower triangle onto the upper one for batches [b0, b0 + nb) of a symmetric product.
-using MirrorFn = std::function<void(uint64_t b0, uint32_t nb)>;
 // GEMM of one element type on the matrix cores (gemm_tile_*.hip). run_if (device, nullable): the
 // kernels exit unless *run_if != 0.
-void tile_gemm_f32(rstsr_hip_ctx* ctx, const GemmProblem& P, float alpha, float beta, bool beta_zero,
-                   const MirrorFn& mirror);
-void tile_gemm_c64(rstsr_hip_ctx* ctx, const GemmProblem& P, c64 alpha, c64 beta, bool beta_zero, const MirrorFn& mirror);
+void tile_gemm_f32(rstsr_hip_ctx* ctx, const GemmProblem& P, float alpha, float beta, bool beta_zero);
+void tile_gemm_c64(rstsr_hip_ctx* ctx, const GemmProblem& P, c64 alpha, c64 beta, bool beta_zero);
 void tile_gemm_f64(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, double beta, bool beta_zero,
-                   const int* run_if, const MirrorFn& mirror);
+                   const int* run_if);
 void tile_gemm_c128(rstsr_hip_ctx* ctx, const GemmProblem& P, c128 alpha, c128 beta, bool beta_zero,
-                    const int* run_if, const MirrorFn& mirror);
+                    const int* run_if);
 // Products with one row or one column (gemv.hip); false when the problem is not one it takes.
 bool gemv(rstsr_hip_ctx* ctx, rstsr_dtype_t t, const GemmProblem& P, const void* alpha, const void* beta, bool beta_zero);
 // Grouped (uneven) GEMMs, one launch per operand form: problems without batches, with M, N, K > 0 and

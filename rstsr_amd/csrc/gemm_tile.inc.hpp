@@ -127,7 +127,7 @@ static int tile_shape_index(int bm) {
 
 template <class T>
 static void tile_gemm_run(rstsr_hip_ctx* ctx, const char* tag, const GemmProblem& P, T alpha, T beta, bool beta_zero,
-                          const int* run_if, const MirrorFn& mirror) {
+                          const int* run_if) {
     using S = TileShapes<T>;
     TileGemmArgs<T> g;
     g.M = P.M;
@@ -165,10 +165,10 @@ static void tile_gemm_run(rstsr_hip_ctx* ctx, const char* tag, const GemmProblem
         g.part = (typename ElemOf<T>::R*)workspace(ctx, (size_t)nsplit * nb * P.M * P.N * sizeof(T));
         if (v16) tile_gemm_launch<T, TileMid<T>, true, true>(ctx, g, nb, nsplit, ak, bk, run_if);
         else tile_gemm_launch<T, TileMid<T>, false, true>(ctx, g, nb, nsplit, ak, bk, run_if);
+        g.tri = syrk ? 1 : 0;
         hipLaunchKernelGGL(k_gemm_split_fin<T>, dim3(ceil_div_u32((uint64_t)P.M * P.N, 256), nb), dim3(256), 0,
                            ctx->stream, g, (int)nsplit, nb, run_if);
         check_launch("gemm split");
-        if (syrk && ElemOf<T>::CX) mirror(0, nb);
         return;
     }
     auto run = [&](int c) {
@@ -184,7 +184,6 @@ static void tile_gemm_run(rstsr_hip_ctx* ctx, const char* tag, const GemmProblem
             else if (c == 1) go(typename S::S1{});
             else if (c == 2) go(typename S::S2{});
             else go(typename S::S3{});
-            if (syrk) mirror(b0, nb);
         }
     };
     // untuned: the largest tile that still gives every CU a block

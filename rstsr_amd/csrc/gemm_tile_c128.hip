@@ -5,8 +5,8 @@ namespace rstsr {
 namespace hip {
 
 void tile_gemm_c128(rstsr_hip_ctx* ctx, const GemmProblem& P, c128 alpha, c128 beta, bool beta_zero,
-                   const int* run_if, const MirrorFn& mirror) {
-    tile_gemm_run<c128>(ctx, "z2", P, alpha, beta, beta_zero, run_if, mirror);
+                   const int* run_if) {
+    tile_gemm_run<c128>(ctx, "z2", P, alpha, beta, beta_zero, run_if);
 }
 
 void tile_grouped_c128(rstsr_hip_ctx* ctx, const std::vector<GemmProblem>& probs, c128 alpha, c128 beta,

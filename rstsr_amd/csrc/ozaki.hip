@@ -1823,7 +1823,7 @@ void ozaki_gemm_f64(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, doub
         check_launch("ozaki crt");
     } else {
         // symmetric product: the lower tiles' CRT writes each tile's mirror too (RI 24000^2:
-        // 1.70-1.86 ms against 1.77-1.95 ms for the row CRT plus 1.07-1.09 ms for k_mirror)
+        // 1.70-1.86 ms against 1.77-1.95 ms for the row CRT plus 1.07-1.09 ms for a mirror kernel)
         using CT = CrtTile<128>;
         const uint64_t tmt = (uint64_t)((M + CT::TR - 1) / CT::TR), tnt = (uint64_t)((N + CT::TC - 1) / CT::TC);
         const uint64_t ntl = lower_tile_prefix(tmt, (uint64_t)(CT::TC / CT::TR));
