@@ -196,10 +196,13 @@ static bool is_zero_scalar(rstsr_dtype_t t, const void* v) {
     }
 }
 
-// S (rows x cols, dense row-major) = Re X + Im X for a strided complex matrix X
+// S (rows x cols, dense row-major) = Re X + Im X for a strided complex matrix X. run_if as for
+// plain_dgemm.
 __global__ void __launch_bounds__(256) k_zsum_parts(double* __restrict__ S, double* __restrict__ Xr,
                                                     double* __restrict__ Xi, const c128* __restrict__ X, int64_t rows,
-                                                    int64_t cols, int64_t rs, int64_t cs) {
+                                                    int64_t cols, int64_t rs, int64_t cs,
+                                                    const int* __restrict__ run_if) {
+    if (run_if && *run_if == 0) return;
     // row blockIdx.y (grid-strided), columns along the block: S = re + im, and the real and
     // imaginary planes as contiguous rows (the split then reads them once, at unit stride)
     for (int64_t i = blockIdx.y; i < rows; i += gridDim.y) {
@@ -217,7 +220,9 @@ __global__ void __launch_bounds__(256) k_zsum_parts(double* __restrict__ S, doub
 // C holds (a T1, a T3) with T1 = Ar Br, T3 = (Ar + Ai)(Br + Bi); T2 = a Ai Bi (dense M x N).
 // C = (a T1 - a T2, a T3 - a T1 - a T2).
 __global__ void __launch_bounds__(256) k_z3m_combine(c128* __restrict__ C, int64_t rsc, int64_t csc,
-                                                     const double* __restrict__ T2, int64_t M, int64_t N) {
+                                                     const double* __restrict__ T2, int64_t M, int64_t N,
+                                                     const int* __restrict__ run_if) {
+    if (run_if && *run_if == 0) return;
     const int64_t n = M * N;
     for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
         const int64_t i = e / N, j = e - i * N;
@@ -228,75 +233,77 @@ __global__ void __launch_bounds__(256) k_z3m_combine(c128* __restrict__ C, int64
     }
 }
 
-// Complex split GEMM from real split products on the real/imaginary planes
-// (stride-2 double views). With beta = 0 and one matrix: three products (below);
-// otherwise four: Cr = a ArBr - a AiBi + b Cr, Ci = a ArBi + a AiBr + b Ci.
+// The three-product form of a complex product (ozaki_zgemm3) by real products of the parts, which
+// lie in `z` (Zgemm3Parts): split products, or with run_if plain ones that run if *run_if != 0.
+struct Zgemm3Parts {
+    size_t nA, nB, nT;  // doubles, each a multiple of 256 bytes
+    explicit Zgemm3Parts(const GemmProblem& P) {
+        auto al = [](int64_t x) { return ((size_t)x + 31) & ~(size_t)31; };
+        nA = al(P.M * P.K);
+        nB = al(P.K * P.N);
+        nT = al(P.M * P.N);
+    }
+    size_t bytes() const { return (3 * nA + 3 * nB + nT) * sizeof(double); }
+};
+
+static void zgemm3_products(rstsr_hip_ctx* ctx, const GemmProblem& P, double a, char* z, const int* run_if) {
+    const int64_t M = P.M, N = P.N, K = P.K;
+    // the sums Ar + Ai and Br + Bi, T2, and the four parts as contiguous planes
+    const Zgemm3Parts s(P);
+    double* SA = (double*)z;
+    double* SB = SA + s.nA;
+    double* T2 = SB + s.nB;
+    double* Ar = T2 + s.nT;
+    double* Ai = Ar + s.nA;
+    double* Br = Ai + s.nA;
+    double* Bi = Br + s.nB;
+    // launches that may not run stay small
+    const int64_t ymax = run_if ? 64 : 65535;
+    auto grid = [&](int64_t rows, int64_t cols) {
+        return dim3((uint32_t)std::min<int64_t>((cols + 255) / 256, 64), (uint32_t)std::min<int64_t>(rows, ymax));
+    };
+    hipLaunchKernelGGL(k_zsum_parts, grid(M, K), dim3(256), 0, ctx->stream, SA, Ar, Ai, (const c128*)P.a, M, K,
+                       P.rsa, P.csa, run_if);
+    hipLaunchKernelGGL(k_zsum_parts, grid(K, N), dim3(256), 0, ctx->stream, SB, Br, Bi, (const c128*)P.b, K, N,
+                       P.rsb, P.csb, run_if);
+    check_launch("complex split sums");
+    GemmProblem Q = P;
+    Q.bd.nbd = 0;
+    Q.nbatch = 1;
+    Q.rsa = K;
+    Q.csa = 1;
+    Q.rsb = N;
+    Q.csb = 1;
+    auto prod = [&](const double* x, const double* y, double* c, int64_t rsc, int64_t csc) {
+        Q.a = x;
+        Q.b = y;
+        Q.c = c;
+        Q.rsc = rsc;
+        Q.csc = csc;
+        if (run_if) plain_dgemm(ctx, Q, a, 0.0, true, run_if);
+        else ozaki_gemm_f64(ctx, Q, a, 0.0, true);
+    };
+    prod(Ar, Br, (double*)P.c, 2 * P.rsc, 2 * P.csc);      // T1 into Re C
+    prod(SA, SB, (double*)P.c + 1, 2 * P.rsc, 2 * P.csc);  // T3 into Im C
+    prod(Ai, Bi, T2, N, 1);
+    const size_t nT = (size_t)M * N;
+    hipLaunchKernelGGL(k_z3m_combine, dim3((uint32_t)std::min<size_t>((nT + 255) / 256, run_if ? 4096 : 65536)),
+                       dim3(256), 0, ctx->stream, (c128*)P.c, P.rsc, P.csc, T2, M, N, run_if);
+    check_launch("complex split combine");
+}
+
+// Complex split GEMM from real split products. With beta = 0 and one matrix: the three-product form,
+// in one run of the split kernels (ozaki_zgemm3) or, for the forms that does not take, one by one;
+// otherwise four on the real/imaginary planes (stride-2 double views): Cr = a ArBr - a AiBi + b Cr,
+// Ci = a ArBi + a AiBr + b Ci.
 static void ozaki_zgemm(rstsr_hip_ctx* ctx, const GemmProblem& P, c128 alpha, c128 beta, bool beta_zero) {
     if (alpha.im != 0.0 || beta.im != 0.0)
         RSTSR_RAISE(UnImplemented, "the complex split GEMM takes real alpha and beta");
     if (beta_zero && P.nbatch == 1 && P.bd.nbd == 0 && P.K > 0) {
-        // Three real split products (Karatsuba form): T1 = Ar Br, T2 = Ai Bi,
-        // T3 = (Ar + Ai)(Br + Bi); Re C = a (T1 - T2), Im C = a (T3 - T1 - T2).
-        // Each product is accurate to the split GEMM's normwise bound, so the
-        // result keeps it relative to (|Ar| + |Ai|)(|Br| + |Bi|).
-        const int64_t M = P.M, N = P.N, K = P.K;
-        const size_t nSA = (size_t)M * K, nSB = (size_t)K * N, nT = (size_t)M * N;
-        auto al = [](size_t x) { return (x * sizeof(double) + 255) & ~(size_t)255; };
-        // the sums Ar + Ai and Br + Bi, T2, and the four parts as contiguous planes
-        char* z = (char*)zbuf_buffer(ctx, 3 * al(nSA) + 3 * al(nSB) + al(nT));
-        double* SA = (double*)z;
-        double* SB = (double*)(z + al(nSA));
-        double* T2 = (double*)(z + al(nSA) + al(nSB));
-        double* Ar = (double*)(z + al(nSA) + al(nSB) + al(nT));
-        double* Ai = Ar + al(nSA) / sizeof(double);
-        double* Br = Ai + al(nSA) / sizeof(double);
-        double* Bi = Br + al(nSB) / sizeof(double);
-        auto grid = [](int64_t rows, int64_t cols) {
-            return dim3((uint32_t)std::min<int64_t>((cols + 255) / 256, 64), (uint32_t)std::min<int64_t>(rows, 65535));
-        };
-        hipLaunchKernelGGL(k_zsum_parts, grid(M, K), dim3(256), 0, ctx->stream, SA, Ar, Ai, (const c128*)P.a, M, K,
-                           P.rsa, P.csa);
-        hipLaunchKernelGGL(k_zsum_parts, grid(K, N), dim3(256), 0, ctx->stream, SB, Br, Bi, (const c128*)P.b, K, N,
-                           P.rsb, P.csb);
-        check_launch("complex split sums");
-        const double a = alpha.re;
-        GemmProblem Q = P;
-        Q.bd.nbd = 0;
-        Q.nbatch = 1;
-        // T1 into Re C
-        Q.a = Ar;
-        Q.rsa = K;
-        Q.csa = 1;
-        Q.b = Br;
-        Q.rsb = N;
-        Q.csb = 1;
-        Q.c = P.c;
-        Q.rsc = 2 * P.rsc;
-        Q.csc = 2 * P.csc;
-        ozaki_gemm_f64(ctx, Q, a, 0.0, true);
-        // T3 into Im C
-        Q.a = SA;
-        Q.rsa = K;
-        Q.csa = 1;
-        Q.b = SB;
-        Q.rsb = N;
-        Q.csb = 1;
-        Q.c = (double*)P.c + 1;
-        ozaki_gemm_f64(ctx, Q, a, 0.0, true);
-        // T2 into the temporary
-        Q.a = Ai;
-        Q.rsa = K;
-        Q.csa = 1;
-        Q.b = Bi;
-        Q.rsb = N;
-        Q.csb = 1;
-        Q.c = T2;
-        Q.rsc = N;
-        Q.csc = 1;
-        ozaki_gemm_f64(ctx, Q, a, 0.0, true);
-        hipLaunchKernelGGL(k_z3m_combine, dim3((uint32_t)std::min<size_t>((nT + 255) / 256, 65536)), dim3(256), 0,
-                           ctx->stream, (c128*)P.c, P.rsc, P.csc, T2, M, N);
-        check_launch("complex split combine");
+        const size_t bytes = Zgemm3Parts(P).bytes();
+        if (!ozaki_zgemm3(ctx, P, alpha.re, bytes,
+                          [&](const int* flag, char* ws) { zgemm3_products(ctx, P, alpha.re, ws, flag); }))
+            zgemm3_products(ctx, P, alpha.re, (char*)zbuf_buffer(ctx, bytes), nullptr);
         return;
     }
     auto part = [&](const void* base, int im) { return (const void*)((const double*)base + im); };

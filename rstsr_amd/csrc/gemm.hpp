@@ -107,6 +107,10 @@ void tile_grouped_c128(rstsr_hip_ctx* ctx, const std::vector<GemmProblem>& probs
 // Ozaki-II split GEMM for f64 (ozaki.hip). Falls back to the plain kernel for
 // non-finite inputs.
 void ozaki_gemm_f64(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, double beta, bool beta_zero);
+// C = alpha A B (complex, one matrix) by the split GEMM's three-product form in one run; false for a
+// form it does not take.
+bool ozaki_zgemm3(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, size_t plain_bytes,
+                  const std::function<void(const int* flag, char* ws)>& plain);
 // Plain FP64 MFMA DGEMM of one problem (gemm.hip). run_if (device, nullable):
 // the kernel exits unless *run_if != 0.
 void plain_dgemm(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, double beta, bool beta_zero,

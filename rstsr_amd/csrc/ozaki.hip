@@ -576,6 +576,152 @@ __global__ void __launch_bounds__(256) k_normsplit_rows_reg(const double* __rest
     }
 }
 
+/* ---------------- complex operands: three real parts ---------------- */
+
+// The complex split GEMM multiplies three pairs of real matrices: the real parts, the imaginary
+// parts and their sums. Part p of an element:
+__device__ __forceinline__ double zpart(double2 x, int p) { return p == 0 ? x.x : (p == 1 ? x.y : x.x + x.y); }
+
+// k_norm_cols for the three parts of a complex operand, read once: part p's exponents at ev + p evs,
+// its partials in "batch" p of `part`. Every part's terms add up in k_norm_cols's order.
+__global__ void __launch_bounds__(256) k_znorm_cols(const double2* __restrict__ x, int64_t nvec, int64_t len, int64_t sv,
+                                                    int64_t st, int64_t chunk, int64_t evs, int g,
+                                                    NormAcc* __restrict__ part, int* __restrict__ ev,
+                                                    int* __restrict__ flag) {
+    __shared__ NormAcc red[3][4][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t v = (int64_t)blockIdx.x * 64 + lane;
+    const uint32_t c = blockIdx.y;
+    NormAcc a[3][4];
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[p][q] = NormAcc{0.0, 0, 0.0};
+    bool bad = false;
+    if (v < nvec) {
+        const int64_t t1 = min(len, (int64_t)(c + 1) * chunk);
+        const double2* xp = x + v * sv;
+        int64_t t = (int64_t)c * chunk + w;
+        for (; t + 12 < t1; t += 16) {
+            double2 y[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) y[q] = xp[(t + 4 * q) * st];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int p = 0; p < 3; ++p) norm_add(a[p][q], zpart(y[q], p), bad);
+        }
+        for (; t < t1; t += 4) {
+            const double2 y = xp[t * st];
+#pragma unroll
+            for (int p = 0; p < 3; ++p) norm_add(a[p][0], zpart(y, p), bad);
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+#pragma unroll
+        for (int q = 1; q < 4; ++q) norm_merge(a[p][0], a[p][q]);
+        red[p][w][lane] = a[p][0];
+    }
+    __syncthreads();
+    if (bad) atomicOr(flag, 1);
+    if (w >= 3 || v >= nvec) return;
+    NormAcc s = red[w][0][lane];  // wave p ends part p
+#pragma unroll
+    for (int q = 1; q < 4; ++q) norm_merge(s, red[w][q][lane]);
+    if (gridDim.y == 1) ev[w * evs + v] = scale_exponent(s, g);
+    else part[((int64_t)w * gridDim.y + c) * nvec + v] = s;
+}
+
+// k_split for the three parts of a complex operand whose vectors lie side by side, read once (part p:
+// exponents ev + p nvp, planes + p nvp lenp). Bound by the residues' vector instructions; the one read instead of a pass that
+// writes the parts and three that read them back: see ozaki_zgemm3.
+template <bool K14>
+__global__ void __launch_bounds__(256) k_zsplit(const double2* __restrict__ s, int64_t nv, int64_t len, int64_t sv,
+                                                int64_t st, const int* __restrict__ ev, int64_t nvp, int64_t lenp,
+                                                int8_t* __restrict__ planes, ModSet ms,
+                                                const int* __restrict__ skip, int64_t plane, int tpb) {
+    if (*skip) return;  // non-finite input: the plain kernels compute this product
+    __shared__ double tile[64][65];
+    // neighbouring blocks take neighbouring vectors, as the lanes do
+    const int64_t v0 = (int64_t)blockIdx.x * 64, ta = (int64_t)blockIdx.y * tpb * 64;
+    const int64_t te = min(lenp, ta + (int64_t)tpb * 64);
+    const int tid = threadIdx.x, fast = tid & 63, slow0 = tid >> 6;
+    for (int64_t t0 = ta; t0 < te; t0 += 64) {
+        double2 x[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const int64_t t = t0 + 4 * k + slow0, v = v0 + fast;
+            x[k] = v < nv && t < len ? s[v * sv + t * st] : double2{0.0, 0.0};
+        }
+#pragma unroll 1
+        for (int p = 0; p < 3; ++p) {
+            double y[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) y[k] = zpart(x[k], p);
+            split_store<K14>(y, nv, ev + p * nvp, nvp, lenp, planes + p * nvp * lenp, ms, false, plane, v0, t0,
+                             tile);
+            __syncthreads();  // the tile is rewritten
+        }
+    }
+}
+
+// k_normsplit_rows_reg for the three parts of a complex operand, held in registers and read once.
+template <bool K14, int RPB, int CH>
+__global__ void __launch_bounds__(256) k_znormsplit_rows(const double2* __restrict__ x, int64_t nv, int64_t len,
+                                                         int64_t sv, int64_t nvp, int64_t lenp, int g,
+                                                         int* __restrict__ ev, int8_t* __restrict__ planes,
+                                                         int64_t plane, ModSet ms, int* __restrict__ flag) {
+    static_assert(RPB == 1 || RPB == 4, "a vector per block or per wave");
+    constexpr int TPR = 256 / RPB;
+    __shared__ NormAcc red[3][4];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, tr = tid % TPR;
+    const int64_t v = (int64_t)blockIdx.x * RPB + tid / TPR;  // uniform across each wave
+    if (v >= nvp) return;
+    double2 xs[CH][16];
+#pragma unroll
+    for (int i = 0; i < CH; ++i) {
+        const int64_t t0 = ((int64_t)tr + TPR * i) * 16;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) xs[i][e] = v < nv && t0 + e < len ? x[v * sv + t0 + e] : double2{0.0, 0.0};
+    }
+    bool bad = false;
+#pragma unroll 1
+    for (int p = 0; p < 3; ++p) {
+        NormAcc a{0.0, 0, 0.0};
+#pragma unroll
+        for (int i = 0; i < CH; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) norm_add(a, zpart(xs[i][e], p), bad);
+        a = wave_norm(a);
+        if constexpr (RPB == 1) {
+            if (lane == 0) red[p][w] = a;
+            __syncthreads();
+            a = red[p][0];
+#pragma unroll
+            for (int q = 1; q < 4; ++q) norm_merge(a, red[p][q]);
+        }
+        const int e = scale_exponent(a, g);
+        if (tr == 0 && v < nv) ev[p * nvp + v] = e;
+        int8_t* pv = planes + (p * nvp + v) * lenp;
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            const int64_t t0 = ((int64_t)tr + TPR * i) * 16;
+            if (t0 >= lenp) continue;
+            Digits dg[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) dg[k] = to_digits(rint(ldexp(zpart(xs[i][k], p), e)));
+            for_moduli<K14>(ms, [&](int l) {
+                const ResConst c = res_const<K14>(ms, l);
+                const uint4 wd{pack_residues(dg, c), pack_residues(dg + 4, c), pack_residues(dg + 8, c),
+                               pack_residues(dg + 12, c)};
+                *(uint4*)(pv + l * plane + t0) = wd;
+            });
+        }
+    }
+    if (bad) atomicOr(flag, 1);
+}
+
 /* ---------------- INT8 MFMA GEMM per modulus ---------------- */
 
 // INT8 tile configurations: a BM x BN block tile from WVM x WVN waves, K slices
@@ -1222,6 +1368,55 @@ __global__ void __launch_bounds__(256) k_crt(const uint8_t* __restrict__ R, int6
     }
 }
 
+// The CRT of a complex product's three real products T1, T2, T3 (batches 0 to 2 of R; planes of pl
+// bytes) in one pass: C = (a T1 - a T2, a T3 - a T1 - a T2). Four columns per thread as in k_crt.
+template <bool K14>
+__global__ void __launch_bounds__(256) k_crt3(const uint8_t* __restrict__ R, int64_t M, int64_t N, int64_t Mp, int64_t Np,
+                                              int64_t pl, CrtConst cc, const int* __restrict__ eA,
+                                              const int* __restrict__ fB, c128* C, int64_t rsc, int64_t csc,
+                                              double alpha, const int* __restrict__ skip, int tpr) {
+    if (*skip) return;
+    const int rpb = 256 / tpr;
+    const int64_t j0 = ((int64_t)blockIdx.x * tpr + (threadIdx.x & (tpr - 1))) * 4;
+    if (j0 >= N) return;
+    const int nm = K14 ? OZ_MAXMOD : cc.n;
+    const int64_t step = (int64_t)gridDim.y * rpb, mn = Mp * Np;
+    int64_t i = (int64_t)blockIdx.y * rpb + threadIdx.x / tpr;
+    auto load = [&](int64_t row, int p, uint32_t (&w)[OZ_MAXMOD]) {
+        const uint8_t* rp = R + p * mn + row * Np + j0;
+#pragma unroll
+        for (int l = 0; l < OZ_MAXMOD; ++l) w[l] = l < nm ? *(const uint32_t*)(rp + l * pl) : 0u;
+    };
+    int fj[3][4];
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) fj[p][k] = fB[p * Np + j0 + k];  // Np >= j0 + 4 entries per part
+    uint32_t w[3][OZ_MAXMOD];
+    if (i < M)
+#pragma unroll
+        for (int p = 0; p < 3; ++p) load(i, p, w[p]);
+    for (; i < M; i += step) {
+        double t[3][4];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            const int ei = eA[p * Mp + i];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                uint32_t r[OZ_MAXMOD];
+#pragma unroll
+                for (int l = 0; l < OZ_MAXMOD; ++l) r[l] = (w[p][l] >> (8 * k)) & 255u;
+                t[p][k] = alpha * ldexp(crt_from<K14>(r, cc), -(ei + fj[p][k]));
+            }
+            if (i + step < M) load(i + step, p, w[p]);  // the next row's words, while the rest runs
+        }
+        c128* cp = C + i * rsc + j0 * csc;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (j0 + k < N) cp[k * csc] = c128{t[0][k] - t[1][k], (t[2][k] - t[0][k]) - t[1][k]};
+    }
+}
+
 /* ---------------- grouped (uneven) split GEMM ---------------- */
 
 // One problem of a grouped split GEMM, with its offsets into the group's shared
@@ -1595,6 +1790,63 @@ static void with_i8_tile(I8Tile t, F&& f) {
     }
 }
 
+// The residue products of nb batches (a_b / b_b: the operand's planes are batched): planes A8
+// [l][batch][Mp][Kp], B8 [l][batch][Np][Kp] -> residues R [l][batch][Mp][Np].
+static void launch_i8gemm(rstsr_hip_ctx* ctx, const OzSetup& su, I8Tile tile, const int8_t* A8, const int8_t* B8,
+                          uint8_t* R, int64_t Mp, int64_t N, int64_t Kp, int64_t Np, uint64_t nb, bool a_b, bool b_b,
+                          const int* flag, bool sym) {
+    const int n = su.n;
+    const CrtConst& cc = su.cc;
+    const ModSet& ms = su.ms;
+    int64_t bm = 0, bn = 0;
+    with_i8_tile(tile, [&](auto c) {
+        bm = decltype(c)::BM;
+        bn = decltype(c)::BN;
+    });
+    const uint32_t tiles_n = (uint32_t)(Np / bn);
+    const uint32_t ntiles = sym ? (uint32_t)lower_tile_prefix((uint64_t)(Mp / bm), (uint64_t)(bn / bm))
+                                : (uint32_t)((Mp / bm) * tiles_n);
+    const size_t planeA = (a_b ? nb : 1) * (size_t)Mp * Kp, planeB = (b_b ? nb : 1) * (size_t)Np * Kp,
+                 planeR = nb * (size_t)Mp * Np;
+    ModList mods{};
+    for (int l = 0; l < n; ++l) {
+        mods.m[l] = (int)cc.mod[l];
+        mods.c16[l] = ms.c16[l];
+        mods.inv[l] = ms.inv[l];
+    }
+    // K beyond I8_KCHUNK: further launches add their residues into R
+    for (int64_t k0 = 0; k0 < Kp; k0 += I8_KCHUNK) {
+        const int64_t Kc = std::min<int64_t>(I8_KCHUNK, Kp - k0);
+        auto go = [&](auto cfg) {
+            using CF = decltype(cfg);
+            // the 256 x 256 tile stores its residues four columns at a time
+            constexpr bool TOUT = CF::BM == 256;
+            // direct-load tiles over one K chunk run gmod moduli per block (a divisor of the
+            // modulus count): as many as keep a block within 96 K slices and the launch at four
+            // blocks per CU or more. Measured: the 65536 x 1024 x 1024 batch (8 slices per
+            // modulus) 1.28 ms at 7 or 14 moduli per block against 1.38-1.44 ms at one; 8192^3
+            // (64 slices) the same at one or two.
+            int gmod = 1;
+            const bool mm = CF::ST > 0 && TOUT && Kp <= I8_KCHUNK;
+            if (mm) {
+                const uint64_t blocks = (uint64_t)ntiles * nb;
+                const int64_t ns = Kp / CF::BK;
+                for (int g = 1; g <= n; ++g)
+                    if (n % g == 0 && g * ns <= 96 && blocks * (uint64_t)(n / g) >= 1024) gmod = g;
+            }
+            auto kern = mm ? k_i8gemm_mod<CF, I8_ROW4G, TOUT, CF::ST != 0 && TOUT>
+                           : k_i8gemm_mod<CF, I8_ROW4G, TOUT, false>;
+            hipLaunchKernelGGL(kern, dim3(ntiles, (uint32_t)nb, (uint32_t)((n + gmod - 1) / gmod)), dim3(CF::NT), 0,
+                               ctx->stream, A8 + k0, B8 + k0, R, Mp, N, Kp, Kc, Np, mods, k0 > 0 ? 1 : 0,
+                               (uint32_t)(Mp / bm), tiles_n, a_b ? Mp * Kp : (int64_t)0,
+                               b_b ? Np * Kp : (int64_t)0, Mp * Np, (int64_t)planeA, (int64_t)planeB,
+                               (int64_t)planeR, flag, sym ? 1 : 0, gmod, n);
+        };
+        with_i8_tile(tile, go);
+        check_launch("ozaki int8 gemm");
+    }
+}
+
 void ozaki_gemm_f64(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, double beta, bool beta_zero) {
     const OzSetup su = ozaki_setup();
     const int n = su.n;
@@ -1688,10 +1940,6 @@ void ozaki_gemm_f64(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, doub
     int8_t* A8 = (int8_t*)(ws + o_A8);
     int8_t* B8 = (int8_t*)(ws + o_B8);
     uint8_t* R = (uint8_t*)(ws + o_R);
-    const uint32_t tiles_n = (uint32_t)(Np / bn);
-    const uint32_t ntiles = sym ? (uint32_t)lower_tile_prefix((uint64_t)(Mp / bm), (uint64_t)(bn / bm))
-                                : (uint32_t)((Mp / bm) * tiles_n);
-
     hipLaunchKernelGGL(k_zero_i32, dim3(ceil_div_u32(n_zero, 256)), dim3(256), 0, ctx->stream, flag, (int64_t)n_zero);
     check_launch("ozaki zero");
     auto run_norm = [&](const NormPlan& q, int* ev) {
@@ -1763,43 +2011,7 @@ void ozaki_gemm_f64(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, doub
     // FP64 kernel (which runs only when *flag != 0) computes C with IEEE special
     // values. No host round trip, so the sequence can be graph-captured.
     plain_dgemm(ctx, P, alpha, beta, beta_zero, flag);
-    ModList mods{};
-    for (int l = 0; l < n; ++l) {
-        mods.m[l] = (int)cc.mod[l];
-        mods.c16[l] = ms.c16[l];
-        mods.inv[l] = ms.inv[l];
-    }
-    // K beyond I8_KCHUNK: further launches add their residues into R
-    for (int64_t k0 = 0; k0 < Kp; k0 += I8_KCHUNK) {
-        const int64_t Kc = std::min<int64_t>(I8_KCHUNK, Kp - k0);
-        auto go = [&](auto cfg) {
-            using CF = decltype(cfg);
-            // the 256 x 256 tile stores its residues four columns at a time
-            constexpr bool TOUT = CF::BM == 256;
-            // direct-load tiles over one K chunk run gmod moduli per block (a divisor of the
-            // modulus count): as many as keep a block within 96 K slices and the launch at four
-            // blocks per CU or more. Measured: the 65536 x 1024 x 1024 batch (8 slices per
-            // modulus) 1.28 ms at 7 or 14 moduli per block against 1.38-1.44 ms at one; 8192^3
-            // (64 slices) the same at one or two.
-            int gmod = 1;
-            const bool mm = CF::ST > 0 && TOUT && Kp <= I8_KCHUNK;
-            if (mm) {
-                const uint64_t blocks = (uint64_t)ntiles * nb;
-                const int64_t ns = Kp / CF::BK;
-                for (int g = 1; g <= n; ++g)
-                    if (n % g == 0 && g * ns <= 96 && blocks * (uint64_t)(n / g) >= 1024) gmod = g;
-            }
-            auto kern = mm ? k_i8gemm_mod<CF, I8_ROW4G, TOUT, CF::ST != 0 && TOUT>
-                           : k_i8gemm_mod<CF, I8_ROW4G, TOUT, false>;
-            hipLaunchKernelGGL(kern, dim3(ntiles, (uint32_t)nb, (uint32_t)((n + gmod - 1) / gmod)), dim3(CF::NT), 0,
-                               ctx->stream, A8 + k0, B8 + k0, R, Mp, N, Kp, Kc, Np, mods, k0 > 0 ? 1 : 0,
-                               (uint32_t)(Mp / bm), tiles_n, a_b ? Mp * Kp : (int64_t)0,
-                               b_b ? Np * Kp : (int64_t)0, Mp * Np, (int64_t)planeA, (int64_t)planeB,
-                               (int64_t)planeR, flag, sym ? 1 : 0, gmod, n);
-        };
-        with_i8_tile(tile, go);
-        check_launch("ozaki int8 gemm");
-    }
+    launch_i8gemm(ctx, su, tile, A8, B8, R, Mp, N, Kp, Np, nb, a_b, b_b, flag, sym);
     // four columns per thread when every row and plane of R starts on a 4-byte boundary
     auto crt = [&](auto v) {
         constexpr int V = decltype(v)::value;
@@ -1837,6 +2049,129 @@ void ozaki_gemm_f64(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, doub
                            alpha, beta, beta_zero ? 1 : 0, flag, (uint32_t)tmt, (uint32_t)tnt);
         check_launch("ozaki crt");
     }
+}
+
+// C = a A B for complex A, B from three real products (Karatsuba form): T1 = Ar Br, T2 = Ai Bi,
+// T3 = (Ar + Ai)(Br + Bi); Re C = a (T1 - T2), Im C = a (T3 - T1 - T2). Each product is accurate to
+// the split GEMM's normwise bound, so the result keeps it relative to (|Ar| + |Ai|)(|Br| + |Bi|).
+// The products are the three batches of one run of the split GEMM: the operands are read once, as
+// they are, into the residue planes of their three parts, and one CRT pass ends all three. (As three
+// runs, the parts were written out and read back, each product's residues went to C or a plane on
+// their own and a last pass combined them: 4096^3 4.31 ms, now 3.71.)
+// Returns false, before anything is enqueued, for forms it does not take: operands whose vectors
+// neither have unit stride and at most 8192 elements nor lie side by side, and planes past
+// Z3_MAX_BYTES, since they are three times those of one real product.
+// plain(flag, ws): enqueue what computes C when *flag is set, in the planes' place (plain_bytes at ws).
+constexpr size_t Z3_MAX_BYTES = (size_t)32 << 30;
+
+bool ozaki_zgemm3(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, size_t plain_bytes,
+                  const std::function<void(const int* flag, char* ws)>& plain) {
+    const OzSetup su = ozaki_setup();
+    const int n = su.n, g = su.g;
+    const ModSet& ms = su.ms;
+    const int64_t M = P.M, N = P.N, K = P.K;
+    if (K > (int64_t)1 << 21 || M > (int64_t)1 << 22 || N > (int64_t)1 << 22) return false;
+    const I8Tile tile = pick_i8_tile(M, N);
+    int64_t bm = 0, bn = 0;
+    with_i8_tile(tile, [&](auto c) {
+        bm = decltype(c)::BM;
+        bn = decltype(c)::BN;
+    });
+    const int64_t Np = (N + bn - 1) / bn * bn, Mp = (M + bm - 1) / bm * bm;
+    const int64_t Kp = (K + I8_KPAD - 1) / I8_KPAD * I8_KPAD;
+    struct Operand {
+        const double2* x;
+        int64_t nv, nvp, sv, st, nchunk, chunk;
+        bool held;  // vectors of unit stride, held in registers
+    };
+    auto operand = [&](const void* x, int64_t nv, int64_t nvp, int64_t sv, int64_t st) {
+        Operand q{(const double2*)x, nv, nvp, sv, st, 1, K, st == 1 && Kp <= 8192};
+        const int64_t blocks = (nv + 63) / 64;
+        q.nchunk = std::max<int64_t>(1, std::min<int64_t>({(2048 + blocks - 1) / blocks, K / 64, 4096}));
+        q.chunk = (K + q.nchunk - 1) / q.nchunk;
+        q.nchunk = (K + q.chunk - 1) / q.chunk;
+        return q;
+    };
+    const Operand qa = operand(P.a, M, Mp, P.rsa, P.csa), qb = operand(P.b, N, Np, P.csb, P.rsb);
+    for (const Operand* q : {&qa, &qb})
+        if (!q->held && std::llabs(q->st) <= std::llabs(q->sv)) return false;
+    auto part_bytes = [](const Operand& q) {
+        return !q.held && q.nchunk > 1 ? 3 * (size_t)q.nchunk * q.nv * sizeof(NormAcc) : (size_t)0;
+    };
+    // workspace layout as in ozaki_gemm_f64, with three batches
+    size_t off = sizeof(int);
+    const size_t o_eA = off;
+    off += 3 * Mp * sizeof(int);
+    const size_t o_fB = off;
+    off += 3 * Np * sizeof(int);
+    const size_t n_zero = off / sizeof(int);
+    auto take = [&](size_t bytes) {
+        off = (off + 255) & ~(size_t)255;
+        const size_t o = off;
+        off += bytes;
+        return o;
+    };
+    const size_t o_part = take(std::max(part_bytes(qa), part_bytes(qb)));
+    const size_t planeA = 3 * (size_t)Mp * Kp, planeB = 3 * (size_t)Np * Kp, planeR = 3 * (size_t)Mp * Np;
+    const size_t o_A8 = take(n * planeA), o_B8 = take(n * planeB), o_R = take(n * planeR);
+    off = std::max(off, o_A8 + plain_bytes);
+    if (off > Z3_MAX_BYTES) return false;
+    char* ws = (char*)workspace(ctx, off);
+    int* flag = (int*)ws;
+    int* eA = (int*)(ws + o_eA);
+    int* fB = (int*)(ws + o_fB);
+    NormAcc* part = (NormAcc*)(ws + o_part);
+    int8_t* A8 = (int8_t*)(ws + o_A8);
+    int8_t* B8 = (int8_t*)(ws + o_B8);
+    uint8_t* R = (uint8_t*)(ws + o_R);
+    hipLaunchKernelGGL(k_zero_i32, dim3(ceil_div_u32(n_zero, 256)), dim3(256), 0, ctx->stream, flag, (int64_t)n_zero);
+    check_launch("ozaki zero");
+    auto split = [&](const Operand& q, int* ev, int8_t* planes, size_t plane, const char* what) {
+        if (q.held) {
+            auto go = [&](auto rpb, auto ch) {
+                constexpr int RPB = decltype(rpb)::value, CH = decltype(ch)::value;
+                auto kern = n == OZ_MAXMOD ? k_znormsplit_rows<true, RPB, CH> : k_znormsplit_rows<false, RPB, CH>;
+                hipLaunchKernelGGL(kern, dim3(ceil_div_u32(q.nvp, RPB)), dim3(256), 0, ctx->stream, q.x, q.nv, K, q.sv,
+                                   q.nvp, Kp, g, ev, planes, (int64_t)plane, ms, flag);
+            };
+            using I1 = std::integral_constant<int, 1>;
+            using I2 = std::integral_constant<int, 2>;
+            using I4 = std::integral_constant<int, 4>;
+            if (Kp <= 1024) go(I4{}, I1{});
+            else if (Kp <= 2048) go(I4{}, I2{});
+            else if (Kp <= 4096) go(I1{}, I1{});
+            else go(I1{}, I2{});
+            check_launch(what);
+            return;
+        }
+        hipLaunchKernelGGL(k_znorm_cols, dim3(ceil_div_u32(q.nv, 64), (uint32_t)q.nchunk), dim3(256), 0, ctx->stream, q.x,
+                           q.nv, K, q.sv, q.st, q.chunk, q.nvp, g, part, ev, flag);
+        if (q.nchunk > 1)
+            hipLaunchKernelGGL(k_norm_fin, dim3(ceil_div_u32(q.nv, 256), 3), dim3(256), 0, ctx->stream, part, q.nv,
+                               (int)q.nchunk, q.nvp, g, ev);
+        check_launch("ozaki norms");
+        // tiles along K per block and the order of the blocks as in ozaki_gemm_f64
+        const uint64_t tiles = (uint64_t)(Kp / 64) * (uint64_t)(q.nvp / 64);
+        int tpb = 1;
+        while (tpb < 8 && tiles / (uint64_t)(2 * tpb) >= (uint64_t)std::max(ctx->num_cu, 1) * 8) tpb *= 2;
+        const uint32_t gx = (uint32_t)((Kp / 64 + tpb - 1) / tpb), gy = (uint32_t)(q.nvp / 64);
+        hipLaunchKernelGGL(n == OZ_MAXMOD ? k_zsplit<true> : k_zsplit<false>, dim3(gy, gx), dim3(256), 0, ctx->stream, q.x,
+                           q.nv, K, q.sv, q.st, ev, q.nvp, Kp, planes, ms, flag, (int64_t)plane, tpb);
+        check_launch(what);
+    };
+    split(qa, eA, A8, planeA, "ozaki split A");
+    split(qb, fB, B8, planeB, "ozaki split B");  // reuses the partials after A's (stream order)
+    plain(flag, ws + o_A8);  // non-finite input: the kernels after it then do nothing
+    launch_i8gemm(ctx, su, tile, A8, B8, R, Mp, N, Kp, Np, 3, true, true, flag, false);
+    const int64_t ncg = (N + 3) / 4;
+    int tpr = 1;
+    while (tpr < 256 && tpr < ncg) tpr *= 2;
+    const int64_t rpb = 256 / tpr, gy = std::min<int64_t>(std::max<int64_t>(1, (M + 4 * rpb - 1) / (4 * rpb)), 65535);
+    hipLaunchKernelGGL(n == OZ_MAXMOD ? k_crt3<true> : k_crt3<false>, dim3(ceil_div_u32(ncg, tpr), (uint32_t)gy), dim3(256),
+                       0, ctx->stream, R, M, N, Mp, Np, (int64_t)planeR, su.cc, eA, fB, (c128*)P.c, P.rsc, P.csc, alpha,
+                       flag, tpr);
+    check_launch("ozaki crt");
+    return true;
 }
 
 // Grouped split GEMM routing (RSTSR_HIP_OZAKI_GROUPED: "auto", the default, or "split").
