@@ -729,16 +729,14 @@ __global__ void __launch_bounds__(256) k_znormsplit_rows(const double2* __restri
 // conflicts of the 16-byte fragment reads).
 // FR: the MFMA's output block, 16 (v_mfma_i32_16x16x64_i8) or 32 (v_mfma_i32_32x32x32_i8).
 // D: K slices whose global loads are in flight at once (register sets).
-// ST: 0 for loads staged through registers; otherwise the slices go straight from global memory
-// into a ring of ST LDS buffers (global_load_lds_dwordx4, unpadded swizzled rows), ST - 1 ahead.
-// SG: the K steps of a slice scheduled as fragment reads interleaved with the MFMAs before them.
-template <int BM_, int BN_, int BK_, int WVM_, int WVN_, int OCC_, int PAD_, int FR_ = 16, int D_ = 1, int ST_ = 0,
-          int SG_ = 0>
+// DL: the slices go straight from global memory into the LDS buffers (unpadded swizzled rows) instead of
+// through registers, and fragments are read a K step ahead, also across slices.
+template <int BM_, int BN_, int BK_, int WVM_, int WVN_, int OCC_, int PAD_, int FR_ = 16, int D_ = 1, bool DL_ = false>
 struct I8Cfg {
-    static constexpr int BM = BM_, BN = BN_, BK = BK_, WVM = WVM_, WVN = WVN_, OCC = OCC_, PAD = PAD_, FR = FR_,
-                         D = D_, ST = ST_, SG = SG_;
+    static constexpr int BM = BM_, BN = BN_, BK = BK_, WVM = WVM_, WVN = WVN_, OCC = OCC_, PAD = PAD_, FR = FR_, D = D_;
+    static constexpr bool DL = DL_;
     static constexpr int NT = 64 * WVM * WVN;
-    static constexpr int NBUF = ST > 2 ? ST : 2;
+    static constexpr int NBUF = 2;
 };
 // products more than 128 wide: eight waves of 64 x 64, two blocks per CU
 using I8Wide8 = I8Cfg<128, 256, 64, 2, 4, 2, 32>;
@@ -746,8 +744,11 @@ using I8Wide8 = I8Cfg<128, 256, 64, 2, 4, 2, 32>;
 using I8Sq = I8Cfg<128, 128, 128, 2, 2, 2, 16>;
 // large products: 256 x 256 block tiles from eight waves of 64 x 128 (a third fewer LDS
 // fragment bytes per MFMA than 64 x 64 waves), 128-byte K slices in XOR-swizzled rows loaded
-// straight into two LDS buffers, fragment reads interleaved with the MFMAs, one block per CU
-using I8Big = I8Cfg<256, 256, 128, 4, 2, 1, 0, 16, 1, 2, 1>;
+// straight into two LDS buffers, one block per CU. What bounds it: power. Its MFMAs keep the matrix
+// cores busy 68 % of the cycles, at which the clock stands at 1.8 of 2.4 GHz (8192^3, 14 moduli).
+// Before the fragment reads ran across slices and the loads were spread over the products it was
+// 62 % at 1.89 GHz: 10.8 against 11.8 million cycles, 5.97 against 6.26 ms.
+using I8Big = I8Cfg<256, 256, 128, 4, 2, 1, 0, 16, 1, true>;
 // planes: rows padded to a multiple of the tile's BM (I8_MPAD for all but the 256-row tiles),
 // K to I8_KPAD (every BK divides it)
 constexpr int I8_MPAD = 128, I8_KPAD = 128;
@@ -806,10 +807,9 @@ struct I8Smem {
 // < M and columns < N, added to the residues already there when `accum`. Each
 // wave owns (BM / WVM) x (BN / WVN) outputs from FR x FR MFMA blocks
 // (v_mfma_i32_16x16x64_i8 or v_mfma_i32_32x32x32_i8). K runs in slices of BK
-// bytes through LDS buffers: with CF::ST == 0 global loads run CF::D slices ahead
+// bytes through LDS buffers: without CF::DL global loads run CF::D slices ahead
 // in registers (D register sets) and two LDS buffers take them in turn, so a load
-// has D slices of MFMA work to arrive; with CF::ST > 0 the slices go straight
-// into a ring of ST buffers, ST - 1 slices ahead.
+// has D slices of MFMA work to arrive; with CF::DL the slices go straight into the buffers.
 // TOUT: each product block is formed transposed (B fragment as the MFMA's row
 // operand), so a lane ends with runs of four consecutive columns of one row of
 // R: one 4-byte store per run (N % 4 == 0), the residue by mod_res. The 32 x 32
@@ -873,7 +873,6 @@ __device__ __forceinline__ void i8_tile(const int8_t* __restrict__ A, const int8
     static_assert(RPP % 8 == 0 && FR % 8 == 0 && WTM % 8 == 0 && WTN % 8 == 0, "swizzle period");
     const int sr = swz(fr);  // fragment rows start at multiples of 8
     auto compute = [&](int buf) {
-        if constexpr (CF::SG) __builtin_amdgcn_sched_barrier(0);  // the slice's reads and MFMAs alone
 #pragma unroll
         for (int kk = 0; kk < BK; kk += FK) {
             v4i af[FM], bf[FN];
@@ -895,25 +894,6 @@ __device__ __forceinline__ void i8_tile(const int8_t* __restrict__ A, const int8
                     else
                         acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[i], bf[j], acc[i][j], 0, 0, 0);
                 }
-        }
-        if constexpr (CF::SG) {
-            // instruction order for the scheduler: the first K step's fragment reads, then each
-            // later step's reads spread over the MFMAs of the step before it (Q MFMAs per read),
-            // so fragments arrive while the matrix cores run
-            constexpr int NR = FM + FN, NMF = FM * FN, NS = BK / FK, Q = NMF / NR >= 2 ? 2 : 1;
-            static_assert(Q * NR <= NMF && NS >= 2, "reads fit between the MFMAs");
-            __builtin_amdgcn_sched_group_barrier(0x100, NR, 0);
-#pragma unroll
-            for (int s = 0; s + 1 < NS; ++s) {
-#pragma unroll
-                for (int r = 0; r < NR; ++r) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, Q, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                }
-                __builtin_amdgcn_sched_group_barrier(0x008, NMF - Q * NR, 0);
-            }
-            __builtin_amdgcn_sched_group_barrier(0x008, NMF, 0);
-            __builtin_amdgcn_sched_barrier(0);
         }
     };
 
@@ -981,41 +961,49 @@ __device__ __forceinline__ void i8_tile(const int8_t* __restrict__ A, const int8
                 for (int r = 0; r < NREG; ++r) acc[i][j][r] = 0;
     };
 
-    if constexpr (CF::ST > 0) {
-        // direct loads: one global_load_lds_dwordx4 fills 1 KiB of LDS (lane i at byte 16 i), RW
+    if constexpr (CF::DL) {
+        // direct loads: one 16-byte load to LDS fills 1 KiB of it (lane i at byte 16 i), RW
         // whole rows of one wave; lane i takes chunk (i % CPR) ^ swz(row) of its row from global
         // memory, so the LDS rows come out swizzled as the fragment reads expect (RW is a multiple
-        // of the swizzle period: swz(row) = swz(i / CPR)). Slice t goes to buffer t % ST, issued
-        // ST - 1 slices ahead into the buffer every wave finished reading at the last barrier.
-        constexpr int S = CF::ST, RW = 1024 / BK, RP = (NT / 64) * RW, NI = BM / RP + BN / RP;
-        static_assert(CF::PAD == 0 && RW % 8 == 0 && BM % RP == 0 && BN % RP == 0 && (S - 2) * NI < 64 && S >= 2,
-                      "direct-load tile shape");
+        // of the swizzle period: swz(row) = swz(i / CPR)). Slice t goes to buffer t % 2, which every
+        // wave has read by the barrier in slice t - 2.
+        constexpr int RW = 1024 / BK, RP = (NT / 64) * RW, NI = BM / RP + BN / RP;
+        static_assert(CF::PAD == 0 && RW % 8 == 0 && BM % RP == 0 && BN % RP == 0 && BK == 2 * FK && FR == 16 && T &&
+                          FM <= FN,
+                      "direct-load tile shape: two steps per slice");
         const int wv = __builtin_amdgcn_readfirstlane(wave);
         const int dr = lane / CPR, dch = ((lane % CPR) ^ swz(lane / CPR)) * 16;
         // the buffers are written only by the direct loads, which the compiler does not count as
         // stores: their address escapes here, so no read of them can be folded away as undefined
         asm volatile("" ::"v"(&sm) : "memory");
-        // the lane's part of each load address (row dr of the wave's rows, its chunk): one 32-bit
-        // offset (dr < 8, ldk < 2^28: the host keeps longer K off this tile) on top of a
-        // wave-uniform base
-        const uint32_t loff = (uint32_t)(dr * ldk + dch);
+        // Buffer loads, whose uniform part (slice base, row group) stays in scalar registers: the
+        // lane's row dr of the wave's rows and its chunk are one 32-bit offset, and row groups another
+        // (ldk < 2^24: the host keeps longer K off this tile). The global form counts as an LDS
+        // access of unknown order too, which makes the compiler wait for every fragment read in
+        // flight where it needs one of them.
+        const uint32_t loff = (uint32_t)(dr * ldk + dch), w0 = (uint32_t)(wv * RW * ldk), rstep = (uint32_t)(RP * ldk);
         // The block's nmod moduli (planes pA, pB, pR apart) run as one sequence of nmod * ns
         // slices: the next modulus's first slices load during the last products and the
         // residue epilogue of the one before.
+        const int64_t nv = Kc / BK * nmod;
+        constexpr int NIA = BM / RP;
         int64_t da = 0, db = 0, dk = 0;  // the next slice to load: plane offsets, K offset
-        auto dma_next = [&](int st) {
-#pragma unroll
-            for (int i = 0; i < BM / RP; ++i) {
-                const int r0 = i * RP + wv * RW;
-                const int8_t* base = Ab + da + (size_t)r0 * ldk + dk;
-                __builtin_amdgcn_global_load_lds(base + loff, &As[st][r0][0], 16, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < BN / RP; ++i) {
-                const int r0 = i * RP + wv * RW;
-                const int8_t* base = Bb + db + (size_t)r0 * ldk + dk;
-                __builtin_amdgcn_global_load_lds(base + loff, &Bs[st][r0][0], 16, 0, 0);
-            }
+        int left = (int)nv;              // slices not loaded yet
+        auto rsrc = [&](const int8_t* p) {
+            return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, __builtin_amdgcn_readfirstlane(left > 0 ? -1 : 0),
+                                                     0x00020000);
+        };
+        // load i of the next slice into buffer st; past the last slice nothing is read (no bytes in range)
+        auto dma_part = [&](int st, int i) {
+            if (i < NIA)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc(Ab + da + dk), &As[st][i * RP + wv * RW][0], 16, loff,
+                                                         w0 + i * rstep, 0, 0);
+            else
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc(Bb + db + dk), &Bs[st][(i - NIA) * RP + wv * RW][0],
+                                                         16, loff, w0 + (i - NIA) * rstep, 0, 0);
+        };
+        auto dma_step = [&]() {
+            --left;
             dk += BK;
             if (dk == Kc) {
                 dk = 0;
@@ -1023,32 +1011,87 @@ __device__ __forceinline__ void i8_tile(const int8_t* __restrict__ A, const int8
                 db += pB;
             }
         };
-        const int64_t nv = Kc / BK * nmod;
+        auto dma_next = [&](int st) {
 #pragma unroll
-        for (int s = 0; s < S - 1; ++s)
-            if (s < nv) dma_next(s);
-        // slice 0 landed (the slices after it may still be in flight)
-        if (nv >= S - 1) vm_wait_barrier<(S - 2) * NI>();
-        else vm_wait_barrier<0>();
-        int st = 0, sn = S - 1;
+            for (int i = 0; i < NI; ++i) dma_part(st, i);
+            dma_step();
+        };
+        // Fragments are read a K step ahead, each of B's into the registers its last product just left
+        // (A's have a second set), also from one slice to the next: otherwise every wave starts a
+        // slice by waiting for twelve reads that all eight have asked for at once.
+        v4i af[2][FM], bf[FN];
+        auto ra1 = [&](int st, int step, int i) {
+            af[step][i] = *(const v4i*)&As[st][wm * WTM + i * FR + fr][(((step * FK + fk) >> 4) ^ sr) << 4];
+        };
+        auto rb1 = [&](int st, int step, int j) {
+            bf[j] = *(const v4i*)&Bs[st][wn * WTN + j * FR + fr][(((step * FK + fk) >> 4) ^ sr) << 4];
+        };
+        auto mul = [&](int step, int j) {
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+                acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(bf[j], af[step][i], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        constexpr int H = 2;        // column groups of a slice's second step that cover the barrier's wait
+        constexpr int PG = FN - H;  // those that the next loads are spread over
+        dma_next(0);
+        if (nv > 1) {
+            dma_next(1);
+            vm_wait_barrier<NI>();  // slice 0 landed
+        } else {
+            vm_wait_barrier<0>();
+        }
+#pragma unroll
+        for (int i = 0; i < FM; ++i) ra1(0, 0, i);
+#pragma unroll
+        for (int j = 0; j < FN; ++j) rb1(0, 0, j);
+        int st = 0;
         int64_t v = 0;
         auto slices = [&](int64_t cnt) {
-            for (int64_t t = 0; t < cnt; ++t, ++v) {
-                const bool more = v + S - 1 < nv;
-                if (more) dma_next(sn);
-                compute(st);
+            // lgkmcnt(0): with scalar loads possibly in flight at the loop's entry the compiler could
+            // not count fragment reads at its head
+            __builtin_amdgcn_s_waitcnt(0xC07F);
+            for (int64_t t = 0; t < cnt; ++t, ++v, st ^= 1) {
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < FN; ++j) {
+                    mul(0, j);
+                    rb1(st, 1, j);
+                    if (j < FM) ra1(st, 1, j);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int j = 0; j < H; ++j) mul(1, j);
                 // slice v + 1 landed, and no wave reads buffer st any more
-                if (more) vm_wait_barrier<(S - 2) * NI>();
-                else vm_wait_barrier<0>();
-                st = st + 1 == S ? 0 : st + 1;
-                sn = sn + 1 == S ? 0 : sn + 1;
+                vm_wait_barrier<0>();
+                // (after the last slice these read what the buffer still holds, unused)
+#pragma unroll
+                for (int j = 0; j < H; ++j) {
+                    rb1(st ^ 1, 0, j);
+                    ra1(st ^ 1, 0, j);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                // slice v + 2 a load or two per group: the eight waves' loads issued at once fill the
+                // memory pipe, and a wave waits in order behind its own (8192^3: 7.00 against 6.88 ms)
+#pragma unroll
+                for (int j = H; j < FN; ++j) {
+                    mul(1, j);
+                    rb1(st ^ 1, 0, j);
+                    if (j < FM) ra1(st ^ 1, 0, j);
+#pragma unroll
+                    for (int i = NI * (j - H) / PG; i < NI * (j - H + 1) / PG; ++i) dma_part(st, i);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                dma_step();
             }
+            // vmcnt(0): the empty loads past the last slice still write LDS, which must be this block's
+            if (v == nv) __builtin_amdgcn_s_waitcnt(0x0F70);
         };
         if constexpr (MM) {
             // rows of R at least tiles x BM, ldr at least tiles x BN (a multiple of 4), nothing to
             // add to: unguarded word stores (guards or a byte-wise path inside this loop would
             // cost the slices' schedule registers)
-            static_assert(T && CF::ST > 0, "word stores from the transposed blocks");
+            static_assert(T && CF::DL, "word stores from the transposed blocks");
             for (int g = 0; g < nmod; ++g) {
                 slices(Kc / BK);
                 const int l = l0 + g;
@@ -1762,8 +1805,8 @@ static OzSetup ozaki_setup() {
 }
 
 // Tile shape of the residue products. Measured (14 moduli): at 8192^3 the 256 x 256
-// tile takes 6.2-6.4 ms (6.8-7.1 with loads staged through registers and the compiler's
-// read order) against 8.0 ms for 128 x 256 from eight 64 x 64 waves (7.8 with direct loads,
+// tile takes 6.0 ms (6.3 with fragments read within their slice only, 6.8-7.1 with loads staged
+// through registers and the compiler's read order) against 8.0 ms for 128 x 256 from eight 64 x 64 waves (7.8 with direct loads,
 // two blocks per CU); 128 x 256 from four 64 x 128 waves, 256 x 256 from four 128 x 128 waves
 // (which spill), 32 x 32 x 32 MFMAs (11 % slower on the direct-load tile), global loads two
 // slices ahead and 64-byte slices in three or four LDS buffers were no faster. Products at most 256 long on a side
@@ -1827,14 +1870,14 @@ static void launch_i8gemm(rstsr_hip_ctx* ctx, const OzSetup& su, I8Tile tile, co
             // modulus) 1.28 ms at 7 or 14 moduli per block against 1.38-1.44 ms at one; 8192^3
             // (64 slices) the same at one or two.
             int gmod = 1;
-            const bool mm = CF::ST > 0 && TOUT && Kp <= I8_KCHUNK;
+            const bool mm = CF::DL && TOUT && Kp <= I8_KCHUNK;
             if (mm) {
                 const uint64_t blocks = (uint64_t)ntiles * nb;
                 const int64_t ns = Kp / CF::BK;
                 for (int g = 1; g <= n; ++g)
                     if (n % g == 0 && g * ns <= 96 && blocks * (uint64_t)(n / g) >= 1024) gmod = g;
             }
-            auto kern = mm ? k_i8gemm_mod<CF, I8_ROW4G, TOUT, CF::ST != 0 && TOUT>
+            auto kern = mm ? k_i8gemm_mod<CF, I8_ROW4G, TOUT, CF::DL && TOUT>
                            : k_i8gemm_mod<CF, I8_ROW4G, TOUT, false>;
             hipLaunchKernelGGL(kern, dim3(ntiles, (uint32_t)nb, (uint32_t)((n + gmod - 1) / gmod)), dim3(CF::NT), 0,
                                ctx->stream, A8 + k0, B8 + k0, R, Mp, N, Kp, Kc, Np, mods, k0 > 0 ? 1 : 0,
@@ -1856,8 +1899,8 @@ void ozaki_gemm_f64(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, doub
     const int64_t M = P.M, N = P.N, K = P.K;
     if (K > (int64_t)1 << 40) RSTSR_RAISE(UnImplemented, "K too large for the split GEMM");
     I8Tile tile = pick_i8_tile(M, N);
-    // the direct-load tile forms its lanes' load offsets in 32 bits (row < 8, ldk < 2^28)
-    if (tile == I8Tile::Big && K >= ((int64_t)1 << 28) - I8_KPAD) tile = I8Tile::Wide8;
+    // the direct-load tile forms its load offsets in 32 bits (row < 256, ldk < 2^24)
+    if (tile == I8Tile::Big && K >= ((int64_t)1 << 24) - I8_KPAD) tile = I8Tile::Wide8;
     int64_t bm = 0, bn = 0;
     with_i8_tile(tile, [&](auto c) {
         bm = decltype(c)::BM;
@@ -2057,7 +2100,7 @@ void ozaki_gemm_f64(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, doub
 // The products are the three batches of one run of the split GEMM: the operands are read once, as
 // they are, into the residue planes of their three parts, and one CRT pass ends all three. (As three
 // runs, the parts were written out and read back, each product's residues went to C or a plane on
-// their own and a last pass combined them: 4096^3 4.31 ms, now 3.71.)
+// their own and a last pass combined them: 4096^3 4.31 ms, now 3.65.)
 // Returns false, before anything is enqueued, for forms it does not take: operands whose vectors
 // neither have unit stride and at most 8192 elements nor lie side by side, and planes past
 // Z3_MAX_BYTES, since they are three times those of one real product.
