@@ -45,14 +45,18 @@ static bool tile_chunks(bool kc, int64_t sk, int64_t smn) {
 }
 
 // Splits of K for a product whose 64 x 64 tiles leave most of the chip idle: enough blocks for
-// two per CU, each at least eight slices long. By sizes only, so that a product rounds the same
-// whatever its strides and load width.
+// two per CU, each at least eight slices long. Shorter K than the lines below goes to 32 x 32 tiles
+// unsplit, which need no second launch (us, split against not; K of 24, 32 and 40 slices): f64
+// 128^2 12.6, 13.0, 13.0 against 12.1, 15.1, 17.9; 512^2 15.4, 17.3, 20.9 against 12.7, 15.8, 18.7;
+// 256 x 1600 21.3, 21.8, 22.2 against 16.4, 20.4, 24.2; f32 and c64 alike, c128 1000 x 400 at 40 and 48
+// 38.7, 42.3 against 32.2, 37.6. By sizes only, so that a product rounds the same whatever its strides
+// and load width.
 template <class T>
 static uint32_t tile_gemm_splits(const rstsr_hip_ctx* ctx, const GemmProblem& P) {
     const int64_t nsl = (P.K * (int64_t)sizeof(T) + 127) / 128;
     const int64_t t = ((P.M + 63) / 64) * ((P.N + 63) / 64) * (int64_t)P.nbatch;
     const int64_t cu = std::max(ctx->num_cu, 1);
-    if (t >= cu || nsl < 16) return 1;
+    if (t >= cu || nsl < (4 * t < cu ? 28 : sizeof(T) == 16 ? 56 : 40)) return 1;
     return (uint32_t)std::max<int64_t>(1, std::min<int64_t>({(2 * cu + t - 1) / t, nsl / 8, 64}));
 }
 
