@@ -666,11 +666,13 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
             }
           }
         } else if constexpr (TILED && OPS != 0) {
-            // tiles: 64x64 for 8-byte elements, 128 (input axis) x 64 for 4-byte and smaller, 32x64 for 16-byte
+            // tiles (input axis x output axis): 64 x 64 for 8-byte elements, 64 x 128 for 4-byte and smaller,
+            // 32 x 64 for 16-byte. Cut output rows cost more than cut input rows: f32 [333, 509, 255] <- its
+            // reverse 87 us from 128 x 64 tiles, 82 from 64 x 128, [1024, 512, 256] 197 and 192.
             constexpr size_t ES = sizeof(typename Body::TA) > sizeof(typename Body::TB) ? sizeof(typename Body::TA)
                                                                                           : sizeof(typename Body::TB);
-            constexpr int TI = ES > 8 ? 32 : (ES > 4 ? 64 : 128);
-            constexpr int TC = 64;
+            constexpr int TI = ES > 8 ? 32 : 64;
+            constexpr int TC = ES > 4 ? 64 : 128;
             uint32_t ntc = ceil_div_u32(dd.shape[0], TC);
             uint32_t nti = ceil_div_u32(dd.shape[ch.di], TI);
             uint64_t nouter = total / (dd.shape[0] * dd.shape[ch.di]);
@@ -692,6 +694,7 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
                                    dim3((uint32_t)nb), dim3(EW_BLOCK), 0, ctx->stream, body, p, ch.di, od, nti, ntc,
                                    FastDiv(nti), FastDiv(ntc), xmap);
             };
+            constexpr bool WIDE = Body::OUT_SIZE > 8;
             // ONE (at most three axes): streaming variants, staged loads all-or-none, stores in launches
             // of whole tiles only; more axes: plain
             auto by_nt = [&](auto stage) {
@@ -702,14 +705,13 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
                     const bool lo = ((S & 1) == 0 || once[1]) && ((S & 2) == 0 || once[2]);
                     const int h = lo ? hint : hint & 2;
                     if (edge) {
-                        if constexpr (Body::OUT_SIZE > 8) {
-                            if (h == 3) {
-                                go(stage, Y{}, std::integral_constant<int, S | 4>{}, Y{});
-                                return;
-                            }
+                        if constexpr (WIDE) {
+                            if (h == 3) go(stage, Y{}, std::integral_constant<int, S | 4>{}, Y{});
+                            else if (h == 1) go(stage, Y{}, std::integral_constant<int, S>{}, Y{});
+                            else go(stage, Y{}, std::integral_constant<int, 0>{}, Y{});
+                        } else {
+                            go(stage, Y{}, std::integral_constant<int, 0>{}, Y{});
                         }
-                        if (h & 1) go(stage, Y{}, std::integral_constant<int, S>{}, Y{});
-                        else go(stage, Y{}, std::integral_constant<int, 0>{}, Y{});
                         return;
                     }
                     switch (h) {
@@ -747,17 +749,17 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
             bool whole = !edge && lines(0, 0, Body::OUT_SIZE);
             if (ch.stage & 1) whole = whole && lines(1, ch.di, sizeof(typename Body::TA));
             if (ch.stage & 2) whole = whole && lines(2, ch.di, sizeof(typename Body::TB));
-            // candidates {order, hints}. Rows cut inside lines, inputs in turn: f32 [333, 509, 255] <- its
-            // reverse (345 MB) 85 to 89 us with CUT, 130 and more with stores hinted; 16-byte elements
-            // (half as many rows per line) the other way round, c128 [31, 900, 700] <- its last two axes
-            // swapped (625 MB) 111 to 116 us hinted, 125 with CUT.
+            // candidates {order, hints}. Rows cut inside lines, inputs in turn: f64 [333, 509, 255] <- its
+            // reverse (690 MB) 156 us with CUT, 166 to 171 with loads hinted too; f32 82 us, with loads 90,
+            // with stores 130 and more. 16-byte elements (half as many rows per line) the other way round:
+            // c128 [31, 900, 700] <- its last two axes swapped (625 MB) 111 to 116 us hinted, 125 with CUT.
             struct Cand {
                 int xmap, hint;
             };
             static constexpr Cand WHOLE[] = {{0, 3}, {1, 3}, {2, 3}, {3, 3}};
-            static constexpr Cand CUT[] = {{3, 0}, {3, 1}, {1, 1}, {1, 0}};
+            static constexpr Cand CUT[] = {{3, 0}, {1, 0}};
             static constexpr Cand CUT16[] = {{1, 3}, {0, 3}, {2, 3}, {3, 3}};
-            constexpr bool WIDE = Body::OUT_SIZE > 8;
+            const int ncand = whole || WIDE ? 4 : 2;
             const Cand* cands = whole ? WHOLE : (WIDE ? CUT16 : CUT);
             auto use = [&](int c) {
                 xmap = cands[c].xmap;
@@ -775,7 +777,7 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
                                   std::to_string(ntc) + "|" + std::to_string(nti) + "|" + std::to_string(nouter) +
                                   "|" + std::to_string(dd.st[0][1] + dd.st[0][2]) + "|" +
                                   std::to_string(dd.st[ch.di][0]);
-                tune_select(ctx, key, 4, 0, true, [&](int c) {
+                tune_select(ctx, key, ncand, 0, true, [&](int c) {
                     use(c);
                     check_launch("elementwise");
                 });
