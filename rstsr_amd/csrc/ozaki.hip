@@ -328,47 +328,60 @@ __device__ __forceinline__ void for_moduli(const ModSet& ms, F&& f) {
 
 // Tile (v0, t0) of the split: source S(v, t) = s[v*sv + t*st] for v < nv,
 // t < len; planes P[l][v][t] for v < nvp, t < lenp (zero padded; lenp a
-// multiple of 64). The 64 x 64 tile is staged through LDS (`tile`) so that
+// multiple of 128). The tile of TV vectors x TT elements is staged through LDS (`tile`) so that
 // reads run along the source's unit-stride axis and each thread writes 16
 // consecutive plane bytes per modulus. split_load fetches a thread's 16 source
 // elements (zero outside the source), split_store scales them into the tile and
 // writes the residues; split_tile is the two in turn.
+constexpr int SPLIT_TV = 32;
+template <int TV>
+struct SplitShape {
+    static constexpr int TT = 4096 / TV, LDT = TT + 1;
+    using Tile = double[TV][LDT];
+};
+
+template <int TV>
 __device__ __forceinline__ void split_load(const double* __restrict__ s, int64_t nv, int64_t len, int64_t sv,
                                            int64_t st, bool read_along_t, int64_t v0, int64_t t0, double (&x)[16]) {
-    // element k of this thread: the fast index tid % 64 along the unit-stride axis, the slow one
-    // 4k + tid / 64; its address is a uniform base plus a per-lane offset plus k steps of a
+    // element k of this thread: the fast index along the unit-stride axis, the slow one
+    // k steps on from slow0; its address is a uniform base plus a per-lane offset plus k steps of a
     // uniform stride (no per-element 64-bit address kept live)
-    const int tid = threadIdx.x, fast = tid & 63, slow0 = tid >> 6;
+    constexpr int TT = SplitShape<TV>::TT;
+    const int nf = read_along_t ? TT : TV, step = 256 / nf;
+    const int tid = threadIdx.x, fast = tid % nf, slow0 = tid / nf;
     const int64_t lane = read_along_t ? (int64_t)slow0 * sv + (int64_t)fast * st : (int64_t)fast * sv + (int64_t)slow0 * st;
-    const int64_t kstep = 4 * (read_along_t ? sv : st);
+    const int64_t kstep = step * (read_along_t ? sv : st);
     const double* base = s + v0 * sv + t0 * st;
-    if (v0 + 64 <= nv && t0 + 64 <= len) {
+    if (v0 + TV <= nv && t0 + TT <= len) {
 #pragma unroll
         for (int k = 0; k < 16; ++k) x[k] = base[k * kstep + lane];
     } else {
 #pragma unroll
         for (int k = 0; k < 16; ++k) {
-            const int tt = read_along_t ? fast : 4 * k + slow0, vv = read_along_t ? 4 * k + slow0 : fast;
+            const int slow = step * k + slow0;
+            const int tt = read_along_t ? fast : slow, vv = read_along_t ? slow : fast;
             x[k] = v0 + vv < nv && t0 + tt < len ? base[k * kstep + lane] : 0.0;
         }
     }
 }
 
-template <bool K14>
+template <bool K14, int TV>
 __device__ __forceinline__ void split_store(const double (&x)[16], int64_t nv, const int* __restrict__ ev, int64_t nvp,
                                             int64_t lenp, int8_t* __restrict__ planes, const ModSet& ms,
                                             bool read_along_t, int64_t plane, int64_t v0, int64_t t0,
-                                            double (&tile)[64][65]) {
-    const int tid = threadIdx.x;
+                                            typename SplitShape<TV>::Tile& tile) {
+    constexpr int TT = SplitShape<TV>::TT;
+    const int nf = read_along_t ? TT : TV, step = 256 / nf;
+    const int tid = threadIdx.x, fast = tid % nf, slow0 = tid / nf;
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
-        const int e = k * 256 + tid, fast = e & 63, slow = e >> 6;
+        const int slow = step * k + slow0;
         const int tt = read_along_t ? fast : slow, vv = read_along_t ? slow : fast;
         const int64_t gv = v0 + vv;
         tile[vv][tt] = gv < nv ? rint(ldexp(x[k], ev[gv])) : 0.0;
     }
     __syncthreads();
-    const int vv = tid >> 2, tq = (tid & 3) * 16;
+    const int vv = tid / (TT / 16), tq = (tid % (TT / 16)) * 16;
     const int64_t gv = v0 + vv;
     if (gv < nvp) {
         Digits dg[16];
@@ -388,42 +401,43 @@ template <bool K14>
 __device__ __forceinline__ void split_tile(const double* __restrict__ s, int64_t nv, int64_t len, int64_t sv,
                                            int64_t st, const int* __restrict__ ev, int64_t nvp, int64_t lenp,
                                            int8_t* __restrict__ planes, const ModSet& ms, bool read_along_t,
-                                           int64_t plane, int64_t v0, int64_t t0, double (&tile)[64][65]) {
+                                           int64_t plane, int64_t v0, int64_t t0, SplitShape<64>::Tile& tile) {
     double x[16];
-    split_load(s, nv, len, sv, st, read_along_t, v0, t0, x);
-    split_store<K14>(x, nv, ev, nvp, lenp, planes, ms, read_along_t, plane, v0, t0, tile);
+    split_load<64>(s, nv, len, sv, st, read_along_t, v0, t0, x);
+    split_store<K14, 64>(x, nv, ev, nvp, lenp, planes, ms, read_along_t, plane, v0, t0, tile);
 }
 
 // Batch b = blockIdx.z of one operand (`which`: 0 = A, 1 = B offsets of bd):
 // exponents ev + b*nvp, planes + b*nvp*lenp. A block splits tpb tiles along t,
 // the next tile's source loads in flight while it computes the residues of the
-// one before: t tile group blockIdx.x and vector tile blockIdx.y, or the other
-// way round when `swap`.
-template <bool K14>
+// one before. TV, vectors per tile: 64 for sources contiguous along t (either way), t tile group
+// blockIdx.x and vector tile blockIdx.y; 32 for sources contiguous along v, the other way round, so
+// that a tile's plane rows are whole 128-byte lines (8192^2: 324 against 405 us with 64).
+template <bool K14, int TV>
 __global__ void __launch_bounds__(256) k_split(const double* __restrict__ s, int64_t nv, int64_t len, int64_t sv,
                                                int64_t st, BatchDesc bd, int which, const int* __restrict__ ev,
                                                int64_t nvp, int64_t lenp, int8_t* __restrict__ planes, ModSet ms,
-                                               int read_along_t, const int* __restrict__ skip, int64_t plane,
-                                               int tpb, int swap) {
+                                               const int* __restrict__ skip, int64_t plane, int tpb) {
     if (*skip) return;  // non-finite input: the plain kernel computes this product
-    __shared__ double tile[64][65];
+    constexpr int TT = SplitShape<TV>::TT;
+    __shared__ typename SplitShape<TV>::Tile tile;
     const uint32_t b = blockIdx.z;
     int64_t oa, ob, oc;
     batch_offsets(bd, b, oa, ob, oc);
     const double* sb = s + (which ? ob : oa);
     const int* evb = ev + (int64_t)b * nvp;
     int8_t* pb = planes + (int64_t)b * nvp * lenp;
-    const bool along = read_along_t != 0;
-    const uint32_t bx = swap ? blockIdx.y : blockIdx.x, by = swap ? blockIdx.x : blockIdx.y;
-    const int64_t v0 = (int64_t)by * 64, ta = (int64_t)bx * tpb * 64;
-    const int64_t te = min(lenp, ta + (int64_t)tpb * 64);
+    constexpr bool along = TV != SPLIT_TV;
+    const uint32_t bx = along ? blockIdx.x : blockIdx.y, by = along ? blockIdx.y : blockIdx.x;
+    const int64_t v0 = (int64_t)by * TV, ta = (int64_t)bx * tpb * TT;
+    const int64_t te = min(lenp, ta + (int64_t)tpb * TT);
     double x[16];
-    split_load(sb, nv, len, sv, st, along, v0, ta, x);
-    for (int64_t t0 = ta; t0 < te; t0 += 64) {
+    split_load<TV>(sb, nv, len, sv, st, along, v0, ta, x);
+    for (int64_t t0 = ta; t0 < te; t0 += TT) {
         double xn[16];
-        const bool more = t0 + 64 < te;
-        if (more) split_load(sb, nv, len, sv, st, along, v0, t0 + 64, xn);
-        split_store<K14>(x, nv, evb, nvp, lenp, pb, ms, along, plane, v0, t0, tile);
+        const bool more = t0 + TT < te;
+        if (more) split_load<TV>(sb, nv, len, sv, st, along, v0, t0 + TT, xn);
+        split_store<K14, TV>(x, nv, evb, nvp, lenp, pb, ms, along, plane, v0, t0, tile);
         __syncthreads();  // the tile is rewritten for the next t0
         if (more) {
 #pragma unroll
@@ -637,21 +651,22 @@ __global__ void __launch_bounds__(256) k_znorm_cols(const double2* __restrict__ 
 // exponents ev + p nvp, planes + p nvp lenp). Bound by the residues' vector instructions; the one read instead of a pass that
 // writes the parts and three that read them back: see ozaki_zgemm3.
 template <bool K14>
-__global__ void __launch_bounds__(256) k_zsplit(const double2* __restrict__ s, int64_t nv, int64_t len, int64_t sv,
+__global__ void __launch_bounds__(256, 3) k_zsplit(const double2* __restrict__ s, int64_t nv, int64_t len, int64_t sv,
                                                 int64_t st, const int* __restrict__ ev, int64_t nvp, int64_t lenp,
                                                 int8_t* __restrict__ planes, ModSet ms,
                                                 const int* __restrict__ skip, int64_t plane, int tpb) {
     if (*skip) return;  // non-finite input: the plain kernels compute this product
-    __shared__ double tile[64][65];
+    constexpr int TV = SPLIT_TV, TT = SplitShape<TV>::TT;
+    __shared__ SplitShape<TV>::Tile tile;
     // neighbouring blocks take neighbouring vectors, as the lanes do
-    const int64_t v0 = (int64_t)blockIdx.x * 64, ta = (int64_t)blockIdx.y * tpb * 64;
-    const int64_t te = min(lenp, ta + (int64_t)tpb * 64);
-    const int tid = threadIdx.x, fast = tid & 63, slow0 = tid >> 6;
-    for (int64_t t0 = ta; t0 < te; t0 += 64) {
+    const int64_t v0 = (int64_t)blockIdx.x * TV, ta = (int64_t)blockIdx.y * tpb * TT;
+    const int64_t te = min(lenp, ta + (int64_t)tpb * TT);
+    const int tid = threadIdx.x, fast = tid % TV, slow0 = tid / TV;
+    for (int64_t t0 = ta; t0 < te; t0 += TT) {
         double2 x[16];
 #pragma unroll
         for (int k = 0; k < 16; ++k) {
-            const int64_t t = t0 + 4 * k + slow0, v = v0 + fast;
+            const int64_t t = t0 + 256 / TV * k + slow0, v = v0 + fast;
             x[k] = v < nv && t < len ? s[v * sv + t * st] : double2{0.0, 0.0};
         }
 #pragma unroll 1
@@ -659,7 +674,7 @@ __global__ void __launch_bounds__(256) k_zsplit(const double2* __restrict__ s, i
             double y[16];
 #pragma unroll
             for (int k = 0; k < 16; ++k) y[k] = zpart(x[k], p);
-            split_store<K14>(y, nv, ev + p * nvp, nvp, lenp, planes + p * nvp * lenp, ms, false, plane, v0, t0,
+            split_store<K14, TV>(y, nv, ev + p * nvp, nvp, lenp, planes + p * nvp * lenp, ms, false, plane, v0, t0,
                              tile);
             __syncthreads();  // the tile is rewritten
         }
@@ -2032,19 +2047,24 @@ void ozaki_gemm_f64(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, doub
             return;
         }
         run_norm(q, ev);
-        // tpb tiles along K per block while the grid keeps at least eight blocks per CU
-        const uint64_t tiles = (uint64_t)(Kp / 64) * (uint64_t)(nvp / 64) * q.nbx;
         // Sources strided along t (B's columns of a row-major B): consecutive blocks take
         // neighbouring vector tiles, so that the rows they read lie side by side (measured on
         // 8192^3: 400-425 us against 460-540 with the t tiles consecutive and one per block)
-        int tpb = 1;
-        const int swap = std::llabs(st) == 1 ? 0 : 1;
-        while (tpb < 8 && tiles / (uint64_t)(2 * tpb) >= (uint64_t)std::max(ctx->num_cu, 1) * 8) tpb *= 2;
-        const uint32_t gx = (uint32_t)((Kp / 64 + tpb - 1) / tpb), gy = (uint32_t)(nvp / 64);
-        hipLaunchKernelGGL(n == OZ_MAXMOD ? k_split<true> : k_split<false>,
-                           dim3(swap ? gy : gx, swap ? gx : gy, (uint32_t)q.nbx),
-                           dim3(256), 0, ctx->stream, x, nv, K, sv, st, P.bd, which, ev, nvp, Kp, planes, ms,
-                           std::llabs(st) == 1 ? 1 : 0, flag, (int64_t)plane, tpb, swap);
+        auto go = [&](auto tv) {
+            constexpr int TV = decltype(tv)::value, TT = SplitShape<TV>::TT;
+            constexpr int swap = TV == SPLIT_TV ? 1 : 0;
+            // tpb tiles along K per block while the grid keeps at least eight blocks per CU
+            const uint64_t tiles = (uint64_t)(Kp / TT) * (uint64_t)(nvp / TV) * q.nbx;
+            int tpb = 1;
+            while (tpb < 8 && tiles / (uint64_t)(2 * tpb) >= (uint64_t)std::max(ctx->num_cu, 1) * 8) tpb *= 2;
+            const uint32_t gx = (uint32_t)((Kp / TT + tpb - 1) / tpb), gy = (uint32_t)(nvp / TV);
+            hipLaunchKernelGGL((n == OZ_MAXMOD ? k_split<true, TV> : k_split<false, TV>),
+                               dim3(swap ? gy : gx, swap ? gx : gy, (uint32_t)q.nbx),
+                               dim3(256), 0, ctx->stream, x, nv, K, sv, st, P.bd, which, ev, nvp, Kp, planes, ms,
+                               flag, (int64_t)plane, tpb);
+        };
+        if (std::llabs(st) == 1) go(std::integral_constant<int, 64>{});
+        else go(std::integral_constant<int, SPLIT_TV>{});
         check_launch(what);
     };
     norm_split(qa, (const double*)P.a, M, Mp, P.rsa, P.csa, 0, eA, A8, planeA, "ozaki split A");
@@ -2194,10 +2214,11 @@ bool ozaki_zgemm3(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, size_t
                                (int)q.nchunk, q.nvp, g, ev);
         check_launch("ozaki norms");
         // tiles along K per block and the order of the blocks as in ozaki_gemm_f64
-        const uint64_t tiles = (uint64_t)(Kp / 64) * (uint64_t)(q.nvp / 64);
+        constexpr int TV = SPLIT_TV, TT = SplitShape<TV>::TT;
+        const uint64_t tiles = (uint64_t)(Kp / TT) * (uint64_t)(q.nvp / TV);
         int tpb = 1;
         while (tpb < 8 && tiles / (uint64_t)(2 * tpb) >= (uint64_t)std::max(ctx->num_cu, 1) * 8) tpb *= 2;
-        const uint32_t gx = (uint32_t)((Kp / 64 + tpb - 1) / tpb), gy = (uint32_t)(q.nvp / 64);
+        const uint32_t gx = (uint32_t)((Kp / TT + tpb - 1) / tpb), gy = (uint32_t)(q.nvp / TV);
         hipLaunchKernelGGL(n == OZ_MAXMOD ? k_zsplit<true> : k_zsplit<false>, dim3(gy, gx), dim3(256), 0, ctx->stream, q.x,
                            q.nv, K, q.sv, q.st, ev, q.nvp, Kp, planes, ms, flag, (int64_t)plane, tpb);
         check_launch(what);
