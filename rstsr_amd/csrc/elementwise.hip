@@ -198,6 +198,7 @@ struct BinBody {
     T sa, sb;
     static constexpr int OPS = (AS ? 0 : 1) | (BS ? 0 : 2);
     static constexpr size_t OUT_SIZE = sizeof(T);
+    static constexpr bool UNARY = false;
     template <bool NT = false>
     __device__ __forceinline__ T la(int64_t o) const { return AS ? sa : ld<NT>(a + o); }
     template <bool NT = false>
@@ -220,6 +221,7 @@ struct MixBody {
     TBv sb;
     static constexpr int OPS = (AS ? 0 : 1) | (BS ? 0 : 2);
     static constexpr size_t OUT_SIZE = sizeof(C);
+    static constexpr bool UNARY = false;
     template <bool NT = false>
     __device__ __forceinline__ TAv la(int64_t o) const { return AS ? sa : ld<NT>(a + o); }
     template <bool NT = false>
@@ -243,6 +245,7 @@ struct CastBody {
     const TAv* a;
     static constexpr int OPS = 1;
     static constexpr size_t OUT_SIZE = sizeof(TCv);
+    static constexpr bool UNARY = false;
     template <bool NT = false>
     __device__ __forceinline__ TAv la(int64_t o) const { return ld<NT>(a + o); }
     template <bool NT = false>
@@ -261,6 +264,7 @@ struct FillBody {
     T v;
     static constexpr int OPS = 0;
     static constexpr size_t OUT_SIZE = sizeof(T);
+    static constexpr bool UNARY = false;
     template <bool NT = false>
     __device__ __forceinline__ None la(int64_t) const { return None{}; }
     template <bool NT = false>
@@ -312,6 +316,7 @@ struct CloseBody {
     int equal_nan;
     static constexpr int OPS = 3;
     static constexpr size_t OUT_SIZE = 0;
+    static constexpr bool UNARY = false;
     template <bool NT = false>
     __device__ __forceinline__ T la(int64_t o) const { return ld<NT>(a + o); }
     template <bool NT = false>

@@ -556,14 +556,60 @@ constexpr uint64_t EW_NT_FLAT_MIN = 256ull << 20;
 // Tiled launches moving at least this many bytes have their tile order tuned.
 constexpr uint64_t EW_TUNE_MIN = 32ull << 20;
 
+// Call f(std::integral_constant<int, v>) for the runtime value v in [0, 8),
+// instantiating only masks whose load bits are operands the body has.
+template <int OPS, class F>
+static void with_ntm(int v, F&& f) {
+    auto one = [&](auto c) {
+        constexpr int V = decltype(c)::value;
+        if constexpr (((V & 3) & ~OPS) == 0) f(c);
+    };
+    switch (v & 7) {
+        case 0: one(std::integral_constant<int, 0>{}); break;
+        case 1: one(std::integral_constant<int, 1>{}); break;
+        case 2: one(std::integral_constant<int, 2>{}); break;
+        case 3: one(std::integral_constant<int, 3>{}); break;
+        case 4: one(std::integral_constant<int, 4>{}); break;
+        case 5: one(std::integral_constant<int, 5>{}); break;
+        case 6: one(std::integral_constant<int, 6>{}); break;
+        default: one(std::integral_constant<int, 7>{}); break;
+    }
+}
+
+template <class T>
+constexpr bool is_complex_v = std::is_same<T, c64>::value || std::is_same<T, c128>::value;
+
+// Whether a body gains from the flat kernel on operands that allow it. Measured (us, rows or generic
+// kernel against flat): f32 [4000, 2048] + the same 16.2 and 12.8, sin of 160 MB 70 and 55; f64 + a row
+// 27 and 22, sin of 320 MB 116 and 106. Not for operands with gaps between their rows, except 4-byte
+// ones (f64 [20000, 2048] of 2100 columns + the same 127 and 141, sin of [4000, 2048] 27 and 31); not
+// for complex functions and single-operand passes over 16-byte elements (c128 exp of 186 MB 68 and
+// 79), which gain no wider access; not for fills.
+template <class Body>
+static bool flat_pays(const Dims& d) {
+    constexpr int OPS = Body::OPS;
+    constexpr size_t EA = sizeof(typename Body::TA), EB = sizeof(typename Body::TB);
+    constexpr size_t ES = std::max({(OPS & 1) ? EA : (size_t)1, (OPS & 2) ? EB : (size_t)1, Body::OUT_SIZE});
+    if (OPS == 0 || (Body::UNARY && is_complex_v<typename Body::TA>) || (ES >= 16 && OPS != 3)) return false;
+    if (ES <= 4) return true;
+    for (int k = 1; k <= 2; ++k) {
+        if (!(OPS >> (k - 1) & 1) || is_flat(d, k)) continue;
+        bool bcast = false;
+        for (int i = 0; i < d.nd; ++i) bcast = bcast || d.st[i][k] == 0;
+        if (!bcast) return false;
+    }
+    return true;
+}
+
 // Launch `body` over the plan, splitting the outermost axis so that every
 // launch indexes fewer than 2^31 elements with 32-bit arithmetic.
 // TILED = false: the LDS-tiled kernel is not instantiated for this body, and a
 // tiled choice runs the generic kernel instead.
 // Streaming hints (compile-time kernel variants): loads of operands read once,
-// stores of outputs of at least EW_NT_STORE_MIN bytes.
-// NTV = false: only the plain (hint-free) variant of the flat kernel is instantiated, for bodies
-// off the hot path.
+// stores of outputs of at least EW_NT_STORE_MIN bytes. Unary bodies take the hints of the row
+// kernel together or not at all.
+// NTV = false: only the plain (hint-free) variants of the row and flat kernels are instantiated, for
+// bodies off the hot path.
 template <class Body, bool TILED = true, bool NTV = true>
 static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch, bool can_time = false) {
     constexpr int OPS = Body::OPS;
@@ -571,7 +617,7 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
     if (OPS == 0 && ch.kind == EwKind::Tiled) ch.kind = EwKind::Generic;
     if (d.nd < 0) return;
     // a piece cut out of a contiguous output need not be contiguous any more; no output, no packs
-    if (ch.kind == EwKind::Flat && (d.nd < 1 || Body::OUT_SIZE == 0 || !is_flat(d, 0)))
+    if (ch.kind == EwKind::Flat && (d.nd < 1 || Body::OUT_SIZE == 0 || !is_flat(d, 0) || !flat_pays<Body>(d)))
         ch.kind = d.nd >= 1 && d.shape[0] >= (uint64_t)(EW_BLOCK * EW_VEC) ? EwKind::Rows : EwKind::Generic;
     if (d.nd == 0) {
         d.nd = 1;
@@ -618,6 +664,7 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
             if (d.shape[i] > 1 && d.st[i][k] == 0) once[k] = false;
     const bool big = Body::OUT_SIZE > 0 && all * Body::OUT_SIZE >= EW_NT_STORE_MIN;
     int lmask = ((OPS & 1) && once[1] ? 1 : 0) | ((OPS & 2) && once[2] ? 2 : 0);
+    const int rows_ntm = !Body::UNARY ? lmask | (big ? 4 : 0) : (lmask == OPS && big ? OPS | 4 : 0);
     const int flat_ntm = lmask != 0 && all * Body::OUT_SIZE >= EW_NT_FLAT_MIN ? (lmask | 4) : 0;
 
     uint64_t inner = 1;
@@ -641,104 +688,43 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
             uint64_t nrows = total / dd.shape[0];
             uint64_t nb = nrows * nchunk;
             if (nb >= LIM) RSTSR_RAISE(UnImplemented, "grid too large");
-            hipLaunchKernelGGL((k_ew_rows<Body, 0>), dim3((uint32_t)nb), dim3(EW_BLOCK), 0, ctx->stream, body, p, nchunk,
-                               FastDiv(nchunk));
-        } else if (ch.kind == EwKind::Flat) {
-          if constexpr (Body::OUT_SIZE > 0) {
-            constexpr size_t EA = sizeof(typename Body::TA), EB = sizeof(typename Body::TB);
-            constexpr size_t ES = std::max({(OPS & 1) ? EA : (size_t)1, (OPS & 2) ? EB : (size_t)1, Body::OUT_SIZE});
-            // two packs per thread for two operands: one leaves the second operand's index math and
-            // load latency uncovered (27 us against 17 above), four cost occupancy
-            constexpr int VEC = ES >= 16 ? 1 : (ES >= 8 ? 2 : 4), U = OPS == 3 ? 2 : 1;
-            const int same = (is_flat(dd, 1) ? 2 : 0) | (is_flat(dd, 2) ? 4 : 0);
-            const uint32_t nb = ceil_div_u32(total, (uint64_t)EW_BLOCK * U * VEC);
             auto go = [&](auto ntm) {
-                hipLaunchKernelGGL((k_ew_flat<Body, VEC, U, decltype(ntm)::value>), dim3(nb), dim3(EW_BLOCK), 0, ctx->stream,
-                                   body, p, (uint32_t)total, same);
+                hipLaunchKernelGGL((k_ew_rows<Body, decltype(ntm)::value>), dim3((uint32_t)nb), dim3(EW_BLOCK), 0,
+                                   ctx->stream, body, p, nchunk, FastDiv(nchunk));
             };
-            if constexpr (!NTV || OPS == 0) {
+            if constexpr (!NTV) {
                 go(std::integral_constant<int, 0>{});
+            } else if constexpr (Body::UNARY) {
+                if (rows_ntm) go(std::integral_constant<int, OPS | 4>{});
+                else go(std::integral_constant<int, 0>{});
             } else {
-                if (flat_ntm == 0) go(std::integral_constant<int, 0>{});
-                else if (flat_ntm == (OPS | 4)) go(std::integral_constant<int, OPS | 4>{});
-                else if (flat_ntm == 5) go(std::integral_constant<int, (OPS & 1) | 4>{});
-                else go(std::integral_constant<int, (OPS & 2) | 4>{});
+                with_ntm<OPS>(rows_ntm, go);
             }
-          }
+        } else if (ch.kind == EwKind::Flat) {
+            if constexpr (Body::OUT_SIZE > 0) {
+                constexpr size_t EA = sizeof(typename Body::TA), EB = sizeof(typename Body::TB);
+                constexpr size_t ES = std::max({(OPS & 1) ? EA : (size_t)1, (OPS & 2) ? EB : (size_t)1, Body::OUT_SIZE});
+                // two packs per thread for two operands: one leaves the second operand's index math and
+                // load latency uncovered (27 us against 17 above), four cost occupancy
+                constexpr int VEC = ES >= 16 ? 1 : (ES >= 8 ? 2 : 4), U = OPS == 3 ? 2 : 1;
+                const int same = (is_flat(dd, 1) ? 2 : 0) | (is_flat(dd, 2) ? 4 : 0);
+                const uint32_t nb = ceil_div_u32(total, (uint64_t)EW_BLOCK * U * VEC);
+                auto go = [&](auto ntm) {
+                    hipLaunchKernelGGL((k_ew_flat<Body, VEC, U, decltype(ntm)::value>), dim3(nb), dim3(EW_BLOCK), 0, ctx->stream,
+                                       body, p, (uint32_t)total, same);
+                };
+                if constexpr (!NTV || OPS == 0) {
+                    go(std::integral_constant<int, 0>{});
+                } else {
+                    if (flat_ntm == 0) go(std::integral_constant<int, 0>{});
+                    else if (flat_ntm == (OPS | 4)) go(std::integral_constant<int, OPS | 4>{});
+                    else if (flat_ntm == 5) go(std::integral_constant<int, (OPS & 1) | 4>{});
+                    else go(std::integral_constant<int, (OPS & 2) | 4>{});
+                }
+            }
         } else if constexpr (TILED && OPS != 0) {
-            // tiles (input axis x output axis): 64 x 64 for 8-byte elements, 64 x 128 for 4-byte and smaller,
-            // 32 x 64 for 16-byte. Cut output rows cost more than cut input rows: f32 [333, 509, 255] <- its
-            // reverse 87 us from 128 x 64 tiles, 82 from 64 x 128, [1024, 512, 256] 197 and 192.
             constexpr size_t ES = sizeof(typename Body::TA) > sizeof(typename Body::TB) ? sizeof(typename Body::TA)
                                                                                           : sizeof(typename Body::TB);
-            constexpr int TI = ES > 8 ? 32 : 64;
-            constexpr int TC = ES > 4 ? 64 : 128;
-            uint32_t ntc = ceil_div_u32(dd.shape[0], TC);
-            uint32_t nti = ceil_div_u32(dd.shape[ch.di], TI);
-            uint64_t nouter = total / (dd.shape[0] * dd.shape[ch.di]);
-            uint64_t nb = nouter * nti * ntc;
-            if (nb >= LIM) RSTSR_RAISE(UnImplemented, "grid too large");
-            int od = -1;
-            for (int k = 1; k < dd.nd; ++k)
-                if (k != ch.di) od = k;
-
-            // Tile orders (xmap) and streaming hints (bit 0: staged loads, bit 1: stores). Rows whose
-            // tile segments start and end inside 128-byte lines share those lines with neighbouring
-            // tiles: hints would fetch or write them twice, so such launches choose among fewer hints,
-            // with orders that keep neighbours on one XCD.
-            int xmap = 0, hint = 0;
-            const bool edge = dd.shape[0] % TC != 0 || dd.shape[ch.di] % TI != 0;
-            auto go = [&](auto stage, auto one, auto ntm, auto eg) {
-                hipLaunchKernelGGL((k_ew_tiled<Body, TI, TC, decltype(stage)::value, decltype(one)::value,
-                                               decltype(ntm)::value, decltype(eg)::value>),
-                                   dim3((uint32_t)nb), dim3(EW_BLOCK), 0, ctx->stream, body, p, ch.di, od, nti, ntc,
-                                   FastDiv(nti), FastDiv(ntc), xmap);
-            };
-            constexpr bool WIDE = Body::OUT_SIZE > 8;
-            // ONE (at most three axes): streaming variants, staged loads all-or-none, stores in launches
-            // of whole tiles only; more axes: plain
-            auto by_nt = [&](auto stage) {
-                constexpr int S = decltype(stage)::value;
-                using Y = std::true_type;
-                using N = std::false_type;
-                if (dd.nd <= 3) {
-                    const bool lo = ((S & 1) == 0 || once[1]) && ((S & 2) == 0 || once[2]);
-                    const int h = lo ? hint : hint & 2;
-                    if (edge) {
-                        if constexpr (WIDE) {
-                            if (h == 3) go(stage, Y{}, std::integral_constant<int, S | 4>{}, Y{});
-                            else if (h == 1) go(stage, Y{}, std::integral_constant<int, S>{}, Y{});
-                            else go(stage, Y{}, std::integral_constant<int, 0>{}, Y{});
-                        } else {
-                            go(stage, Y{}, std::integral_constant<int, 0>{}, Y{});
-                        }
-                        return;
-                    }
-                    switch (h) {
-                        case 0: go(stage, Y{}, std::integral_constant<int, 0>{}, N{}); break;
-                        case 1: go(stage, Y{}, std::integral_constant<int, S>{}, N{}); break;
-                        case 2: go(stage, Y{}, std::integral_constant<int, 4>{}, N{}); break;
-                        default: go(stage, Y{}, std::integral_constant<int, S | 4>{}, N{}); break;
-                    }
-                } else {
-                    go(stage, N{}, std::integral_constant<int, 0>{}, Y{});
-                }
-            };
-            // choose() tiles along an input's unit axis, so that input is always staged:
-            // a body with one array operand stages exactly that one
-            auto launch = [&]() {
-                if constexpr (OPS == 1) {
-                    by_nt(std::integral_constant<int, 1>{});
-                } else if constexpr (OPS == 2) {
-                    by_nt(std::integral_constant<int, 2>{});
-                } else {
-                    switch (ch.stage) {
-                        case 1: by_nt(std::integral_constant<int, 1>{}); break;
-                        case 2: by_nt(std::integral_constant<int, 2>{}); break;
-                        default: by_nt(std::integral_constant<int, 3>{}); break;
-                    }
-                }
-            };
             // whole lines: the output's rows along dim 0 and the staged inputs' rows along the input axis
             auto lines = [&](int k, int unit, size_t es) {
                 bool ok = dd.off[k] * (int64_t)es % 128 == 0 && dd.shape[unit] * es % 128 == 0;
@@ -746,44 +732,120 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
                     if (i != unit) ok = ok && dd.st[i][k] * (int64_t)es % 128 == 0;
                 return ok;
             };
-            bool whole = !edge && lines(0, 0, Body::OUT_SIZE);
+            bool whole = lines(0, 0, Body::OUT_SIZE) && dd.shape[0] % 64 == 0 &&
+                         dd.shape[ch.di] % (ES > 8 ? 32 : ES > 4 ? 64 : 128) == 0;
             if (ch.stage & 1) whole = whole && lines(1, ch.di, sizeof(typename Body::TA));
             if (ch.stage & 2) whole = whole && lines(2, ch.di, sizeof(typename Body::TB));
-            // candidates {order, hints}. Rows cut inside lines, inputs in turn: f64 [333, 509, 255] <- its
-            // reverse (690 MB) 156 us with CUT, 166 to 171 with loads hinted too; f32 82 us, with loads 90,
-            // with stores 130 and more. 16-byte elements (half as many rows per line) the other way round:
-            // c128 [31, 900, 700] <- its last two axes swapped (625 MB) 111 to 116 us hinted, 125 with CUT.
-            struct Cand {
-                int xmap, hint;
+            auto tiled = [&](auto cut_c) {
+                constexpr bool CUTL = decltype(cut_c)::value;
+                // tiles (input axis x output axis): 64 x 64 for 8-byte elements, 32 x 64 for 16-byte; for 4-byte and
+                // smaller 128 x 64, of cut lines 64 x 128, since cut output rows cost more than cut input
+                // rows: f32 [333, 509, 255] <- its reverse 87 us from 128 x 64 tiles, 82 from 64 x 128, the whole
+                // lines of the strided [1024, 256, 256] multiply 95 and 100.
+                constexpr int TI = ES > 8 ? 32 : (ES > 4 || CUTL ? 64 : 128);
+                constexpr int TC = ES > 4 || !CUTL ? 64 : 128;
+                uint32_t ntc = ceil_div_u32(dd.shape[0], TC);
+                uint32_t nti = ceil_div_u32(dd.shape[ch.di], TI);
+                uint64_t nouter = total / (dd.shape[0] * dd.shape[ch.di]);
+                uint64_t nb = nouter * nti * ntc;
+                if (nb >= LIM) RSTSR_RAISE(UnImplemented, "grid too large");
+                int od = -1;
+                for (int k = 1; k < dd.nd; ++k)
+                    if (k != ch.di) od = k;
+
+                // Tile orders (xmap) and streaming hints (bit 0: staged loads, bit 1: stores). Rows whose
+                // tile segments start and end inside 128-byte lines share those lines with neighbouring
+                // tiles: hints would fetch or write them twice, so such launches choose among fewer hints,
+                // with orders that keep neighbours on one XCD.
+                int xmap = 0, hint = 0;
+                auto go = [&](auto stage, auto one, auto ntm, auto eg) {
+                    hipLaunchKernelGGL((k_ew_tiled<Body, TI, TC, decltype(stage)::value, decltype(one)::value,
+                                                   decltype(ntm)::value, decltype(eg)::value>),
+                                       dim3((uint32_t)nb), dim3(EW_BLOCK), 0, ctx->stream, body, p, ch.di, od, nti, ntc,
+                                       FastDiv(nti), FastDiv(ntc), xmap);
+                };
+                constexpr bool WIDE = Body::OUT_SIZE > 8;
+                // ONE (at most three axes): streaming variants, staged loads all-or-none, stores in launches
+                // of whole tiles only; more axes: plain
+                auto by_nt = [&](auto stage) {
+                    constexpr int S = decltype(stage)::value;
+                    using Y = std::true_type;
+                    using N = std::false_type;
+                    if (dd.nd <= 3) {
+                        const bool lo = ((S & 1) == 0 || once[1]) && ((S & 2) == 0 || once[2]);
+                        const int h = lo ? hint : hint & 2;
+                        if constexpr (CUTL) {
+                            if constexpr (WIDE) {
+                                if (h == 3) go(stage, Y{}, std::integral_constant<int, S | 4>{}, Y{});
+                                else if (h == 1) go(stage, Y{}, std::integral_constant<int, S>{}, Y{});
+                                else go(stage, Y{}, std::integral_constant<int, 0>{}, Y{});
+                            } else {
+                                go(stage, Y{}, std::integral_constant<int, 0>{}, Y{});
+                            }
+                        } else
+                        switch (h) {
+                            case 0: go(stage, Y{}, std::integral_constant<int, 0>{}, N{}); break;
+                            case 1: go(stage, Y{}, std::integral_constant<int, S>{}, N{}); break;
+                            case 2: go(stage, Y{}, std::integral_constant<int, 4>{}, N{}); break;
+                            default: go(stage, Y{}, std::integral_constant<int, S | 4>{}, N{}); break;
+                        }
+                    } else {
+                        go(stage, N{}, std::integral_constant<int, 0>{}, Y{});
+                    }
+                };
+                // choose() tiles along an input's unit axis, so that input is always staged:
+                // a body with one array operand stages exactly that one
+                auto launch = [&]() {
+                    if constexpr (OPS == 1) {
+                        by_nt(std::integral_constant<int, 1>{});
+                    } else if constexpr (OPS == 2) {
+                        by_nt(std::integral_constant<int, 2>{});
+                    } else {
+                        switch (ch.stage) {
+                            case 1: by_nt(std::integral_constant<int, 1>{}); break;
+                            case 2: by_nt(std::integral_constant<int, 2>{}); break;
+                            default: by_nt(std::integral_constant<int, 3>{}); break;
+                        }
+                    }
+                };
+                // candidates {order, hints}. Rows cut inside lines, inputs in turn: f64 [333, 509, 255] <- its
+                // reverse (690 MB) 156 us with CUT, 166 to 171 with loads hinted too; f32 82 us, with loads 90,
+                // with stores 130 and more. 16-byte elements (half as many rows per line) the other way round:
+                // c128 [31, 900, 700] <- its last two axes swapped (625 MB) 111 to 116 us hinted, 125 with CUT.
+                struct Cand {
+                    int xmap, hint;
+                };
+                static constexpr Cand WHOLE[] = {{0, 3}, {1, 3}, {2, 3}, {3, 3}};
+                static constexpr Cand CUT[] = {{3, 0}, {1, 0}};
+                static constexpr Cand CUT16[] = {{1, 3}, {0, 3}, {2, 3}, {3, 3}};
+                constexpr int ncand = !CUTL || WIDE ? 4 : 2;
+                const Cand* cands = !CUTL ? WHOLE : (WIDE ? CUT16 : CUT);
+                auto use = [&](int c) {
+                    xmap = cands[c].xmap;
+                    hint = cands[c].hint;
+                    if ((!CUTL || WIDE) && !big) hint &= 1;  // outputs that the last-level cache can hold are not streamed
+                    launch();
+                };
+                // The fastest order depends on how the shapes and strides meet the
+                // HBM channel interleave (measured: either order can win by 5-10 %), so it
+                // is tuned per problem class on launches of at least EW_TUNE_MIN bytes.
+                const uint64_t bytes = total * (sizeof(typename Body::TA) + Body::OUT_SIZE);
+                if (can_time && per >= nlast && bytes >= EW_TUNE_MIN) {
+                    std::string key = std::string(!CUTL ? "ew|" : "ew|c|") + std::to_string(sizeof(typename Body::TA)) + "|" +
+                                      std::to_string(Body::OUT_SIZE) + "|" + std::to_string(ch.stage) + "|" +
+                                      std::to_string(ntc) + "|" + std::to_string(nti) + "|" + std::to_string(nouter) +
+                                      "|" + std::to_string(dd.st[0][1] + dd.st[0][2]) + "|" +
+                                      std::to_string(dd.st[ch.di][0]);
+                    tune_select(ctx, key, ncand, 0, true, [&](int c) {
+                        use(c);
+                        check_launch("elementwise");
+                    });
+                } else {
+                    use(0);
+                }
             };
-            static constexpr Cand WHOLE[] = {{0, 3}, {1, 3}, {2, 3}, {3, 3}};
-            static constexpr Cand CUT[] = {{3, 0}, {1, 0}};
-            static constexpr Cand CUT16[] = {{1, 3}, {0, 3}, {2, 3}, {3, 3}};
-            const int ncand = whole || WIDE ? 4 : 2;
-            const Cand* cands = whole ? WHOLE : (WIDE ? CUT16 : CUT);
-            auto use = [&](int c) {
-                xmap = cands[c].xmap;
-                hint = cands[c].hint;
-                if ((whole || WIDE) && !big) hint &= 1;  // outputs that the last-level cache can hold are not streamed
-                launch();
-            };
-            // The fastest order depends on how the shapes and strides meet the
-            // HBM channel interleave (measured: either order can win by 5-10 %), so it
-            // is tuned per problem class on launches of at least EW_TUNE_MIN bytes.
-            const uint64_t bytes = total * (sizeof(typename Body::TA) + Body::OUT_SIZE);
-            if (can_time && per >= nlast && bytes >= EW_TUNE_MIN) {
-                std::string key = std::string(whole ? "ew|" : "ew|c|") + std::to_string(sizeof(typename Body::TA)) + "|" +
-                                  std::to_string(Body::OUT_SIZE) + "|" + std::to_string(ch.stage) + "|" +
-                                  std::to_string(ntc) + "|" + std::to_string(nti) + "|" + std::to_string(nouter) +
-                                  "|" + std::to_string(dd.st[0][1] + dd.st[0][2]) + "|" +
-                                  std::to_string(dd.st[ch.di][0]);
-                tune_select(ctx, key, ncand, 0, true, [&](int c) {
-                    use(c);
-                    check_launch("elementwise");
-                });
-            } else {
-                use(0);
-            }
+            if (whole) tiled(std::false_type{});
+            else tiled(std::true_type{});
         }
         check_launch("elementwise");
     }

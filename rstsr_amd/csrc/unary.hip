@@ -316,6 +316,7 @@ struct UnBody {
     const TAv* a;
     static constexpr int OPS = 1;
     static constexpr size_t OUT_SIZE = sizeof(TCv);
+    static constexpr bool UNARY = true;
     template <bool NT = false>
     __device__ __forceinline__ TAv la(int64_t o) const { return ld<NT>(a + o); }
     template <bool NT = false>
@@ -335,6 +336,7 @@ struct ToF64Body {
     const TAv* a;
     static constexpr int OPS = 1;
     static constexpr size_t OUT_SIZE = sizeof(double);
+    static constexpr bool UNARY = true;
     template <bool NT = false>
     __device__ __forceinline__ TAv la(int64_t o) const { return ld<NT>(a + o); }
     template <bool NT = false>
