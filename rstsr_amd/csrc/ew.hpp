@@ -111,9 +111,10 @@ __device__ __forceinline__ void store_pack(T* p, const T (&v)[N]) {
 // flat: the output is contiguous, so each thread takes U packs of VEC consecutive elements and
 // stores each as one word. Operands laid out like the output (bit k of `same`) load the same way;
 // others are broadcast or contiguous along dim 0 (stride 0 or 1): their row (dims 1 ..) is
-// unravelled once per pack, and once more for a pack that crosses into the next row. Bound by HBM (or the last-level cache): what it saves over the generic kernel is
-// the index math per element and three quarters of the load and store instructions of 4-byte types.
-// NTM as below. Measurements at untiled_kind.
+// unravelled once per pack, and once more for a pack that crosses into the next row. Bound by HBM
+// (or the last-level cache): what it saves over the generic kernel is the index math per element and
+// three quarters of the load and store instructions of 4-byte types.
+// NTM as below. Measurements at untiled_kind and flat_pays.
 template <class Body, int VEC, int U, int NTM>
 __global__ void __launch_bounds__(EW_BLOCK) k_ew_flat(Body body, EwPlan p, uint32_t total, int same) {
     using TA = typename Body::TA;
