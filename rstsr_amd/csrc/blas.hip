@@ -77,9 +77,11 @@ __device__ __forceinline__ T t_mul(T a, T b) {
     else return a * b;
 }
 
-// Quotients by one divisor, as accurate as divisions and without their branches: both parts are
-// scaled to [1/2, 1), q = a r is corrected by its exact remainder (r = 1/d), and the exponents are put
-// back; v_div_fixup gives zeros, infinities and NaN their IEEE results.
+// Quotients by one divisor, rounded as IEEE divisions are and without their setup per quotient: both
+// parts are scaled to [1/2, 1); q = a r (r the rounded reciprocal) is corrected by its exact remainder
+// to a neighbour of the quotient, and once more to the rounded one (Markstein's theorem); the
+// exponents are put back, and v_div_fixup gives zeros, infinities and NaN their IEEE results. A result
+// below the normal range would be rounded a second time there: such lanes divide.
 template <class R>
 struct Recip {
     R d, m, r;
@@ -97,12 +99,17 @@ struct Recip {
         return {d, m, (R)1 / m, expo(d)};
     }
     __device__ __forceinline__ R quot(R a) const {
+        constexpr int LOW = sizeof(R) == 8 ? -1021 : -125;  // frexp exponent of the smallest normal number
         const R am = mant(a);
+        const int ex = expo(a) - e;
         R q = am * r;
         q = fma(fma(-m, q, am), r, q);
-        q = ldexp(q, expo(a) - e);
-        if constexpr (sizeof(R) == 8) return __builtin_amdgcn_div_fixup(q, d, a);
-        else return __builtin_amdgcn_div_fixupf(q, d, a);
+        q = fma(fma(-m, q, am), r, q);
+        q = ldexp(q, ex);
+        if constexpr (sizeof(R) == 8) q = __builtin_amdgcn_div_fixup(q, d, a);
+        else q = __builtin_amdgcn_div_fixupf(q, d, a);
+        if (ex < LOW) q = a / d;  // the quotient's own exponent is ex or ex + 1
+        return q;
     }
 };
 // The divisor of one row of the solve. Complex: a conj(b) / |b|^2 with b scaled by its larger part

@@ -1,0 +1,30 @@
+"""Values the triangular solve must return exactly: quotients, unit diagonals, sums of many terms."""
+import numpy as np
+import pytest
+
+import rstsr_amd as rt
+from test_gpu_trsm_block import LEFT, LOWER, NONUNIT, UNIT, UPPER, solve
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return rt.DeviceHIP(0)
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_quotients_round_as_divisions(dev, dt):
+    """A diagonal matrix of 40 divisors: every element is one quotient (b - 0 is b), equal to the IEEE
+    division's, subnormal results among them. 40 rows: the block kernel."""
+    rng = np.random.default_rng(21)
+    fi = np.finfo(dt)
+    s, r = 40, 3000
+    d = (rng.uniform(1, 2, size=s) * np.exp2(rng.integers(-20, 21, size=s))).astype(dt)
+    d[::7] = -d[::7]
+    lo = np.exp2(rng.integers(fi.minexp - fi.nmant, fi.minexp + 25, size=(s, r)).astype(np.float64))
+    b = rng.uniform(-2, 2, size=(s, r)) * np.where(rng.random((s, r)) < 0.5, 1.0, lo)
+    b = b.astype(dt)
+    want = b / d[:, None]
+    assert np.any((want != 0) & (np.abs(want) < fi.tiny)) and np.all(np.isfinite(want))
+    assert np.array_equal(solve(dev, np.diag(d), b, LEFT, LOWER, NONUNIT), want)
