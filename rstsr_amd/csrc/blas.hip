@@ -271,7 +271,8 @@ __global__ void __launch_bounds__(64 * TRSM_NW) k_trsm_block(const T* __restrict
 #pragma unroll
                 for (int k = 0; k < 4; ++k) d[k] = diag[f][c + 1][MM::row(k, lane)];
             }
-            const T xc = dc.quot(b[k0]);
+            // no quotient by one: (inf + i nan) / 1 would spread the NaN
+            const T xc = unit ? b[k0] : dc.quot(b[k0]);
             if (q == g) b[k0] = xc;
             const T xb = bcast_rows(xc, g);
 #pragma unroll

@@ -28,3 +28,21 @@ def test_quotients_round_as_divisions(dev, dt):
     want = b / d[:, None]
     assert np.any((want != 0) & (np.abs(want) < fi.tiny)) and np.all(np.isfinite(want))
     assert np.array_equal(solve(dev, np.diag(d), b, LEFT, LOWER, NONUNIT), want)
+
+
+@pytest.mark.parametrize("dt", [np.complex64, np.complex128])
+@pytest.mark.parametrize("uplo", [LOWER, UPPER])
+def test_unit_diagonal_keeps_non_finite_parts(dev, dt, uplo):
+    """A unit diagonal divides nothing: rows that nothing is subtracted from come back as they are,
+    each part's infinities and NaN to itself."""
+    parts = [3.0, -0.5, np.inf, -np.inf, np.nan]
+    b0 = np.array([complex(re, im) for re in parts for im in parts], dtype=dt)
+    for s in (1, 20, 40):
+        b = np.ones((s, b0.size), dtype=dt)
+        first = 0 if uplo == LOWER else s - 1
+        b[first] = b0
+        a = np.zeros((s, s), dtype=dt)
+        np.fill_diagonal(a, np.nan)  # not read
+        got = solve(dev, a, b, LEFT, uplo, UNIT)[first]
+        for g, w in ((got.real, b0.real), (got.imag, b0.imag)):
+            assert np.array_equal(g, w, equal_nan=True), s
