@@ -173,8 +173,8 @@ constexpr int TRSM_FPW = TRSM_F / TRSM_NW;   // fragments per wave
 //
 // What bounds it: the chain over the rows (a column's x[i] needs every x before it), so all of it
 // runs in one launch and each step is kept short. A block owns 16 columns of X, which are
-// independent of all others: r / 16 blocks without any exchange. X stays in the matrix cores'
-// accumulators, fragment f (rows 16 f ..) in wave f % 8. Step j: the wave that owns fragment j
+// independent of all others: r / 16 blocks without any exchange. X stays in registers, its updates in
+// the matrix cores' accumulators, fragment f (rows 16 f ..) in wave f % 8. Step j: the wave that owns fragment j
 // subtracts block j - 1's share from it (four MFMAs), solves its 16 rows by substitution in the
 // accumulators' own layout and publishes x through LDS; after one barrier the waves subtract
 // T(f, j) x from their fragments below, with the blocks of T loaded a step ahead.
@@ -210,19 +210,18 @@ __global__ void __launch_bounds__(64 * TRSM_NW) k_trsm_block(const T* __restrict
         if (!unit && i < kb) d = Tm[(int64_t)i * (trs + tcs)];
         divs[i] = Divisor<T>::of(d);
     }
+    // Rows' right-hand sides and, apart from them, the sums of their updates: terms below the rounding of
+    // a right-hand side still count together. The sums start at -0, which leaves every value as it is.
+    T rhs[TRSM_FPW][4];
     typename MM::Acc acc[TRSM_FPW][NP];
 #pragma unroll
     for (int i = 0; i < TRSM_FPW; ++i)
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const int row = 16 * (i * TRSM_NW + wave) + MM::row(k, lane);
-            const T v = row < kb && col < r ? X[(int64_t)row * xrs + col * xcs] : T{};
-            if constexpr (CX) {
-                acc[i][0][k] = v.re;
-                acc[i][NP - 1][k] = v.im;
-            } else {
-                acc[i][0][k] = v;
-            }
+            rhs[i][k] = row < kb && col < r ? X[(int64_t)row * xrs + col * xcs] : T{};
+#pragma unroll
+            for (int p = 0; p < NP; ++p) acc[i][p][k] = -(R)0;
         }
     // T(f, j) of this lane: row n of the fragment, positions 4 q + e of block j
     auto load_t = [&](T (&t)[4], int f, int j) {
@@ -245,16 +244,16 @@ __global__ void __launch_bounds__(64 * TRSM_NW) k_trsm_block(const T* __restrict
             }
         }
     };
-    // substitution of fragment f (this wave's accumulators): x replaces it and goes to xs[f & 1]. Lane
+    // substitution of fragment f (this wave's right-hand sides b0 and update sums a): x goes to xs[f & 1]. Lane
     // (n, q) holds rows MM::row(k, lane) of column n; each quotient is formed in the lanes that hold its
     // row and handed to the column's other lanes by two lane swaps. The divisors and columns of the
     // diagonal block do not depend on x: they are read a step ahead.
-    auto solve = [&](typename MM::Acc (&a)[NP], int f) __attribute__((always_inline)) {
+    auto solve = [&](const T (&b0)[4], const typename MM::Acc (&a)[NP], int f) __attribute__((always_inline)) {
         T b[4], d[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            if constexpr (CX) b[k] = T{a[0][k], a[NP - 1][k]};
-            else b[k] = a[0][k];
+            if constexpr (CX) b[k] = T{b0[k].re + a[0][k], b0[k].im + a[NP - 1][k]};
+            else b[k] = b0[k] + a[0][k];
             d[k] = diag[f][0][MM::row(k, lane)];
         }
         Divisor<T> dv = divs[16 * f];
@@ -300,7 +299,7 @@ __global__ void __launch_bounds__(64 * TRSM_NW) k_trsm_block(const T* __restrict
         diag[e >> 8][e & 15][e >> 4 & 15] = dl[u];
     }
     __syncthreads();  // diagonal blocks and divisors staged
-    if (wave == 0) solve(acc[0], 0);
+    if (wave == 0) solve(rhs[0], acc[0], 0);
     lds_barrier();
     for (int j = 0; j < nf; ++j) {
         // x of block j is in xs[j & 1], T(., j) in t
@@ -312,7 +311,7 @@ __global__ void __launch_bounds__(64 * TRSM_NW) k_trsm_block(const T* __restrict
         for (int i = 0; i < TRSM_FPW; ++i)
             if (i == own) {
                 subtract(acc[i], t[i], x);
-                solve(acc[i], j + 1);
+                solve(rhs[i], acc[i], j + 1);
             }
 #pragma unroll
         for (int i = 0; i < TRSM_FPW; ++i)

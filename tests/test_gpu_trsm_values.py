@@ -46,3 +46,22 @@ def test_unit_diagonal_keeps_non_finite_parts(dev, dt, uplo):
         got = solve(dev, a, b, LEFT, uplo, UNIT)[first]
         for g, w in ((got.real, b0.real), (got.imag, b0.imag)):
             assert np.array_equal(g, w, equal_nan=True), s
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64, np.complex64, np.complex128])
+@pytest.mark.parametrize("uplo", [LOWER, UPPER])
+def test_small_updates_add_up_before_they_are_subtracted(dev, dt, uplo):
+    """240 updates of u / 2 each (u: the unit roundoff) of one row: 1 - u / 2 rounds to 1, their sum
+    120 u is exact, and so is 1 - 120 u."""
+    s, m = 256, 240
+    u = np.finfo(dt).epsneg
+    a = np.eye(s, dtype=dt)
+    b = np.ones((s, 20), dtype=dt)
+    want = b.copy()
+    if uplo == LOWER:
+        a[-1, :m] = u / 2
+        want[-1] = 1 - 120 * u
+    else:
+        a[0, -m:] = u / 2
+        want[0] = 1 - 120 * u
+    assert np.array_equal(solve(dev, a, b, LEFT, uplo, NONUNIT), want)
