@@ -77,41 +77,41 @@ __device__ __forceinline__ T t_mul(T a, T b) {
     else return a * b;
 }
 
-// Quotients by one divisor, rounded as IEEE divisions are and without their setup per quotient: both
-// parts are scaled to [1/2, 1); q = a r (r the rounded reciprocal) is corrected by its exact remainder
-// to a neighbour of the quotient, and once more to the rounded one (Markstein's theorem); the
-// exponents are put back, and v_div_fixup gives zeros, infinities and NaN their IEEE results. A result
-// below the normal range would be rounded a second time there: such lanes divide.
+// Quotients by one divisor, as accurate as divisions and without their setup per quotient, by a
+// reciprocal of twice the precision. exact() divides.
 template <class R>
-struct Recip {
-    R d, m, r;
-    int e;
-    __device__ static R mant(R x) {
-        if constexpr (sizeof(R) == 8) return __builtin_amdgcn_frexp_mant(x);
-        else return __builtin_amdgcn_frexp_mantf(x);
-    }
-    __device__ static int expo(R x) {
-        if constexpr (sizeof(R) == 8) return __builtin_amdgcn_frexp_exp(x);
-        else return __builtin_amdgcn_frexp_expf(x);
-    }
-    __device__ static Recip of(R d) {
-        const R m = mant(d);
-        return {d, m, (R)1 / m, expo(d)};
-    }
-    __device__ __forceinline__ R quot(R a) const {
-        constexpr int LOW = sizeof(R) == 8 ? -1021 : -125;  // frexp exponent of the smallest normal number
-        const R am = mant(a);
-        const int ex = expo(a) - e;
-        R q = am * r;
-        q = fma(fma(-m, q, am), r, q);
-        q = fma(fma(-m, q, am), r, q);
-        q = ldexp(q, ex);
-        if constexpr (sizeof(R) == 8) q = __builtin_amdgcn_div_fixup(q, d, a);
-        else q = __builtin_amdgcn_div_fixupf(q, d, a);
-        if (ex < LOW) q = a / d;  // the quotient's own exponent is ex or ex + 1
-        return q;
-    }
+struct Recip;
+// f32: the f64 product with the f64 reciprocal has an error below 2^-28 f32 ulp, and no quotient of two
+// f32 lies within 2^-25 ulp of the middle of two: rounded as the division, subnormal results too.
+template <>
+struct Recip<float> {
+    double r;
+    float d;
+    __device__ static Recip of(float d) { return {1.0 / d, d}; }
+    __device__ __forceinline__ float quot(float a) const { return (float)(a * r); }
+    __device__ float exact(float a) const { return a / d; }
 };
+// f64: a (r + rl), r + rl = 1 / d to 2^-105, both parts scaled to [1/2, 1): half an ulp and 2^-50 ulp,
+// that is rounded as the division but for quotients that close to the middle of two numbers. The
+// exponents are put back, and v_div_fixup gives zeros, infinities and NaN their IEEE results.
+// Subnormal results are rounded a second time there.
+template <>
+struct Recip<double> {
+    double d, r, rl;
+    int e;
+    __device__ static Recip of(double d) {
+        const double m = __builtin_amdgcn_frexp_mant(d), r = 1 / m;
+        return {d, r, fma(-m, r, 1.0) * r, __builtin_amdgcn_frexp_exp(d)};
+    }
+    __device__ __forceinline__ double quot(double a) const {
+        const double m = __builtin_amdgcn_frexp_mant(a);
+        const double q = fma(m, r, m * rl);
+        return __builtin_amdgcn_div_fixup(ldexp(q, __builtin_amdgcn_frexp_exp(a) - e), d, a);
+    }
+    __device__ double exact(double a) const { return a / d; }
+};
+__device__ __forceinline__ bool subnormal(double x) { return __builtin_amdgcn_class(x, 0x90); }
+__device__ __forceinline__ bool subnormal(c128 x) { return subnormal(x.re) || subnormal(x.im); }
 // The divisor of one row of the solve. Complex: a conj(b) / |b|^2 with b scaled by its larger part
 // (no overflow for moderate b).
 template <class T>
@@ -119,6 +119,7 @@ struct Divisor {
     Recip<T> s;
     __device__ static Divisor of(T b) { return {Recip<T>::of(b)}; }
     __device__ __forceinline__ T quot(T a) const { return s.quot(a); }
+    __device__ T exact(T a) const { return s.exact(a); }
 };
 template <class T, class R>
 struct DivisorC {
@@ -130,6 +131,9 @@ struct DivisorC {
     }
     __device__ __forceinline__ T quot(T a) const {
         return T{s.quot(d.quot(a.re * br + a.im * bi)), s.quot(d.quot(a.im * br - a.re * bi))};
+    }
+    __device__ T exact(T a) const {
+        return T{s.exact(d.exact(a.re * br + a.im * bi)), s.exact(d.exact(a.im * br - a.re * bi))};
     }
 };
 template <>
@@ -181,7 +185,7 @@ constexpr int TRSM_FPW = TRSM_F / TRSM_NW;   // fragments per wave
 // Measured: 256 rows x 1600 columns f64 29-37 us; 2000 rows 0.52 ms in all, eight such launches and
 // the updates between them by the GEMM (3.5 ms with 64-row blocks, one thread per column).
 template <class T>
-__global__ void __launch_bounds__(64 * TRSM_NW) k_trsm_block(const T* __restrict__ Tm, int64_t trs, int64_t tcs, int unit,
+__global__ void __launch_bounds__(64 * TRSM_NW, sizeof(T) == 16 ? 2 : 4) k_trsm_block(const T* __restrict__ Tm, int64_t trs, int64_t tcs, int unit,
                                                             int kb, T* __restrict__ X, int64_t xrs, int64_t xcs,
                                                             int64_t r) {
     using R = typename ElemOf<T>::R;
@@ -210,19 +214,27 @@ __global__ void __launch_bounds__(64 * TRSM_NW) k_trsm_block(const T* __restrict
         if (!unit && i < kb) d = Tm[(int64_t)i * (trs + tcs)];
         divs[i] = Divisor<T>::of(d);
     }
-    // Rows' right-hand sides and, apart from them, the sums of their updates: terms below the rounding of
-    // a right-hand side still count together. The sums start at -0, which leaves every value as it is.
-    T rhs[TRSM_FPW][4];
+    // The right-hand sides of the wave's next fragment to solve and, apart from them, the sums of the
+    // updates: terms below the rounding of a right-hand side still count together. The sums start at
+    // -0, which leaves every value as it is.
+    constexpr bool LATE = sizeof(T) == 16;  // c128: a fragment's right-hand sides come when the one before is solved
+    T rhs[LATE ? 1 : TRSM_FPW][4];
+    auto load_rhs = [&](int i) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int row = 16 * (i * TRSM_NW + wave) + MM::row(k, lane);
+            rhs[LATE ? 0 : i][k] = row < kb && col < r ? X[(int64_t)row * xrs + col * xcs] : T{};
+        }
+    };
+    load_rhs(0);
+    if (!LATE) load_rhs(1);
     typename MM::Acc acc[TRSM_FPW][NP];
 #pragma unroll
     for (int i = 0; i < TRSM_FPW; ++i)
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int row = 16 * (i * TRSM_NW + wave) + MM::row(k, lane);
-            rhs[i][k] = row < kb && col < r ? X[(int64_t)row * xrs + col * xcs] : T{};
+        for (int p = 0; p < NP; ++p)
 #pragma unroll
-            for (int p = 0; p < NP; ++p) acc[i][p][k] = -(R)0;
-        }
+            for (int k = 0; k < 4; ++k) acc[i][p][k] = -(R)0;
     // T(f, j) of this lane: row n of the fragment, positions 4 q + e of block j
     auto load_t = [&](T (&t)[4], int f, int j) {
 #pragma unroll
@@ -244,16 +256,41 @@ __global__ void __launch_bounds__(64 * TRSM_NW) k_trsm_block(const T* __restrict
             }
         }
     };
-    // substitution of fragment f (this wave's right-hand sides b0 and update sums a): x goes to xs[f & 1]. Lane
-    // (n, q) holds rows MM::row(k, lane) of column n; each quotient is formed in the lanes that hold its
-    // row and handed to the column's other lanes by two lane swaps. The divisors and columns of the
-    // diagonal block do not depend on x: they are read a step ahead.
-    auto solve = [&](const T (&b0)[4], const typename MM::Acc (&a)[NP], int f) __attribute__((always_inline)) {
+    // substitution of fragment f (this wave's right-hand sides and update sums a): x goes to xs[f & 1],
+    // which nothing else reads any more. Lane (n, q) holds rows MM::row(k, lane) of column n; each quotient
+    // is formed in the lanes that hold its row and handed to the column's other lanes by two lane swaps.
+    // The divisors and columns of the diagonal block do not depend on x: they are read a step ahead.
+    constexpr bool F64 = sizeof(R) == 8;
+    // the same by divisions, a lane per column, for results below the normal range: xf holds the
+    // right-hand sides less the updates
+    auto divide = [&](T (&xf)[16][16], int f) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (q != 0) return;
+#pragma unroll 1
+        for (int i = 0; i < 16; ++i) {
+            T v = xf[i][n];
+#pragma unroll 1
+            for (int c = 0; c < i; ++c) {
+                const T e = diag[f][c][i], x = xf[c][n];
+                if constexpr (CX) {
+                    v.re = fma(e.im, x.im, fma(-e.re, x.re, v.re));
+                    v.im = fma(-e.im, x.re, fma(-e.re, x.im, v.im));
+                } else {
+                    v = fma(-e, x, v);
+                }
+            }
+            xf[i][n] = divs[16 * f + i].exact(v);
+        }
+    };
+    auto solve = [&](const T (&rf)[4], const typename MM::Acc (&a)[NP], int f) __attribute__((always_inline)) {
+        T(&xf)[16][16] = xs[f & 1];
+        constexpr bool NARROW = std::is_same<T, c64>::value;  // not a step ahead: 128 registers are two blocks per CU
         T b[4], d[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            if constexpr (CX) b[k] = T{b0[k].re + a[0][k], b0[k].im + a[NP - 1][k]};
-            else b[k] = b0[k] + a[0][k];
+            if constexpr (CX) b[k] = T{rf[k].re + a[0][k], rf[k].im + a[NP - 1][k]};
+            else b[k] = rf[k] + a[0][k];
+            if constexpr (F64) xf[MM::row(k, lane)][n] = b[k];
             d[k] = diag[f][0][MM::row(k, lane)];
         }
         Divisor<T> dv = divs[16 * f];
@@ -264,11 +301,12 @@ __global__ void __launch_bounds__(64 * TRSM_NW) k_trsm_block(const T* __restrict
             const Divisor<T> dc = dv;
             T e[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) e[k] = d[k];
+            for (int k = 0; k < 4; ++k) e[k] = NARROW ? diag[f][c][MM::row(k, lane)] : d[k];
             if (c < 15) {
                 dv = divs[16 * f + c + 1];
 #pragma unroll
-                for (int k = 0; k < 4; ++k) d[k] = diag[f][c + 1][MM::row(k, lane)];
+                for (int k = 0; k < 4; ++k)
+                    if (!NARROW) d[k] = diag[f][c + 1][MM::row(k, lane)];
             }
             // no quotient by one: (inf + i nan) / 1 would spread the NaN
             const T xc = unit ? b[k0] : dc.quot(b[k0]);
@@ -287,8 +325,17 @@ __global__ void __launch_bounds__(64 * TRSM_NW) k_trsm_block(const T* __restrict
                 if (MM::row(k, lane) > c) b[k] = v;
             }
         }
+        if constexpr (F64) {
+            bool low = false;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) xs[f & 1][MM::row(k, lane)][n] = b[k];
+            for (int k = 0; k < 4; ++k) low = low || subnormal(b[k]);
+            if (__any(low) && !unit) {
+                divide(xf, f);
+                return;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) xf[MM::row(k, lane)][n] = b[k];
     };
     T t[TRSM_FPW][4];
 #pragma unroll
@@ -299,7 +346,10 @@ __global__ void __launch_bounds__(64 * TRSM_NW) k_trsm_block(const T* __restrict
         diag[e >> 8][e & 15][e >> 4 & 15] = dl[u];
     }
     __syncthreads();  // diagonal blocks and divisors staged
-    if (wave == 0) solve(rhs[0], acc[0], 0);
+    if (wave == 0) {
+        solve(rhs[0], acc[0], 0);
+        if (LATE) load_rhs(1);
+    }
     lds_barrier();
     for (int j = 0; j < nf; ++j) {
         // x of block j is in xs[j & 1], T(., j) in t
@@ -311,7 +361,8 @@ __global__ void __launch_bounds__(64 * TRSM_NW) k_trsm_block(const T* __restrict
         for (int i = 0; i < TRSM_FPW; ++i)
             if (i == own) {
                 subtract(acc[i], t[i], x);
-                solve(rhs[i], acc[i], j + 1);
+                solve(rhs[LATE ? 0 : i], acc[i], j + 1);
+                if (LATE && i + 1 < TRSM_FPW) load_rhs(i + 1);
             }
 #pragma unroll
         for (int i = 0; i < TRSM_FPW; ++i)
