@@ -78,7 +78,7 @@ __device__ __forceinline__ T t_mul(T a, T b) {
 }
 
 // Quotients by one divisor, as accurate as divisions and without their setup per quotient, by a
-// reciprocal of twice the precision. exact() divides.
+// reciprocal of twice the precision. exact() (f64) divides.
 template <class R>
 struct Recip;
 // f32: the f64 product with the f64 reciprocal has an error below 2^-28 f32 ulp, and no quotient of two
@@ -86,10 +86,8 @@ struct Recip;
 template <>
 struct Recip<float> {
     double r;
-    float d;
-    __device__ static Recip of(float d) { return {1.0 / d, d}; }
+    __device__ static Recip of(float d) { return {1.0 / d}; }
     __device__ __forceinline__ float quot(float a) const { return (float)(a * r); }
-    __device__ float exact(float a) const { return a / d; }
 };
 // f64: a (r + rl), r + rl = 1 / d to 2^-105, both parts scaled to [1/2, 1): half an ulp and 2^-50 ulp,
 // that is rounded as the division but for quotients that close to the middle of two numbers. The
@@ -112,6 +110,17 @@ struct Recip<double> {
 };
 __device__ __forceinline__ bool subnormal(double x) { return __builtin_amdgcn_class(x, 0x90); }
 __device__ __forceinline__ bool subnormal(c128 x) { return subnormal(x.re) || subnormal(x.im); }
+// a / b. Complex: as by Divisor below.
+template <class T>
+__device__ __forceinline__ T t_div(T a, T b) {
+    if constexpr (std::is_same<T, c128>::value || std::is_same<T, c64>::value) {
+        const auto m = fmax(fabs(b.re), fabs(b.im));
+        const auto br = b.re / m, bi = b.im / m, d = br * br + bi * bi;
+        return T{(a.re * br + a.im * bi) / d / m, (a.im * br - a.re * bi) / d / m};
+    } else {
+        return a / b;
+    }
+}
 // The divisor of one row of the solve. Complex: a conj(b) / |b|^2 with b scaled by its larger part
 // (no overflow for moderate b).
 template <class T>
@@ -165,6 +174,43 @@ __device__ __forceinline__ T bcast_rows(T v, int g) {
 // Barrier for data that waves exchange through LDS: unlike __syncthreads it leaves global loads and
 // stores in flight.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+constexpr int TRSM_CB = 32;  // rows the column kernel takes at most
+
+// Triangular solve of few rows, arguments as for k_trsm_block: one thread per column of X, 64 per
+// block, T and the columns staged in LDS. Bound by reading and writing X where columns are many; for
+// few columns by its chain, longer per row than k_trsm_block's. That one, eight waves per 16 columns,
+// takes 5 us (f32) to 12 us (c128) per round of blocks however few the rows. So: up to 8 rows always
+// here (no slower at one column), up to 32 from 16 rows CUs bytes of a row of X on, where the others
+// need several rounds (us, f64, k_trsm_block against this: 2 rows x 1000000 382, 7; 8 x 300000 230, 16; 16
+// x 10000 16, 8; 32 x 30000 42, 21; the other way round 16 x 3000 6.3, 8.5; 32 x 10000 16, 19).
+template <class T>
+__global__ void __launch_bounds__(64) k_trsm_cols(const T* __restrict__ Tm, int64_t trs, int64_t tcs, int unit, int kb,
+                                                  T* __restrict__ X, int64_t xrs, int64_t xcs, int64_t r) {
+    __shared__ T ts[TRSM_CB][TRSM_CB + 1];
+    __shared__ T xs[TRSM_CB][64];
+    const int j = threadIdx.x;
+    const int64_t col = (int64_t)blockIdx.x * 64 + j;
+    for (int e = j; e < kb * kb; e += 64) {
+        const int i = e / kb, k = e - i * kb;
+        // only the triangle is read, and a unit diagonal not at all
+        if (k < i || (k == i && !unit)) ts[i][k] = Tm[(int64_t)i * trs + (int64_t)k * tcs];
+    }
+    if (col < r)
+        for (int i = 0; i < kb; ++i) xs[i][j] = X[(int64_t)i * xrs + col * xcs];
+    __syncthreads();
+    if (col >= r) return;
+    for (int i = 0; i < kb; ++i) {
+        T acc = xs[i][j];
+        for (int k = 0; k < i; ++k) {
+            const T p = t_mul(ts[i][k], xs[k][j]);
+            if constexpr (ElemOf<T>::CX) acc = T{acc.re - p.re, acc.im - p.im};
+            else acc = acc - p;
+        }
+        xs[i][j] = unit ? acc : t_div(acc, ts[i][i]);
+    }
+    for (int i = 0; i < kb; ++i) X[(int64_t)i * xrs + col * xcs] = xs[i][j];
+}
 
 constexpr int TRSM_NB = 256;                 // rows solved by one launch
 constexpr int TRSM_F = TRSM_NB / 16;         // 16-row fragments of them
@@ -263,7 +309,7 @@ __global__ void __launch_bounds__(64 * TRSM_NW, sizeof(T) == 16 ? 2 : 4) k_trsm_
     constexpr bool F64 = sizeof(R) == 8;
     // the same by divisions, a lane per column, for results below the normal range: xf holds the
     // right-hand sides less the updates
-    auto divide = [&](T (&xf)[16][16], int f) {
+    auto divide = [&](auto& xf, int f) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (q != 0) return;
 #pragma unroll 1
@@ -642,7 +688,10 @@ static void driver_trsm(rstsr_hip_ctx* ctx, rstsr_dtype_t t, rstsr_gemm_mode_t m
             if (len <= TRSM_NB) {
                 // an upper triangle is a lower one with every row order reversed
                 const int64_t at = lower ? lo : hi - 1, sg = lower ? 1 : -1;
-                hipLaunchKernelGGL(k_trsm_block<T>, dim3((uint32_t)((r + 15) / 16)), dim3(64 * TRSM_NW), 0, ctx->stream,
+                const int64_t cu = std::max(ctx->num_cu, 1);
+                const bool cols = len <= TRSM_CB && (len <= 8 || r * (int64_t)sizeof(T) >= 16 * len * cu);
+                const dim3 grid((uint32_t)(cols ? (r + 63) / 64 : (r + 15) / 16)), blk(cols ? 64 : 64 * TRSM_NW);
+                hipLaunchKernelGGL(cols ? k_trsm_cols<T> : k_trsm_block<T>, grid, blk, 0, ctx->stream,
                                    Tm + at * (trs + tcs), sg * trs, sg * tcs, diag == DIAG_U ? 1 : 0, (int)len,
                                    Y + at * yrs, sg * yrs, ycs, r);
                 check_launch("trsm diagonal block");
