@@ -690,10 +690,15 @@ static void driver_trsm(rstsr_hip_ctx* ctx, rstsr_dtype_t t, rstsr_gemm_mode_t m
                 const int64_t at = lower ? lo : hi - 1, sg = lower ? 1 : -1;
                 const int64_t cu = std::max(ctx->num_cu, 1);
                 const bool cols = len <= TRSM_CB && (len <= 8 || r * (int64_t)sizeof(T) >= 16 * len * cu);
-                const dim3 grid((uint32_t)(cols ? (r + 63) / 64 : (r + 15) / 16)), blk(cols ? 64 : 64 * TRSM_NW);
-                hipLaunchKernelGGL(cols ? k_trsm_cols<T> : k_trsm_block<T>, grid, blk, 0, ctx->stream,
-                                   Tm + at * (trs + tcs), sg * trs, sg * tcs, diag == DIAG_U ? 1 : 0, (int)len,
-                                   Y + at * yrs, sg * yrs, ycs, r);
+                // at most 2^32 - 1 threads per launch
+                const int64_t step = (int64_t)1 << 26;
+                for (int64_t c0 = 0; c0 < r; c0 += step) {
+                    const int64_t rc = std::min(step, r - c0);
+                    const dim3 grid((uint32_t)(cols ? (rc + 63) / 64 : (rc + 15) / 16)), blk(cols ? 64 : 64 * TRSM_NW);
+                    hipLaunchKernelGGL(cols ? k_trsm_cols<T> : k_trsm_block<T>, grid, blk, 0, ctx->stream,
+                                       Tm + at * (trs + tcs), sg * trs, sg * tcs, diag == DIAG_U ? 1 : 0, (int)len,
+                                       Y + at * yrs + c0 * ycs, sg * yrs, ycs, rc);
+                }
                 check_launch("trsm diagonal block");
                 return;
             }

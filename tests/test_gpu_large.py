@@ -54,3 +54,18 @@ def test_reduction_with_2_31_outputs(dev, big):
     assert out.shape == (ROWS * COLS,)
     e = out.reshape([ROWS, COLS]) - a
     assert np.all(e.max_axes([1]).to_numpy() == 0) and np.all(e.min_axes([1]).to_numpy() == 0)
+
+
+def test_solve_with_2_27_columns(dev):
+    """33 rows x (2^27 + 3) right-hand sides of a diagonal solve, more than one launch covers."""
+    import ctypes as C
+
+    from rstsr_amd import abi
+
+    s, r = 33, (1 << 27) + 3
+    a = rt.asarray(np.diag(np.full(s, 2.0, dtype=np.float32)), device=dev)
+    b = rt.full((s, r), 6.0, dtype=np.float32, device=dev)
+    one = np.array(1, dtype=np.float32)
+    abi.check(abi.lib().rstsr_hip_driver_trsm(C.c_void_p(dev._ctx_ptr()), rt._code(np.float32), 0, 101, 141, 122, 111, 131,
+                                              s, r, one.ctypes.data, a.as_ptr(), s, b.as_ptr(), r))
+    assert b.max_all() == 3.0 and b.min_all() == 3.0
