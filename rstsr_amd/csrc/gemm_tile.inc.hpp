@@ -23,7 +23,7 @@ static void tile_gemm_launch(rstsr_hip_ctx* ctx, TileGemmArgs<T> g, uint32_t nb,
     g.tiles_n = ceil_div_u32(g.N, CF::BN);
     uint64_t nt = (uint64_t)g.tiles_m * g.tiles_n;
     if (g.tri) nt = (uint64_t)g.tiles_m * (g.tiles_m + 1) / 2;
-    if (nt >= (1ull << 31)) RSTSR_RAISE(UnImplemented, "GEMM grid too large");
+    if (nt >= (1ull << 31) || nt * CF::NT >= (1ull << 32)) RSTSR_RAISE(UnImplemented, "GEMM grid too large");
     auto go = [&](auto a, auto b) {
         hipLaunchKernelGGL((k_gemm_tile<T, CF, decltype(a)::value, decltype(b)::value, V16, SPLIT>),
                            dim3((uint32_t)nt, nb, nsplit), dim3(CF::NT), 0, ctx->stream, g, run_if);
@@ -175,7 +175,15 @@ static void tile_gemm_run(rstsr_hip_ctx* ctx, const char* tag, const GemmProblem
         check_launch("gemm split");
         return;
     }
+    const int big = tile_shape_index<T>(128), mid = tile_shape_index<T>(64), small = tile_shape_index<T>(32);
+    // a launch holds fewer than 2^32 threads: outputs of 2^34 elements and more only fit the larger tiles
+    const int bms[4] = {S::S0::BM, S::S1::BM, S::S2::BM, S::S3::BM}, nts[4] = {S::S0::NT, S::S1::NT, S::S2::NT, S::S3::NT};
+    auto fits = [&](int c) {
+        const uint64_t bm = (uint64_t)bms[c], tm = (P.M + bm - 1) / bm, tn = (P.N + bm - 1) / bm;
+        return tm * tn * (uint64_t)nts[c] < (1ull << 32);
+    };
     auto run = [&](int c) {
+        if (!fits(c)) c = big;
         for (uint64_t b0 = 0; b0 < P.nbatch; b0 += YMAX) {
             g.batch0 = (uint32_t)b0;
             g.tri = syrk ? 1 : 0;
@@ -193,7 +201,6 @@ static void tile_gemm_run(rstsr_hip_ctx* ctx, const char* tag, const GemmProblem
     // untuned: the largest tile that still gives every CU a block
     const int64_t cu = std::max(ctx->num_cu, 1);
     auto tiles = [&](int64_t s) { return ((P.M + s - 1) / s) * ((P.N + s - 1) / s) * (int64_t)P.nbatch; };
-    const int big = tile_shape_index<T>(128), mid = tile_shape_index<T>(64), small = tile_shape_index<T>(32);
     const int heur = tiles(128) >= cu ? big : (tiles(64) >= cu / 2 ? mid : small);
     auto bkt = [](int64_t x) {
         int b = 0;

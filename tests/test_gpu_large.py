@@ -69,3 +69,23 @@ def test_solve_with_2_27_columns(dev):
     abi.check(abi.lib().rstsr_hip_driver_trsm(C.c_void_p(dev._ctx_ptr()), rt._code(np.float32), 0, 101, 141, 122, 111, 131,
                                               s, r, one.ctypes.data, a.as_ptr(), s, b.as_ptr(), r))
     assert b.max_all() == 3.0 and b.min_all() == 3.0
+
+
+def test_product_with_2_34_outputs(dev):
+    """An f64 outer product of 128 GiB, whose smallest tiles would need more threads than a launch
+    holds: the tuner leaves those out."""
+    n = 1 << 17
+    x = np.arange(n, dtype=np.float64)
+    rt.empty_cache(dev)
+    a, b = rt.asarray(x.reshape(n, 1), device=dev), rt.asarray(x.reshape(1, n), device=dev)
+    try:
+        c = a % b
+    except rt.RSTSRError as e:
+        if e.args[0] != "MemoryError":
+            raise
+        pytest.skip("no 128 GiB for the output")
+    for i in (0, 1, n // 2 + 1, n - 1):
+        assert np.array_equal(c[i].to_numpy(), i * x)
+        assert np.array_equal(c[:, i].to_numpy(), i * x)
+    del c
+    rt.empty_cache(dev)
