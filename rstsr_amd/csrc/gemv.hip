@@ -314,45 +314,54 @@ static void gemv_run(rstsr_hip_ctx* ctx, const GemmProblem& P, T alpha, T beta, 
     const uint32_t nb = (uint32_t)P.nbatch;
     const int64_t cu = std::max(ctx->num_cu, 1);
     const bool row = std::llabs(g.cs) <= std::llabs(g.rs);
-    // waves before splitting k, k positions a split should have at least, blocks along the outputs
+    // waves per row group, outputs per block, k positions a split should have at least
     int wpr = 1, vec = 1;
-    int64_t blocks, least;
+    int64_t per, least;
     if (row) {
         vec = g.cs == 1 ? V16 : 1;
         // four waves per row group until the rows alone give four waves per CU
         wpr = (g.M * nb + GV_RPW - 1) / GV_RPW >= 4 * cu ? 1 : 4;
-        blocks = (g.M + GV_RPW * (4 / wpr) - 1) / (GV_RPW * (4 / wpr));
+        per = GV_RPW * (4 / wpr);
         least = (int64_t)64 * vec * wpr * 4;
     } else {
         vec = g.rs == 1 ? V16 : 1;
-        blocks = (g.M + 64 * vec - 1) / (64 * vec);
+        per = 64 * vec;
         least = 64;
     }
     // eight (row) or sixteen (col: one step per lane in flight instead of four rows) waves per CU
-    const int64_t want = (row ? 2 : 4) * cu, have = blocks * nb;
+    const int64_t want = (row ? 2 : 4) * cu, have = (g.M + per - 1) / per * nb;
     int64_t ns = have >= want ? 1 : std::min<int64_t>((want + have - 1) / have, std::max<int64_t>(1, g.K / least));
     ns = std::min<int64_t>(ns, 1024);
     g.chunk = ((g.K + ns - 1) / ns + vec - 1) / vec * vec;
     g.nsplit = (int)((g.K + g.chunk - 1) / g.chunk);
     g.part = g.nsplit > 1 ? (T*)workspace(ctx, (size_t)nb * g.nsplit * g.M * sizeof(T)) : nullptr;
-    const dim3 grid((uint32_t)blocks, (uint32_t)g.nsplit, nb), blk(256);
-    auto rows = [&](auto v, auto w) {
-        constexpr int V = decltype(v)::value, W = decltype(w)::value;
-        if (g.xs == 1) hipLaunchKernelGGL((k_gemv_row<T, V, W, true>), grid, blk, 0, ctx->stream, g);
-        else hipLaunchKernelGGL((k_gemv_row<T, V, W, false>), grid, blk, 0, ctx->stream, g);
-    };
-    using One = std::integral_constant<int, 1>;
-    using Four = std::integral_constant<int, 4>;
-    using Vec = std::integral_constant<int, V16>;
-    if (row) {
-        if (vec == 1) wpr == 1 ? rows(One{}, One{}) : rows(One{}, Four{});
-        else wpr == 1 ? rows(Vec{}, One{}) : rows(Vec{}, Four{});
-    } else if (vec == 1) {
-        hipLaunchKernelGGL((k_gemv_col<T, 1>), grid, blk, 0, ctx->stream, g);
-    } else {
-        hipLaunchKernelGGL((k_gemv_col<T, V16>), grid, blk, 0, ctx->stream, g);
+    const dim3 blk(256);
+    // a launch holds fewer than 2^32 threads (16 per output at most): more outputs in pieces
+    constexpr int64_t PIECE = (int64_t)1 << 27;
+    for (int64_t i = 0; i < g.M; i += PIECE) {
+        GemvArgs<T> q = g;
+        q.M = std::min(PIECE, g.M - i);  // all of them where k is split
+        q.a += i * g.rs;
+        q.y += i * g.ys;
+        const dim3 grid((uint32_t)((q.M + per - 1) / per), (uint32_t)g.nsplit, nb);
+        auto rows = [&](auto v, auto w) {
+            constexpr int V = decltype(v)::value, W = decltype(w)::value;
+            if (g.xs == 1) hipLaunchKernelGGL((k_gemv_row<T, V, W, true>), grid, blk, 0, ctx->stream, q);
+            else hipLaunchKernelGGL((k_gemv_row<T, V, W, false>), grid, blk, 0, ctx->stream, q);
+        };
+        using One = std::integral_constant<int, 1>;
+        using Four = std::integral_constant<int, 4>;
+        using Vec = std::integral_constant<int, V16>;
+        if (row) {
+            if (vec == 1) wpr == 1 ? rows(One{}, One{}) : rows(One{}, Four{});
+            else wpr == 1 ? rows(Vec{}, One{}) : rows(Vec{}, Four{});
+        } else if (vec == 1) {
+            hipLaunchKernelGGL((k_gemv_col<T, 1>), grid, blk, 0, ctx->stream, q);
+        } else {
+            hipLaunchKernelGGL((k_gemv_col<T, V16>), grid, blk, 0, ctx->stream, q);
+        }
+        check_launch("gemv");
     }
-    check_launch("gemv");
     if (g.nsplit > 1) {
         if (g.nsplit >= 16 && g.M * nb <= 4096)
             hipLaunchKernelGGL(k_gemv_fin_wave<T>, dim3(ceil_div_u32((uint64_t)g.M, 4), 1, nb), blk, 0, ctx->stream, g);

@@ -86,6 +86,17 @@ def test_product_with_2_34_outputs(dev):
         pytest.skip("no 128 GiB for the output")
     for i in (0, 1, n // 2 + 1, n - 1):
         assert np.array_equal(c[i].to_numpy(), i * x)
-        assert np.array_equal(c[:, i].to_numpy(), i * x)
+        assert np.array_equal(c[:, i].to_contig().to_numpy(), i * x)
     del c
     rt.empty_cache(dev)
+
+
+def test_matrix_vector_product_with_2_28_rows(dev):
+    """[2^28 + 5, 1] @ [1], row by row and (a vector of the matrix's rows) as columns: more rows than
+    one launch covers."""
+    m = (1 << 28) + 5
+    a = rt.full((m, 1), 3.0, dtype=np.float32, device=dev)
+    x = rt.asarray(np.array([7.0], dtype=np.float32), device=dev)
+    for mat in (a, a.reshape([1, m]).transpose()):
+        y = mat % x
+        assert y.shape == (m,) and y.max_all() == 21.0 and y.min_all() == 21.0
