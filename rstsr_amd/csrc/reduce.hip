@@ -22,7 +22,7 @@
 //    stride a unit-stride reduced axis with 16-byte loads, group shuffles combine;
 //  - col: lanes along the outputs on the input's unit-stride kept axis
 //    (coalesced), sequential over a part of the reduced range; few parts are the
-//    waves of one block, many the blocks along grid y;
+//    waves of one block, many lie one after the other over the threads;
 //  - finalize: combine the split partials of each output in fixed order.
 // Built with -ffp-contract=off so that TwoSum is not fused or reassociated.
 #include <array>
@@ -532,10 +532,10 @@ __global__ void __launch_bounds__(RB) k_red_row(const T* __restrict__ a, typenam
 }
 
 // VEC adjacent outputs per thread along the unit-stride kept axis, sequential over a part of the
-// reduced range. KS = 1: four waves side by side, parts along blockIdx.y, partials combined by
-// k_red_fin. KS = 16: the waves of a block share its 64 VEC outputs, a part each, combined in order
-// through LDS, so that a reduction with few parts needs no second launch ([64, 128, 256] f64 over
-// axis 1: 16.2 -> 7.7 us in all; for many parts splitting inside the block measured 2 % slower).
+// reduced range. KS = 1: parts one after the other over the threads, partials combined by k_red_fin.
+// KS = 16: the waves of a block share its 64 VEC outputs, a part each, combined in order through LDS, so
+// that a reduction with few parts needs no second launch ([64, 128, 256] f64 over axis 1: 16.2 -> 7.7 us
+// in all; which numbers of parts: reduce_plan).
 template <class A, class T, int VEC, int KS>
 __global__ void __launch_bounds__(KS == 1 ? RB : 64 * KS) k_red_col(const T* __restrict__ a, typename A::Out* out,
                                                 typename A::S* part, RedPlan p) {
@@ -544,10 +544,13 @@ __global__ void __launch_bounds__(KS == 1 ? RB : 64 * KS) k_red_col(const T* __r
     constexpr int COLU = col_unroll((int)(sizeof(T) * VEC));
     __shared__ S red[KS > 1 ? KS : 1][KS > 1 ? 64 * VEC : 1];
     const uint32_t lane = threadIdx.x & 63, wave = KS > 1 ? threadIdx.x >> 6 : 0;
-    const uint64_t mv = KS > 1 ? (uint64_t)blockIdx.x * 64 + lane : (uint64_t)blockIdx.x * RB + threadIdx.x;
-    const uint32_t sp = blockIdx.y;
-    const bool active = mv < p.M / VEC;
-    const uint32_t o = active ? (uint32_t)mv * VEC : 0;
+    const uint32_t nv = p.M / VEC;
+    // KS = 1: the parts' outputs side by side, so that few of them leave no lanes idle
+    const uint64_t t = KS > 1 ? (uint64_t)blockIdx.x * 64 + lane : (uint64_t)blockIdx.x * RB + threadIdx.x;
+    const uint32_t sp = KS > 1 ? 0 : (uint32_t)(t / nv);
+    const bool active = KS > 1 ? t < nv : sp < p.nsplit;
+    if (KS == 1 && !active) return;
+    const uint32_t o = active ? (uint32_t)(t - (uint64_t)sp * nv) * VEC : 0;
     int64_t oin, oout;
     kept_offsets(p, o, oin, oout);
     S acc[VEC];
@@ -849,9 +852,13 @@ static RedSetup reduce_plan(rstsr_hip_ctx* ctx, const Layout& la, const std::vec
         const uint64_t vec = (uint64_t)col_vec(t);
         const uint64_t wpc = (uint64_t)col_waves_per_cu((int)(esize * vec));
         uint64_t want = std::max<uint64_t>(1, ((uint64_t)std::max(ctx->num_cu, 1) * wpc * 64 * vec) / M);
-        // two to sixteen parts of at least four positions: the waves of one block
-        p.ks = want > 1 && want <= 16 && R >= 64 ? 16 : 1;
-        uint64_t nsplit = p.ks > 1 ? 1 : std::min<uint64_t>({want, std::max<uint64_t>(1, R / 64), 65535});
+        uint64_t nsplit = std::min<uint64_t>({want, std::max<uint64_t>(1, R / 64), 65536});
+        // Two to six parts: the waves of one block, which saves the second launch. With more parts
+        // the outputs are too few blocks to read at full rate (us, parts as blocks against waves of one:
+        // f64 128 x 16384 16, 6; 1000 x 32768 53, 44; but 1000 x 5000, 15 parts, 17, 26; c64 3000 x
+        // 8192, 8 parts, 43, 48).
+        p.ks = nsplit > 1 && nsplit <= 6 ? 16 : 1;
+        if (p.ks > 1) nsplit = 1;
         p.upw = (R + nsplit * p.ks - 1) / (nsplit * p.ks);
         nsplit = (R + p.upw * p.ks - 1) / (p.upw * p.ks);
         p.nsplit = (uint32_t)nsplit;
@@ -911,7 +918,8 @@ static void run_reduce(rstsr_hip_ctx* ctx, const RedSetup& s, const T* a, typena
         const bool vec = VC > 1 && p.nk >= 1 && p.kin[0] == 1 && p.kshape[0] % VC == 0 && p.M % VC == 0;
         auto go = [&](auto v, auto ks) {
             constexpr int V = decltype(v)::value, KS = decltype(ks)::value;
-            hipLaunchKernelGGL((k_red_col<A, T, V, KS>), dim3(ceil_div_u32(p.M / V, KS == 1 ? RB : 64), p.nsplit),
+            hipLaunchKernelGGL((k_red_col<A, T, V, KS>),
+                               dim3(KS == 1 ? ceil_div_u32((uint64_t)(p.M / V) * p.nsplit, RB) : ceil_div_u32(p.M / V, 64)),
                                dim3(KS == 1 ? RB : 64 * KS), 0, ctx->stream, a, out, part, p);
         };
         auto by_ks = [&](auto v) {

@@ -74,3 +74,15 @@ def test_nan(dev, rows, cols):
     for axis in (0, 1):
         got = rt.asarray(x, device=dev).sum_axes([axis]).to_numpy()
         assert np.array_equal(got, x.sum(axis=axis), equal_nan=True)
+
+
+@pytest.mark.parametrize("dt", DTYPES[:4])
+@pytest.mark.parametrize("rows,cols", [(20001, 33), (9000, 40), (127, 16384), (129, 16383), (450, 16386), (1000, 5001)])
+def test_column_parts_side_by_side(dev, dt, rows, cols):
+    """Few outputs with many parts, one part, two to six in one block, and more than six."""
+    rng = np.random.default_rng(rows + cols)
+    x = ints(rng, (rows, cols), dt)
+    for t in (inside(dev, x, 1), mid(dev, x)):
+        assert np.array_equal(t.sum_axes([0]).to_numpy(), x.sum(axis=0, dtype=x.dtype))
+        if np.dtype(dt).kind != "c":
+            assert np.array_equal(t.argmax_axes([0]).to_numpy(), x.argmax(axis=0))
