@@ -368,6 +368,7 @@ struct RedPlan {
     // row kernel segmentation of the reduced space: units = rows(rest) x nseg0
     uint32_t seg0 = 1, nseg0 = 1;
     uint64_t units = 1, upw = 1;  // units per split
+    int g = 64;                   // row kernel: lanes per group
     int ks = 1;                   // column kernel: waves per block that share the reduced range
     int stream = 0;               // every input element is read once: streaming loads
 };
@@ -836,9 +837,13 @@ static RedSetup reduce_plan(rstsr_hip_ctx* ctx, const Layout& la, const std::vec
         p.seg0 = std::min<uint32_t>(L0, 8192);
         p.nseg0 = (L0 + p.seg0 - 1) / p.seg0;
         p.units = (R / L0) * p.nseg0;
-        uint64_t want = std::max<uint64_t>(1, target_waves / M);
+        // short rows: 16 lanes each, unless that leaves the chip short of waves
+        const uint64_t v16 = p.rin[0] == 1 && col_vec(t) == 2 ? 16 / esize : 1;
+        const bool brief = L0 / v16 < 128;
+        uint64_t want = std::max<uint64_t>(1, (brief ? 4 : 1) * target_waves / M);
         uint64_t nsplit = std::min<uint64_t>(want, p.units);
         nsplit = std::min<uint64_t>(nsplit, 65536);
+        if (brief && M * nsplit >= target_waves) p.g = 16;
         p.upw = (p.units + nsplit - 1) / nsplit;
         nsplit = (p.units + p.upw - 1) / p.upw;
         p.nsplit = (uint32_t)nsplit;
@@ -902,10 +907,8 @@ static void run_reduce(rstsr_hip_ctx* ctx, const RedSetup& s, const T* a, typena
             hipLaunchKernelGGL((k_red_row<A, T, V, G>), dim3(ceil_div_u32(ngroups, RB / G)), dim3(RB), 0, ctx->stream, a,
                                out, part, p);
         };
-        // short rows: 16 lanes each, unless that leaves the chip short of waves
         auto by_group = [&](auto vec) {
-            const uint64_t packs = p.rshape[0] / decltype(vec)::value, full = (uint64_t)std::max(ctx->num_cu, 1) * 8;
-            if (packs < 128 && ngroups * 16 >= full * 64) go(vec, std::integral_constant<int, 16>{});
+            if (p.g == 16) go(vec, std::integral_constant<int, 16>{});
             else go(vec, std::integral_constant<int, 64>{});
         };
         // whole 16-byte packs along the row (any alignment)
