@@ -843,7 +843,7 @@ static RedSetup reduce_plan(rstsr_hip_ctx* ctx, const Layout& la, const std::vec
         uint64_t want = std::max<uint64_t>(1, (brief ? 4 : 1) * target_waves / M);
         uint64_t nsplit = std::min<uint64_t>(want, p.units);
         nsplit = std::min<uint64_t>(nsplit, 65536);
-        if (brief && M * nsplit >= target_waves) p.g = 16;
+        if ((brief && M * nsplit >= target_waves) || M * nsplit >= (1ull << 26)) p.g = 16;  // at most 2^32 threads
         p.upw = (p.units + nsplit - 1) / nsplit;
         nsplit = (p.units + p.upw - 1) / p.upw;
         p.nsplit = (uint32_t)nsplit;
@@ -1121,9 +1121,10 @@ static void reduce_axes_impl(rstsr_hip_ctx* ctx, rstsr_redop_t op, rstsr_dtype_t
             RSTSR_RAISE(InvalidValue, "zero-size array is not supported for max/min");
         RSTSR_RAISE(InvalidLayout, "empty sequence is not allowed for reduce_arg.");
     }
-    // Launches address at most 2^31 - 1 outputs: 2^31 or more are reduced in pieces of the
-    // largest kept axis (2^30 positions each), input and output views narrowed alike.
-    if (lo.size() >= (1ull << 31)) {
+    // A launch holds fewer than 2^32 threads, of which an output takes up to 16: 2^28 outputs and more
+    // are reduced in pieces of at most 2^27 along the largest kept axis (a piece of one position along
+    // it that is still too large: along the next), input and output views narrowed alike.
+    if (lo.size() >= (1ull << 28)) {
         auto ax = normalize_axes_index(axes, la.ndim(), false);
         std::vector<size_t> kept;
         for (size_t i = 0; i < la.ndim(); ++i)
@@ -1132,7 +1133,7 @@ static void reduce_axes_impl(rstsr_hip_ctx* ctx, rstsr_redop_t op, rstsr_dtype_t
         for (size_t q = 1; q < kept.size(); ++q)
             if (la.shape[kept[q]] > la.shape[kept[j]]) j = q;
         const size_t ia = kept[j];
-        const uint64_t n = la.shape[ia], step = 1ull << 30;
+        const uint64_t n = la.shape[ia], step = std::max<uint64_t>(1, (1ull << 27) / (lo.size() / n));
         for (uint64_t s0 = 0; s0 < n; s0 += step) {
             const uint64_t cnt = std::min(step, n - s0);
             Layout la2 = la, lo2 = lo;

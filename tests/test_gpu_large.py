@@ -100,3 +100,18 @@ def test_matrix_vector_product_with_2_28_rows(dev):
     for mat in (a, a.reshape([1, m]).transpose()):
         y = mat % x
         assert y.shape == (m,) and y.max_all() == 21.0 and y.min_all() == 21.0
+
+
+def test_reductions_with_many_outputs(dev):
+    """2^26 + 1 rows of 512 (a wave per row would be 2^32 threads), and 46341^2 > 2^31 outputs none of
+    whose axes is long."""
+    row = np.arange(512, dtype=np.float32)
+    rows = (1 << 26) + 1
+    t = rt.asarray(row.reshape(1, 512), device=dev).broadcast_to([rows, 512])
+    s = t.sum_axes([1])
+    assert s.shape == (rows,) and s.max_all() == row.sum() and s.min_all() == row.sum()
+    n = 46341
+    pairs = np.arange(2 * n, dtype=np.float32).reshape(1, n, 2)
+    s = rt.asarray(pairs, device=dev).broadcast_to([n, n, 2]).sum_axes([2])
+    e = s - rt.asarray(pairs.sum(axis=2), device=dev)
+    assert s.shape == (n, n) and e.max_all() == 0 and e.min_all() == 0
