@@ -63,6 +63,8 @@ __device__ __forceinline__ T g_add(T a, T b) {
 }
 __device__ __forceinline__ c64 g_mul(c64 a, c64 b) { return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re}; }
 __device__ __forceinline__ c64 g_add(c64 a, c64 b) { return {a.re + b.re, a.im + b.im}; }
+__device__ __forceinline__ c128 g_mul(c128 a, c128 b) { return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re}; }
+__device__ __forceinline__ c128 g_add(c128 a, c128 b) { return {a.re + b.re, a.im + b.im}; }
 
 template <class T>
 __global__ void __launch_bounds__(256) k_gemm_simt(GemmArgs<T> g) {
@@ -98,26 +100,45 @@ __global__ void __launch_bounds__(256) k_gemm_simt(GemmArgs<T> g) {
 
 /* ---------------- host side ---------------- */
 
+// The SIMT kernel: one output per thread, in pieces along the rows where a launch would hold more
+// than 2^32 threads.
 template <class T>
-static void launch_gemm_t(rstsr_hip_ctx* ctx, const GemmProblem& P, T alpha, T beta, bool beta_zero,
-                          const int* run_if = nullptr) {
+static void simt_gemm(rstsr_hip_ctx* ctx, const GemmProblem& P, T alpha, T beta, bool beta_zero) {
     GemmArgs<T> g;
-    g.M = P.M;
     g.N = P.N;
     g.K = P.K;
-    g.a = (const T*)P.a;
     g.rsa = P.rsa;
     g.csa = P.csa;
     g.b = (const T*)P.b;
     g.rsb = P.rsb;
     g.csb = P.csb;
-    g.c = (T*)P.c;
     g.rsc = P.rsc;
     g.csc = P.csc;
     g.alpha = alpha;
     g.beta = beta;
     g.beta_zero = beta_zero ? 1 : 0;
     g.bd = P.bd;
+    g.tiles_n = ceil_div_u32(P.N, 16);
+    const uint64_t YMAX = 65535, TMAX = (1ull << 24) - 1;
+    if (g.tiles_n > TMAX) RSTSR_RAISE(UnImplemented, "GEMM grid too large");
+    const int64_t step = (int64_t)(TMAX / g.tiles_n) * 16;
+    for (int64_t m0 = 0; m0 < P.M; m0 += step) {
+        g.M = std::min(step, P.M - m0);
+        g.a = (const T*)P.a + m0 * P.rsa;
+        g.c = (T*)P.c + m0 * P.rsc;
+        g.tiles_m = ceil_div_u32(g.M, 16);
+        for (uint64_t b0 = 0; b0 < P.nbatch; b0 += YMAX) {
+            g.batch0 = (uint32_t)b0;
+            const uint32_t nb = (uint32_t)std::min<uint64_t>(YMAX, P.nbatch - b0);
+            hipLaunchKernelGGL(k_gemm_simt<T>, dim3(g.tiles_m * g.tiles_n, nb), dim3(256), 0, ctx->stream, g);
+            check_launch("gemm");
+        }
+    }
+}
+
+template <class T>
+static void launch_gemm_t(rstsr_hip_ctx* ctx, const GemmProblem& P, T alpha, T beta, bool beta_zero,
+                          const int* run_if = nullptr) {
     if constexpr (!std::is_integral<T>::value) {
         // SYRK shortcut (device_faer/matmul.rs:38-48): beta = 0 and A is B's transpose
         // in the same buffer, so C is symmetric. Only the tiles on and below the
@@ -130,17 +151,7 @@ static void launch_gemm_t(rstsr_hip_ctx* ctx, const GemmProblem& P, T alpha, T b
         else if constexpr (std::is_same<T, double>::value) tile_gemm_f64(ctx, P, alpha, beta, beta_zero, run_if);
         else tile_gemm_c128(ctx, P, alpha, beta, beta_zero, run_if);
     } else {
-        const uint64_t YMAX = 65535;
-        for (uint64_t b0 = 0; b0 < P.nbatch; b0 += YMAX) {
-            uint32_t nb = (uint32_t)std::min<uint64_t>(YMAX, P.nbatch - b0);
-            g.batch0 = (uint32_t)b0;
-            g.tiles_m = ceil_div_u32(P.M, 16);
-            g.tiles_n = ceil_div_u32(P.N, 16);
-            uint64_t nt = (uint64_t)g.tiles_m * g.tiles_n;
-            if (nt >= (1ull << 31)) RSTSR_RAISE(UnImplemented, "GEMM grid too large");
-            hipLaunchKernelGGL(k_gemm_simt<T>, dim3((uint32_t)nt, nb), dim3(256), 0, ctx->stream, g);
-            check_launch("gemm");
-        }
+        simt_gemm(ctx, P, alpha, beta, beta_zero);
     }
 }
 
@@ -162,7 +173,6 @@ __global__ void k_scale_c(GemmArgs<T> g) {
     T* cp = g.c + oc + m * g.rsc + n * g.csc;
     *cp = g.beta_zero ? T{} : g_mul(g.beta, *cp);
 }
-__device__ __forceinline__ c128 g_mul(c128 a, c128 b) { return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re}; }
 
 template <class T>
 static void scale_c(rstsr_hip_ctx* ctx, const GemmProblem& P, T beta, bool beta_zero) {

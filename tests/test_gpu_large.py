@@ -115,3 +115,13 @@ def test_reductions_with_many_outputs(dev):
     s = rt.asarray(pairs, device=dev).broadcast_to([n, n, 2]).sum_axes([2])
     e = s - rt.asarray(pairs.sum(axis=2), device=dev)
     assert s.shape == (n, n) and e.max_all() == 0 and e.min_all() == 0
+
+
+def test_integer_product_with_2_32_outputs(dev):
+    """An i32 outer product of 2^32 + 2^16 outputs, a thread each."""
+    m, n = (1 << 16) + 1, 1 << 16
+    a = rt.asarray(np.arange(m, dtype=np.int32).reshape(m, 1), device=dev)
+    b = rt.asarray((np.arange(n, dtype=np.int32) % 1000).reshape(1, n), device=dev)
+    c = a % b
+    for i in (0, 1, m // 2, m - 1):
+        assert np.array_equal(c[i].to_numpy(), i * (np.arange(n, dtype=np.int32) % 1000))
