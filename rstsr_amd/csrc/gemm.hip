@@ -1,6 +1,6 @@
 // GEMM on gfx950: the matmul entry point with rstsr's batch-broadcast rules, the dispatch to the
 // matrix-core tile kernel (gemm_tile.hpp: f32, f64, c64, c128) or the split GEMM (ozaki.hip), and
-// a SIMT kernel for integers.
+// a SIMT kernel for integers and for short products.
 //
 // Replaces DeviceMatMulAPI for DeviceFaer (rstsr-core/src/device_faer/matmul.rs:
 // 19-239 -> faer) and the naive kernels of rstsr-native-impl/src/cpu_serial/
@@ -41,7 +41,7 @@ struct GemmArgs {
     BatchDesc bd;
 };
 
-/* ---------------- SIMT kernel: i32, i64 ---------------- */
+/* ---------------- SIMT kernel: i32, i64, short products ---------------- */
 
 template <class T>
 __device__ __forceinline__ T g_mul(T a, T b) {
@@ -136,10 +136,25 @@ static void simt_gemm(rstsr_hip_ctx* ctx, const GemmProblem& P, T alpha, T beta,
     }
 }
 
+// Short products with few rows or columns leave most of a matrix-core tile and of its 128-byte K
+// slice empty. By sizes only, like the tile kernel's own choices (us, tile against SIMT: 10000 products of 4 x 4
+// x 4 f32 31, 9, f64 29, 12, c128 34, 15, of 16 x 16 x 16 f64 33, 16; 200000 x 5 x 5 f32 23, 10, f64 23, 15; f32
+// 5000 x 200 x 2 7.2, 5.4; but 200000 x 20 x 20 f32 18, 33, f64 24, 52; f32 1500 x 1500 x 4 8.0, 9.4). Complex
+// symmetric products stay with the tile kernel, which makes them exactly symmetric.
+template <class T>
+static bool simt_pays(const GemmProblem& P) {
+    constexpr bool CX = std::is_same<T, c64>::value || std::is_same<T, c128>::value;
+    return P.K <= 16 && std::min(P.M, P.N) <= (sizeof(T) == 4 ? 256 : 16) && !(CX && P.a == P.b);
+}
+
 template <class T>
 static void launch_gemm_t(rstsr_hip_ctx* ctx, const GemmProblem& P, T alpha, T beta, bool beta_zero,
                           const int* run_if = nullptr) {
     if constexpr (!std::is_integral<T>::value) {
+        if (!run_if && simt_pays<T>(P)) {
+            simt_gemm(ctx, P, alpha, beta, beta_zero);
+            return;
+        }
         // SYRK shortcut (device_faer/matmul.rs:38-48): beta = 0 and A is B's transpose
         // in the same buffer, so C is symmetric. Only the tiles on and below the
         // diagonal are multiplied, and stored twice. For real types C[i][j] and
