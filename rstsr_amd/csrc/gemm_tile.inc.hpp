@@ -12,9 +12,10 @@ namespace rstsr {
 namespace hip {
 
 // 64 x 64 tiles: K splits, and operands read by words (whose loads leave the registers of larger
-// tiles no room)
+// tiles no room); 32 x 32 ones for the latter where 64 x 64 leave most of the chip idle
 template <class T>
 using TileMid = TCfg<2, 2, 2, 2, 4, 2, !std::is_same<T, double>::value>;
+using TileLow = TCfg<2, 2, 1, 1, 2, 6, false>;
 
 template <class T, class CF, bool V16, bool SPLIT>
 static void tile_gemm_launch(rstsr_hip_ctx* ctx, TileGemmArgs<T> g, uint32_t nb, uint32_t nsplit, bool ak, bool bk,
@@ -191,7 +192,8 @@ static void tile_gemm_run(rstsr_hip_ctx* ctx, const char* tag, const GemmProblem
             auto go = [&](auto cf) {
                 tile_gemm_launch<T, decltype(cf), true, false>(ctx, g, nb, 1, ak, bk, run_if);
             };
-            if (!v16) tile_gemm_launch<T, TileMid<T>, false, false>(ctx, g, nb, 1, ak, bk, run_if);
+            if (!v16 && c == small) tile_gemm_launch<T, TileLow, false, false>(ctx, g, nb, 1, ak, bk, run_if);
+            else if (!v16) tile_gemm_launch<T, TileMid<T>, false, false>(ctx, g, nb, 1, ak, bk, run_if);
             else if (c == 0) go(typename S::S0{});
             else if (c == 1) go(typename S::S1{});
             else if (c == 2) go(typename S::S2{});
