@@ -174,7 +174,17 @@ __global__ void __launch_bounds__(256) k_gemv_row(GemvArgs<T> g) {
                     acc[r] = gv_fma(a1[r].v[v], x1.v[v], acc[r]);
                 }
         }
-        for (; k < k1; k += W) {
+        for (; k + VEC <= k1; k += W) {
+            GvPack<T, VEC> a0[GV_RPW];
+#pragma unroll
+            for (int r = 0; r < GV_RPW; ++r) a0[r] = gv_load<T, VEC, true>(row[r] + k * g.cs);
+            const GvPack<T, VEC> x0 = load_x(k);
+#pragma unroll
+            for (int r = 0; r < GV_RPW; ++r)
+#pragma unroll
+                for (int v = 0; v < VEC; ++v) acc[r] = gv_fma(a0[r].v[v], x0.v[v], acc[r]);
+        }
+        if (VEC > 1 && k < k1) {
 #pragma unroll
             for (int v = 0; v < VEC; ++v)
                 if (k + v < k1) {
