@@ -323,7 +323,8 @@ static void gemv_run(rstsr_hip_ctx* ctx, const GemmProblem& P, T alpha, T beta, 
     constexpr int V16 = sizeof(T) >= 16 ? 1 : 16 / (int)sizeof(T);
     const uint32_t nb = (uint32_t)P.nbatch;
     const int64_t cu = std::max(ctx->num_cu, 1);
-    const bool row = std::llabs(g.cs) <= std::llabs(g.rs);
+    // one output (a dot product) leaves the column kernel one lane
+    const bool row = g.M == 1 || std::llabs(g.cs) <= std::llabs(g.rs);
     // waves per row group, outputs per block, k positions a split should have at least
     int wpr = 1, vec = 1;
     int64_t per, least;
