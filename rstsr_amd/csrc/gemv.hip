@@ -7,7 +7,8 @@
 //   k_gemv_row: lanes along k, four rows per wave share each load of x;
 //   k_gemv_col: lanes along i, four waves of a block take a quarter of the k range each.
 // Where the outputs alone give too few waves, k is split over blocks and k_gemv_fin adds the
-// partial sums in order. Splits follow from the sizes only.
+// partial sums in order. Kernel and splits follow from the sizes, A's layout and the number of CUs, so
+// a product in another layout may round differently.
 // Measured: f64 8000 x 8000 79 us row-major (6.5 TB/s), 86 us column-major; 528 us on a tile kernel.
 #include <type_traits>
 
@@ -128,7 +129,7 @@ constexpr int GV_RPW = 4;  // rows per wave: four rows' loads share one load of 
 
 // WPR waves (of a block of four) share each group of four rows, k interleaved between them.
 // XU: x has unit stride. VEC > 1: A has unit stride along k.
-template <class T, int VEC, int WPR, bool XU>
+template <class T, int VEC, int WPR, bool XU, bool NT>
 __global__ void __launch_bounds__(256) k_gemv_row(GemvArgs<T> g) {
     constexpr int G = 4 / WPR;  // row groups per block
     constexpr int64_t W = 64 * VEC * WPR;
@@ -162,8 +163,8 @@ __global__ void __launch_bounds__(256) k_gemv_row(GemvArgs<T> g) {
             GvPack<T, VEC> a0[GV_RPW], a1[GV_RPW];
 #pragma unroll
             for (int r = 0; r < GV_RPW; ++r) {
-                a0[r] = gv_load<T, VEC, true>(row[r] + k * g.cs);
-                a1[r] = gv_load<T, VEC, true>(row[r] + (k + W) * g.cs);
+                a0[r] = gv_load<T, VEC, NT>(row[r] + k * g.cs);
+                a1[r] = gv_load<T, VEC, NT>(row[r] + (k + W) * g.cs);
             }
             const GvPack<T, VEC> x0 = load_x(k), x1 = load_x(k + W);
 #pragma unroll
@@ -177,7 +178,7 @@ __global__ void __launch_bounds__(256) k_gemv_row(GemvArgs<T> g) {
         for (; k + VEC <= k1; k += W) {
             GvPack<T, VEC> a0[GV_RPW];
 #pragma unroll
-            for (int r = 0; r < GV_RPW; ++r) a0[r] = gv_load<T, VEC, true>(row[r] + k * g.cs);
+            for (int r = 0; r < GV_RPW; ++r) a0[r] = gv_load<T, VEC, NT>(row[r] + k * g.cs);
             const GvPack<T, VEC> x0 = load_x(k);
 #pragma unroll
             for (int r = 0; r < GV_RPW; ++r)
@@ -217,7 +218,7 @@ __global__ void __launch_bounds__(256) k_gemv_row(GemvArgs<T> g) {
 
 // Lane l of every wave owns outputs i0 + l VEC .. + VEC - 1; the block's four waves take a quarter of
 // its k range each. VEC > 1: A has unit stride along i.
-template <class T, int VEC>
+template <class T, int VEC, bool NT>
 __global__ void __launch_bounds__(256) k_gemv_col(GemvArgs<T> g) {
     constexpr int U = 8;
     __shared__ T red[4][64 * VEC];
@@ -239,7 +240,7 @@ __global__ void __launch_bounds__(256) k_gemv_col(GemvArgs<T> g) {
             T xv[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                a[u] = gv_load<T, VEC, true>(p + (k + u) * g.cs);
+                a[u] = gv_load<T, VEC, NT>(p + (k + u) * g.cs);
                 xv[u] = x[(k + u) * g.xs];
             }
 #pragma unroll
@@ -248,7 +249,7 @@ __global__ void __launch_bounds__(256) k_gemv_col(GemvArgs<T> g) {
                 for (int v = 0; v < VEC; ++v) acc[v] = gv_fma(a[u].v[v], xv[u], acc[v]);
         }
         for (; k < k1; ++k) {
-            const GvPack<T, VEC> a = gv_load<T, VEC, true>(p + k * g.cs);
+            const GvPack<T, VEC> a = gv_load<T, VEC, NT>(p + k * g.cs);
             const T xv = x[k * g.xs];
 #pragma unroll
             for (int v = 0; v < VEC; ++v) acc[v] = gv_fma(a.v[v], xv, acc[v]);
@@ -347,6 +348,14 @@ static void gemv_run(rstsr_hip_ctx* ctx, const GemmProblem& P, T alpha, T beta, 
     g.nsplit = (int)((g.K + g.chunk - 1) / g.chunk);
     g.part = g.nsplit > 1 ? (T*)workspace(ctx, (size_t)nb * g.nsplit * g.M * sizeof(T)) : nullptr;
     const dim3 blk(256);
+    using One = std::integral_constant<int, 1>;
+    using Four = std::integral_constant<int, 4>;
+    using Vec = std::integral_constant<int, V16>;
+    // Streaming loads of A, which leave nothing in the last-level cache, unless A is small or shared by
+    // batches (us, with and without: the same 32 MB f32 matrix again 6.8, 5.1, many in turn 7.6, 8.0; 200
+    // MB f64 37, 32 and 38, 41; 512 MB 80, 91).
+    bool once = (uint64_t)g.M * g.K * nb * sizeof(T) >= (40ull << 20);
+    for (int d = 0; d < g.bd.nbd; ++d) once = once && g.bd.sa[d] != 0;
     // a launch holds fewer than 2^32 threads (16 per output at most): more outputs in pieces
     constexpr int64_t PIECE = (int64_t)1 << 27;
     for (int64_t i = 0; i < g.M; i += PIECE) {
@@ -355,21 +364,23 @@ static void gemv_run(rstsr_hip_ctx* ctx, const GemmProblem& P, T alpha, T beta, 
         q.a += i * g.rs;
         q.y += i * g.ys;
         const dim3 grid((uint32_t)((q.M + per - 1) / per), (uint32_t)g.nsplit, nb);
-        auto rows = [&](auto v, auto w) {
+        auto rows = [&](auto v, auto w, auto nt) {
             constexpr int V = decltype(v)::value, W = decltype(w)::value;
-            if (g.xs == 1) hipLaunchKernelGGL((k_gemv_row<T, V, W, true>), grid, blk, 0, ctx->stream, q);
-            else hipLaunchKernelGGL((k_gemv_row<T, V, W, false>), grid, blk, 0, ctx->stream, q);
+            constexpr bool H = decltype(nt)::value;
+            if (g.xs == 1) hipLaunchKernelGGL((k_gemv_row<T, V, W, true, H>), grid, blk, 0, ctx->stream, q);
+            else hipLaunchKernelGGL((k_gemv_row<T, V, W, false, H>), grid, blk, 0, ctx->stream, q);
         };
-        using One = std::integral_constant<int, 1>;
-        using Four = std::integral_constant<int, 4>;
-        using Vec = std::integral_constant<int, V16>;
-        if (row) {
-            if (vec == 1) wpr == 1 ? rows(One{}, One{}) : rows(One{}, Four{});
-            else wpr == 1 ? rows(Vec{}, One{}) : rows(Vec{}, Four{});
-        } else if (vec == 1) {
-            hipLaunchKernelGGL((k_gemv_col<T, 1>), grid, blk, 0, ctx->stream, q);
+        auto wide = [&](auto nt) {
+            if (!row) hipLaunchKernelGGL((k_gemv_col<T, V16, decltype(nt)::value>), grid, blk, 0, ctx->stream, q);
+            else if (wpr == 1) rows(Vec{}, One{}, nt);
+            else rows(Vec{}, Four{}, nt);
+        };
+        if (vec > 1) {
+            if constexpr (V16 > 1) once ? wide(std::true_type{}) : wide(std::false_type{});
+        } else if (row) {
+            wpr == 1 ? rows(One{}, One{}, std::false_type{}) : rows(One{}, Four{}, std::false_type{});
         } else {
-            hipLaunchKernelGGL((k_gemv_col<T, V16>), grid, blk, 0, ctx->stream, q);
+            hipLaunchKernelGGL((k_gemv_col<T, 1, false>), grid, blk, 0, ctx->stream, q);
         }
         check_launch("gemv");
     }

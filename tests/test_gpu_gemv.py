@@ -108,3 +108,19 @@ def test_alpha_beta(dev, dt):
         abi.check(abi.lib().rstsr_hip_gemm(C.c_void_p(dev._ctx_ptr()), rt._code(dt), 0, m, 1, k, al.ctypes.data,
                                            ta.as_ptr(), k, 1, tx.as_ptr(), 1, 1, be.ctypes.data, ty.as_ptr(), 1, 1))
         assert np.array_equal(ty.to_numpy()[:, 0], (2 * product(a, x[:, 0]) - 3 * y[:, 0]).astype(dt)), (m, k)
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+def test_hints_by_size_and_sharing(dev, dt):
+    """Matrices either side of 40 MB, and one matrix shared by all batches: the same exact results."""
+    rng = np.random.default_rng(23)
+    es = np.dtype(dt).itemsize
+    for m in (1 + (30 << 20) // (1000 * es), 1 + (44 << 20) // (1000 * es)):
+        a, x = ints(rng, (m, 1000), dt), ints(rng, 1000, dt)
+        want = (a.real.astype(np.int64) @ x.real.astype(np.int64) if np.dtype(dt).kind != "c" else a @ x).astype(dt)
+        for form in "cf":
+            assert np.array_equal((matrix(dev, a, form) % rt.asarray(x, device=dev)).to_numpy(), want), (m, form)
+    a, x = ints(rng, (300, 77), dt), ints(rng, (5, 77, 1), dt)
+    got = (rt.asarray(a, device=dev).broadcast_to([5, 300, 77]) % rt.asarray(x, device=dev)).to_numpy()
+    assert np.array_equal(got, (a.astype(np.complex128) @ x.astype(np.complex128)).astype(dt) if np.dtype(dt).kind == "c"
+                          else (a.astype(np.int64) @ x.astype(np.int64)).astype(dt))
