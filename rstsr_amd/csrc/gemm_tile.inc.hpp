@@ -289,16 +289,23 @@ static void tile_grouped_run(rstsr_hip_ctx* ctx, const char* tag, const std::vec
         return;
     }
     double mean = 0;
-    int64_t work = 0, tiles = 0;
+    int64_t work = 0, tiles = 0, area128 = 0, area64 = 0;  // areas: tiled outputs times K
     for (auto& p : probs) {
         mean += (double)std::min(p.M, p.N);
         work += p.M * p.N * p.K;
-        tiles += ((p.M + 127) / 128) * ((p.N + 127) / 128);
+        const int64_t t = ((p.M + 127) / 128) * ((p.N + 127) / 128);
+        tiles += t;
+        area128 += 4 * t * p.K;
+        area64 += ((p.M + 63) / 64) * ((p.N + 63) / 64) * p.K;
     }
-    // Enough 128 x 128 tiles to keep every CU busy for many rounds: always the largest tile, which the
+    // Enough 128 x 128 tiles to keep every CU busy for many rounds, and at most a fifth more work in them
+    // than in 64 x 64 ones (512 problems of 32 to 1024: a ninth): always the largest tile, which the
     // tuner's two timed runs at a changing clock miss by a few per cent (ms, 128 x 128 against 64 x 64:
-    // 10700 tiles 2.72 and 2.88, 5000 tiles 1.98 and 2.11; 830 tiles 0.188 and 0.156).
-    if (std::is_same<T, double>::value && tiles >= 16 * (int64_t)std::max(ctx->num_cu, 1)) {
+    // 10700 tiles 2.72 and 2.88, 5000 tiles 1.98 and 2.11; 830 tiles 0.188 and 0.156; with more padding
+    // 4500 problems of 140 1.37 and 0.79, 2500 of 192 1.01 and 0.64, 1200 of 260 1.24 and 1.07, 4500 of 48
+    // 0.122 and 0.084).
+    if (std::is_same<T, double>::value && tiles >= 16 * (int64_t)std::max(ctx->num_cu, 1) &&
+        5 * area128 <= 6 * area64) {
         run(0);
         return;
     }

@@ -42,3 +42,19 @@ def test_complex_symmetric_products_stay_symmetric(dev, dt):
     t = rt.asarray(x, device=dev)
     got = (t.transpose() % t).to_numpy()
     assert np.array_equal(got, got.T)
+
+
+def test_exact_many_small_grouped(dev):
+    """More problems than 16 per CU, nearly empty in 128 x 128 tiles: the tuner's tile shape."""
+    rng = np.random.default_rng(20)
+    probs, want, n0 = [], [], 0
+    out = rt.zeros((4300 * 70 * 70,), device=dev)
+    for _ in range(4300):
+        m, n, k = (int(v) for v in rng.integers(1, 71, size=3))
+        a, b = ints(rng, (m, k), np.float64), ints(rng, (k, n), np.float64)
+        c = out._view(([m, n], [n, 1], n0))
+        probs.append((rt.asarray(a, device=dev), rt.asarray(b, device=dev), c))
+        want.append(a @ b)
+        n0 += m * n
+    rt.gemm_grouped(probs)
+    assert np.array_equal(out.to_numpy()[:n0], np.concatenate([w.ravel() for w in want]))
