@@ -2132,7 +2132,7 @@ void ozaki_gemm_f64(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, doub
 // their own and a last pass combined them: 4096^3 4.31 ms, now 3.65.)
 // Returns false, before anything is enqueued, for forms it does not take: operands whose vectors
 // neither have unit stride and at most 8192 elements nor lie side by side, and planes past
-// Z3_MAX_BYTES, since they are three times those of one real product.
+// Z3_MAX_BYTES or past the memory there is, since they are three times those of one real product.
 // plain(flag, ws): enqueue what computes C when *flag is set, in the planes' place (plain_bytes at ws).
 constexpr size_t Z3_MAX_BYTES = (size_t)32 << 30;
 
@@ -2188,7 +2188,13 @@ bool ozaki_zgemm3(rstsr_hip_ctx* ctx, const GemmProblem& P, double alpha, size_t
     const size_t o_A8 = take(n * planeA), o_B8 = take(n * planeB), o_R = take(n * planeR);
     off = std::max(off, o_A8 + plain_bytes);
     if (off > Z3_MAX_BYTES) return false;
-    char* ws = (char*)workspace(ctx, off);
+    char* ws = nullptr;
+    try {
+        ws = (char*)workspace(ctx, off);
+    } catch (const Error& e) {
+        if (e.kind != ErrorKind::MemoryError) throw;
+        return false;  // the products one by one need less
+    }
     int* flag = (int*)ws;
     int* eA = (int*)(ws + o_eA);
     int* fB = (int*)(ws + o_fB);

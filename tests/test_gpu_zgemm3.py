@@ -89,3 +89,41 @@ def test_captured(dev):
         g.launch()
         want = rt.matmul(rt.asarray(a * scale, device=dev), tb, mode="ozaki").to_numpy()
         assert np.array_equal(out.to_numpy(), want), scale
+
+
+def test_products_one_by_one_where_memory_is_short():
+    """4096^3: the three products at once need 2.1 GB of workspace, one by one 1.65 GB. With 1.8 GB left
+    besides the output the call still runs, with the same bits."""
+    import ctypes as C
+
+    hip = C.CDLL("libamdhip64.so")
+    free, total = C.c_size_t(), C.c_size_t()
+
+    def left():
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    n = 4096
+    rng = np.random.default_rng(5)
+    a = np.resize(rng.normal(size=4099) + 1j * rng.normal(size=4099), (n, n))
+    one, two = rt.DeviceHIP(0), rt.DeviceHIP(0)
+    t1 = rt.asarray(a, device=one)
+    want = rt.matmul(t1, t1, mode="ozaki").to_numpy()
+    t2 = rt.asarray(a, device=two)
+    one.synchronize()
+    out = 16 * n * n
+    rt.empty_cache(one)
+    hogs = []
+    try:
+        for _ in range(4):  # the free memory reported lags behind what is freed
+            spare = left() - out - (1800 << 20)
+            if spare < 32 << 20:
+                break
+            hogs.append(C.c_void_p())
+            assert hip.hipMalloc(C.byref(hogs[-1]), C.c_size_t(spare)) == 0
+        assert 1700 << 20 < left() - out < 1900 << 20
+        got = rt.matmul(t2, t2, mode="ozaki")
+    finally:
+        for h in hogs:
+            assert hip.hipFree(h) == 0
+    assert np.array_equal(got.to_numpy(), want)
