@@ -909,7 +909,7 @@ def allclose(a, b, rtol=1e-5, atol=1e-8, equal_nan=False):
 def gemm_grouped(problems, mode="plain", alpha=1.0, beta=0.0):
     """C_g = alpha * A_g @ B_g + beta * C_g for a list of 2-D (A, B, C) tensors of uneven shapes.
 
-    Plain f64 / c128 run as one persistent launch with autotuned tiles."""
+    Plain f64 / c128 run as one launch per form of the operands (unit strides), with autotuned tiles."""
     import ctypes as C
     from . import abi
 

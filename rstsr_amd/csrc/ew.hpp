@@ -550,10 +550,12 @@ static EwChoice choose(const Dims& d, bool has_a, bool has_b) {
 // Outputs at least this large are written with streaming stores: they cannot
 // stay in the 256 MB last-level cache for a following kernel anyway.
 constexpr uint64_t EW_NT_STORE_MIN = 128ull << 20;
-// The flat kernel's streaming hints: below, its operands were often written just before and lie in
-// the last-level cache, which hinted loads do not use (131 MB: 37 us without, 48 with hints; 410 MB:
-// 152 and 149, exp 132 and 124).
-constexpr uint64_t EW_NT_FLAT_MIN = 256ull << 20;
+// Launches that move at least this much take streaming hints in the flat kernel and where the tiled
+// kernel's tiles are cut. Less fits the last-level cache, where operands often still lie from the call
+// before and which hinted loads do not use; more would push itself out (us, without and with hints:
+// f64 [1000, 15000] + the same, 360 MB, 65 and 58; exp of 180 MB f32 61 and 55, of 122 MB 35 and 38; f32
+// [1000, 30500] + a row, 244 MB, 38 and 48; f64 [4000, 4000] + its transposed like 82 and 68).
+constexpr uint64_t EW_NT_MOVED_MIN = 288ull * 1000 * 1000;
 // Tiled launches moving at least this many bytes have their tile order tuned.
 constexpr uint64_t EW_TUNE_MIN = 32ull << 20;
 
@@ -666,7 +668,10 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
     const bool big = Body::OUT_SIZE > 0 && all * Body::OUT_SIZE >= EW_NT_STORE_MIN;
     int lmask = ((OPS & 1) && once[1] ? 1 : 0) | ((OPS & 2) && once[2] ? 2 : 0);
     const int rows_ntm = !Body::UNARY ? lmask | (big ? 4 : 0) : (lmask == OPS && big ? OPS | 4 : 0);
-    const int flat_ntm = lmask != 0 && all * Body::OUT_SIZE >= EW_NT_FLAT_MIN ? (lmask | 4) : 0;
+    // bytes the launch moves, operands that repeat counted as nothing
+    const uint64_t moved = all * ((lmask & 1 ? sizeof(typename Body::TA) : 0) + (lmask & 2 ? sizeof(typename Body::TB) : 0) +
+                                  Body::OUT_SIZE);
+    const int flat_ntm = lmask != 0 && moved >= EW_NT_MOVED_MIN ? (lmask | 4) : 0;
 
     uint64_t inner = 1;
     for (int i = 0; i + 1 < d.nd; ++i) inner *= d.shape[i];
@@ -733,18 +738,18 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
                     if (i != unit) ok = ok && dd.st[i][k] * (int64_t)es % 128 == 0;
                 return ok;
             };
-            bool whole = lines(0, 0, Body::OUT_SIZE) && dd.shape[0] % 64 == 0 &&
-                         dd.shape[ch.di] % (ES > 8 ? 32 : ES > 4 ? 64 : 128) == 0;
+            bool whole = lines(0, 0, Body::OUT_SIZE);
             if (ch.stage & 1) whole = whole && lines(1, ch.di, sizeof(typename Body::TA));
             if (ch.stage & 2) whole = whole && lines(2, ch.di, sizeof(typename Body::TB));
-            auto tiled = [&](auto cut_c) {
-                constexpr bool CUTL = decltype(cut_c)::value;
-                // tiles (input axis x output axis): 64 x 64 for 8-byte elements, 32 x 64 for 16-byte; for 4-byte and
+            auto tiled = [&](auto cut_c, auto edge_c, auto slim_c) {
+                constexpr bool CUTL = decltype(cut_c)::value, EDGE = decltype(edge_c)::value;
+                // tiles (input axis x output axis): 64 x 64 for 8-byte elements, 32 x 64 for 16-byte (32 x 32 where
+                // the output axis is no longer: c128 [50, 30, 40, 20] 8 us, 12 on the others); for 4-byte and
                 // smaller 128 x 64, of cut lines 64 x 128, since cut output rows cost more than cut input
                 // rows: f32 [333, 509, 255] <- its reverse 87 us from 128 x 64 tiles, 82 from 64 x 128, the whole
                 // lines of the strided [1024, 256, 256] multiply 95 and 100.
                 constexpr int TI = ES > 8 ? 32 : (ES > 4 || CUTL ? 64 : 128);
-                constexpr int TC = ES > 4 || !CUTL ? 64 : 128;
+                constexpr int TC = decltype(slim_c)::value ? 32 : (ES > 4 || !CUTL ? 64 : 128);
                 uint32_t ntc = ceil_div_u32(dd.shape[0], TC);
                 uint32_t nti = ceil_div_u32(dd.shape[ch.di], TI);
                 uint64_t nouter = total / (dd.shape[0] * dd.shape[ch.di]);
@@ -775,21 +780,28 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
                     if (dd.nd <= 3) {
                         const bool lo = ((S & 1) == 0 || once[1]) && ((S & 2) == 0 || once[2]);
                         const int h = lo ? hint : hint & 2;
-                        if constexpr (CUTL) {
-                            if constexpr (WIDE) {
-                                if (h == 3) go(stage, Y{}, std::integral_constant<int, S | 4>{}, Y{});
-                                else if (h == 1) go(stage, Y{}, std::integral_constant<int, S>{}, Y{});
-                                else go(stage, Y{}, std::integral_constant<int, 0>{}, Y{});
-                            } else {
-                                go(stage, Y{}, std::integral_constant<int, 0>{}, Y{});
+                        if constexpr (!EDGE) {
+                            switch (h) {
+                                case 0: go(stage, Y{}, std::integral_constant<int, 0>{}, N{}); break;
+                                case 1: go(stage, Y{}, std::integral_constant<int, S>{}, N{}); break;
+                                case 2: go(stage, Y{}, std::integral_constant<int, 4>{}, N{}); break;
+                                default: go(stage, Y{}, std::integral_constant<int, S | 4>{}, N{}); break;
                             }
-                        } else
-                        switch (h) {
-                            case 0: go(stage, Y{}, std::integral_constant<int, 0>{}, N{}); break;
-                            case 1: go(stage, Y{}, std::integral_constant<int, S>{}, N{}); break;
-                            case 2: go(stage, Y{}, std::integral_constant<int, 4>{}, N{}); break;
-                            default: go(stage, Y{}, std::integral_constant<int, S | 4>{}, N{}); break;
+                            return;
                         }
+                        if constexpr (WIDE || (CUTL && OPS == 3 && S != 3)) {
+                            if (h == 1) {
+                                go(stage, Y{}, std::integral_constant<int, S>{}, Y{});
+                                return;
+                            }
+                        }
+                        if constexpr (WIDE || (!CUTL && S != 3)) {
+                            if (h == 3) {
+                                go(stage, Y{}, std::integral_constant<int, S | 4>{}, Y{});
+                                return;
+                            }
+                        }
+                        go(stage, Y{}, std::integral_constant<int, 0>{}, Y{});
                     } else {
                         go(stage, N{}, std::integral_constant<int, 0>{}, Y{});
                     }
@@ -818,13 +830,16 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
                 };
                 static constexpr Cand WHOLE[] = {{0, 3}, {1, 3}, {2, 3}, {3, 3}};
                 static constexpr Cand CUT[] = {{3, 0}, {1, 0}};
+                static constexpr Cand CUT_BIG[] = {{3, 1}, {1, 1}};  // beside a staged operand one that is not
                 static constexpr Cand CUT16[] = {{1, 3}, {0, 3}, {2, 3}, {3, 3}};
                 constexpr int ncand = !CUTL || WIDE ? 4 : 2;
-                const Cand* cands = !CUTL ? WHOLE : (WIDE ? CUT16 : CUT);
+                const bool far = moved >= EW_NT_MOVED_MIN;
+                const Cand* cands = !CUTL ? WHOLE : (WIDE ? CUT16 : (OPS == 3 && ch.stage != 3 && far ? CUT_BIG : CUT));
                 auto use = [&](int c) {
                     xmap = cands[c].xmap;
                     hint = cands[c].hint;
-                    if ((!CUTL || WIDE) && !big) hint &= 1;  // outputs that the last-level cache can hold are not streamed
+                    if (EDGE && !CUTL && !WIDE) hint = far ? 3 : 0;
+                    else if ((!CUTL || WIDE) && !big) hint &= 1;  // outputs that the last-level cache can hold are not streamed
                     launch();
                 };
                 // The fastest order depends on how the shapes and strides meet the
@@ -845,8 +860,19 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
                     use(0);
                 }
             };
-            if (whole) tiled(std::false_type{});
-            else tiled(std::true_type{});
+            // Whole lines in tiles that end past the matrix: tiles as for whole ones (f32 [100000, 64] + its
+            // transposed like 16 us, on 64 x 128 tiles 27), unless two operands are staged.
+            const bool ragged = dd.shape[0] % 64 != 0 || dd.shape[ch.di] % (ES > 8 ? 32 : ES > 4 ? 64 : 128) != 0;
+            using Y = std::true_type;
+            using N = std::false_type;
+            if (!whole || (ragged && (ch.stage == 3 || Body::OUT_SIZE > 8))) {
+                if constexpr (ES > 8) dd.shape[0] <= 32 ? tiled(Y{}, Y{}, Y{}) : tiled(Y{}, Y{}, N{});
+                else tiled(Y{}, Y{}, N{});
+            } else if (ragged) {
+                tiled(N{}, Y{}, N{});
+            } else {
+                tiled(N{}, N{}, N{});
+            }
         }
         check_launch("elementwise");
     }

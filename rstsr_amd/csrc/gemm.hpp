@@ -50,11 +50,11 @@ __device__ __forceinline__ void tile_coords(uint32_t id, uint32_t tiles_m, uint3
     tn = r / gsz;
 }
 
-// Index t of the lower triangle (diag = 0: i >= j, t = i(i+1)/2 + j; diag = 1:
-// i > j, t = i(i-1)/2 + j) -> (i, j). The floating root is corrected exactly.
-__device__ __forceinline__ void tri_coords(uint32_t t, int diag, uint32_t& i, uint32_t& j) {
-    auto first = [&](uint64_t r) { return diag ? r * (r - 1) / 2 : r * (r + 1) / 2; };
-    uint64_t r = (uint64_t)((diag ? 1.0 + sqrt(1.0 + 8.0 * t) : sqrt(1.0 + 8.0 * t) - 1.0) * 0.5);
+// Index t of the lower triangle (i >= j, t = i(i+1)/2 + j) -> (i, j). The floating root is corrected
+// exactly.
+__device__ __forceinline__ void tri_coords(uint32_t t, uint32_t& i, uint32_t& j) {
+    auto first = [](uint64_t r) { return r * (r + 1) / 2; };
+    uint64_t r = (uint64_t)((sqrt(1.0 + 8.0 * t) - 1.0) * 0.5);
     while (r > 0 && first(r) > t) --r;
     while (first(r + 1) <= t) ++r;
     i = (uint32_t)r;

@@ -480,7 +480,7 @@ __global__ void __launch_bounds__(CF::NT, CF::OCC) k_gemm_tile(TileGemmArgs<T> g
     constexpr int BK = 128 / (int)sizeof(T);
     uint32_t tm, tn;
     if (g.tri) {
-        tri_coords(xcd_remap8(blockIdx.x, g.tiles_m * (g.tiles_m + 1) / 2), 0, tm, tn);
+        tri_coords(xcd_remap8(blockIdx.x, g.tiles_m * (g.tiles_m + 1) / 2), tm, tn);
     } else {
         tile_coords<8>(blockIdx.x, g.tiles_m, g.tiles_n, tm, tn);
     }
