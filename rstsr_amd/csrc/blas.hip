@@ -110,19 +110,34 @@ struct Recip<double> {
 };
 __device__ __forceinline__ bool subnormal(double x) { return __builtin_amdgcn_class(x, 0x90); }
 __device__ __forceinline__ bool subnormal(c128 x) { return subnormal(x.re) || subnormal(x.im); }
-// a / b. Complex: as by Divisor below.
+
+// Complex quotients: a conj(b) / |b|^2, b scaled to parts in [1/2, 1) and below by a power of two 2^k (exact; no
+// overflow of |b|^2), which the quotient is scaled back by.
+template <class T, class R>
+struct Scaled {
+    R br, bi, d;
+    int k;
+    __device__ static Scaled of(T b) {
+        const int k = ilogb2(fmax(fabs(b.re), fabs(b.im)));
+        const R br = ldexp(b.re, -k), bi = ldexp(b.im, -k);
+        return {br, bi, br * br + bi * bi, k};
+    }
+    __device__ static int ilogb2(double m) { return __builtin_amdgcn_frexp_exp(m); }
+    __device__ static int ilogb2(float m) { return __builtin_amdgcn_frexp_expf(m); }
+    __device__ __forceinline__ R re(T a) const { return a.re * br + a.im * bi; }
+    __device__ __forceinline__ R im(T a) const { return a.im * br - a.re * bi; }
+};
+// a / b
 template <class T>
 __device__ __forceinline__ T t_div(T a, T b) {
-    if constexpr (std::is_same<T, c128>::value || std::is_same<T, c64>::value) {
-        const auto m = fmax(fabs(b.re), fabs(b.im));
-        const auto br = b.re / m, bi = b.im / m, d = br * br + bi * bi;
-        return T{(a.re * br + a.im * bi) / d / m, (a.im * br - a.re * bi) / d / m};
+    if constexpr (ElemOf<T>::CX) {
+        const auto s = Scaled<T, typename ElemOf<T>::R>::of(b);
+        return T{ldexp(s.re(a) / s.d, -s.k), ldexp(s.im(a) / s.d, -s.k)};
     } else {
         return a / b;
     }
 }
-// The divisor of one row of the solve. Complex: a conj(b) / |b|^2 with b scaled by its larger part
-// (no overflow for moderate b).
+// The divisor of one row of the solve.
 template <class T>
 struct Divisor {
     Recip<T> s;
@@ -132,18 +147,16 @@ struct Divisor {
 };
 template <class T, class R>
 struct DivisorC {
-    R br, bi;
-    Recip<R> d, s;
-    __device__ static DivisorC of(T b) {
-        const R m = fmax(fabs(b.re), fabs(b.im)), br = b.re / m, bi = b.im / m;
-        return {br, bi, Recip<R>::of(br * br + bi * bi), Recip<R>::of(m)};
+    Scaled<T, R> b;
+    Recip<R> d;
+    __device__ static DivisorC of(T x) {
+        const auto b = Scaled<T, R>::of(x);
+        return {b, Recip<R>::of(b.d)};
     }
     __device__ __forceinline__ T quot(T a) const {
-        return T{s.quot(d.quot(a.re * br + a.im * bi)), s.quot(d.quot(a.im * br - a.re * bi))};
+        return T{ldexp(d.quot(b.re(a)), -b.k), ldexp(d.quot(b.im(a)), -b.k)};
     }
-    __device__ T exact(T a) const {
-        return T{s.exact(d.exact(a.re * br + a.im * bi)), s.exact(d.exact(a.im * br - a.re * bi))};
-    }
+    __device__ T exact(T a) const { return T{ldexp(d.exact(b.re(a)), -b.k), ldexp(d.exact(b.im(a)), -b.k)}; }
 };
 template <>
 struct Divisor<c64> : DivisorC<c64, float> {
@@ -228,10 +241,10 @@ constexpr int TRSM_FPW = TRSM_F / TRSM_NW;   // fragments per wave
 // subtracts block j - 1's share from it (four MFMAs), solves its 16 rows by substitution in the
 // accumulators' own layout and publishes x through LDS; after one barrier the waves subtract
 // T(f, j) x from their fragments below, with the blocks of T loaded a step ahead.
-// Measured: 256 rows x 1600 columns f64 29-37 us; 2000 rows 0.52 ms in all, eight such launches and
+// Measured: 256 rows x 1600 columns f64 37 us; 2000 rows 0.51 ms in all, eight such launches and
 // the updates between them by the GEMM (3.5 ms with 64-row blocks, one thread per column).
 template <class T>
-__global__ void __launch_bounds__(64 * TRSM_NW, sizeof(T) == 16 ? 2 : 4) k_trsm_block(const T* __restrict__ Tm, int64_t trs, int64_t tcs, int unit,
+__global__ void __launch_bounds__(64 * TRSM_NW, sizeof(T) == 16 ? 2 : sizeof(T) == 4 ? 6 : 4) k_trsm_block(const T* __restrict__ Tm, int64_t trs, int64_t tcs, int unit,
                                                             int kb, T* __restrict__ X, int64_t xrs, int64_t xcs,
                                                             int64_t r) {
     using R = typename ElemOf<T>::R;
@@ -330,7 +343,7 @@ __global__ void __launch_bounds__(64 * TRSM_NW, sizeof(T) == 16 ? 2 : 4) k_trsm_
     };
     auto solve = [&](const T (&rf)[4], const typename MM::Acc (&a)[NP], int f) __attribute__((always_inline)) {
         T(&xf)[16][16] = xs[f & 1];
-        constexpr bool NARROW = std::is_same<T, c64>::value;  // not a step ahead: 128 registers are two blocks per CU
+        constexpr bool NARROW = CX;  // not a step ahead: their registers are scarce
         T b[4], d[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {

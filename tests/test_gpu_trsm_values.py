@@ -65,3 +65,19 @@ def test_small_updates_add_up_before_they_are_subtracted(dev, dt, uplo):
         a[0, -m:] = u / 2
         want[0] = 1 - 120 * u
     assert np.array_equal(solve(dev, a, b, LEFT, uplo, NONUNIT), want)
+
+
+@pytest.mark.parametrize("dt", [np.complex64, np.complex128])
+@pytest.mark.parametrize("s", [5, 40])
+def test_complex_quotients(dev, dt, s):
+    """Diagonal solves on both kernels against extended precision, divisors of every magnitude. The parts
+    of a conj(b) are off by 2 u |a||b|, |b|^2 and the quotient by 2 u and u: 2 sqrt(2) u + 3 u < 6 u of |a / b|."""
+    rng = np.random.default_rng(25)
+    u = np.finfo(dt).eps / 2
+    e = 40 if dt == np.complex64 else 300
+    d = (rng.normal(size=s) + 1j * rng.normal(size=s)) * np.exp2(rng.integers(-e, e + 1, size=s))
+    d[::3] = d[::3].real  # one part zero
+    d, b = d.astype(dt), (rng.normal(size=(s, 700)) + 1j * rng.normal(size=(s, 700))).astype(dt)
+    want = b.astype(np.clongdouble) / d.astype(np.clongdouble)[:, None]
+    got = solve(dev, np.diag(d), b, LEFT, LOWER, NONUNIT)
+    assert np.all(np.abs(got - want) <= 6 * u * np.abs(want))
