@@ -22,7 +22,7 @@
 //    stride a unit-stride reduced axis with 16-byte loads, group shuffles combine;
 //  - col: lanes along the outputs on the input's unit-stride kept axis
 //    (coalesced), sequential over a part of the reduced range; few parts are the
-//    waves of one block, many lie one after the other over the threads;
+//    waves of one block, many lie along grid y or one after the other over the threads;
 //  - finalize: combine the split partials of each output in fixed order.
 // Built with -ffp-contract=off so that TwoSum is not fused or reassociated.
 #include <array>
@@ -533,11 +533,12 @@ __global__ void __launch_bounds__(RB) k_red_row(const T* __restrict__ a, typenam
 }
 
 // VEC adjacent outputs per thread along the unit-stride kept axis, sequential over a part of the
-// reduced range. KS = 1: parts one after the other over the threads, partials combined by k_red_fin.
+// reduced range. KS = 1: parts along grid y (a wave's walk is then uniform), or with LIN one after the
+// other over the threads (so that few outputs leave no lanes idle), partials combined by k_red_fin.
 // KS = 16: the waves of a block share its 64 VEC outputs, a part each, combined in order through LDS, so
 // that a reduction with few parts needs no second launch ([64, 128, 256] f64 over axis 1: 16.2 -> 7.7 us
 // in all; which numbers of parts: reduce_plan).
-template <class A, class T, int VEC, int KS>
+template <class A, class T, int VEC, int KS, bool LIN>
 __global__ void __launch_bounds__(KS == 1 ? RB : 64 * KS) k_red_col(const T* __restrict__ a, typename A::Out* out,
                                                 typename A::S* part, RedPlan p) {
     using S = typename A::S;
@@ -546,12 +547,11 @@ __global__ void __launch_bounds__(KS == 1 ? RB : 64 * KS) k_red_col(const T* __r
     __shared__ S red[KS > 1 ? KS : 1][KS > 1 ? 64 * VEC : 1];
     const uint32_t lane = threadIdx.x & 63, wave = KS > 1 ? threadIdx.x >> 6 : 0;
     const uint32_t nv = p.M / VEC;
-    // KS = 1: the parts' outputs side by side, so that few of them leave no lanes idle
     const uint64_t t = KS > 1 ? (uint64_t)blockIdx.x * 64 + lane : (uint64_t)blockIdx.x * RB + threadIdx.x;
-    const uint32_t sp = KS > 1 ? 0 : (uint32_t)(t / nv);
-    const bool active = KS > 1 ? t < nv : sp < p.nsplit;
+    const uint32_t sp = LIN ? (uint32_t)(t / nv) : (KS > 1 ? 0 : blockIdx.y);
+    const bool active = LIN ? sp < p.nsplit : t < nv;
     if (KS == 1 && !active) return;
-    const uint32_t o = active ? (uint32_t)(t - (uint64_t)sp * nv) * VEC : 0;
+    const uint32_t o = active ? (uint32_t)(LIN ? t - (uint64_t)sp * nv : t) * VEC : 0;
     int64_t oin, oout;
     kept_offsets(p, o, oin, oout);
     S acc[VEC];
@@ -857,12 +857,13 @@ static RedSetup reduce_plan(rstsr_hip_ctx* ctx, const Layout& la, const std::vec
         const uint64_t vec = (uint64_t)col_vec(t);
         const uint64_t wpc = (uint64_t)col_waves_per_cu((int)(esize * vec));
         uint64_t want = std::max<uint64_t>(1, ((uint64_t)std::max(ctx->num_cu, 1) * wpc * 64 * vec) / M);
-        uint64_t nsplit = std::min<uint64_t>({want, std::max<uint64_t>(1, R / 64), 65536});
+        uint64_t nsplit = std::min<uint64_t>({want, std::max<uint64_t>(1, R / 64), 65535});
         // Two to six parts: the waves of one block, which saves the second launch. With more parts
         // the outputs are too few blocks to read at full rate (us, parts as blocks against waves of one:
         // f64 128 x 16384 16, 6; 1000 x 32768 53, 44; but 1000 x 5000, 15 parts, 17, 26; c64 3000 x
-        // 8192, 8 parts, 43, 48).
-        p.ks = nsplit > 1 && nsplit <= 6 ? 16 : 1;
+        // 8192, 8 parts, 43, 48). Shorter ranges, not split otherwise, where the outputs alone are a quarter
+        // of the waves wanted or less (f64 64 x 32768 8.9, 6.5; but c64, half of them, 7.9, 10.9).
+        p.ks = (nsplit > 1 && nsplit <= 6) || (R >= 64 && R < 128 && want >= 4 && want <= 16) ? 16 : 1;
         if (p.ks > 1) nsplit = 1;
         p.upw = (R + nsplit * p.ks - 1) / (nsplit * p.ks);
         nsplit = (R + p.upw * p.ks - 1) / (p.upw * p.ks);
@@ -919,15 +920,26 @@ static void run_reduce(rstsr_hip_ctx* ctx, const RedSetup& s, const T* a, typena
         // split covers the same number of lanes as for 8-byte elements
         constexpr int VC = V16 > 2 ? 2 : V16;
         const bool vec = VC > 1 && p.nk >= 1 && p.kin[0] == 1 && p.kshape[0] % VC == 0 && p.M % VC == 0;
-        auto go = [&](auto v, auto ks) {
+        auto go = [&](auto v, auto ks, auto lin) {
             constexpr int V = decltype(v)::value, KS = decltype(ks)::value;
-            hipLaunchKernelGGL((k_red_col<A, T, V, KS>),
-                               dim3(KS == 1 ? ceil_div_u32((uint64_t)(p.M / V) * p.nsplit, RB) : ceil_div_u32(p.M / V, 64)),
-                               dim3(KS == 1 ? RB : 64 * KS), 0, ctx->stream, a, out, part, p);
+            constexpr bool LIN = decltype(lin)::value;
+            const uint64_t nv = p.M / V;
+            const dim3 grid = LIN ? dim3(ceil_div_u32(nv * p.nsplit, RB))
+                                  : dim3(ceil_div_u32(nv, KS == 1 ? RB : 64), p.nsplit);
+            hipLaunchKernelGGL((k_red_col<A, T, V, KS, LIN>), grid, dim3(KS == 1 ? RB : 64 * KS), 0, ctx->stream, a, out, part,
+                               p);
         };
         auto by_ks = [&](auto v) {
-            if (p.ks == 1) go(v, std::integral_constant<int, 1>{});
-            else go(v, std::integral_constant<int, 16>{});
+            using One = std::integral_constant<int, 1>;
+            // Parts along grid y round the outputs up to whole blocks, which may give a few CUs one block
+            // more than the others: long reductions then wait for those (us, along y against packed: f64 20000
+            // x 1000 40, 32, 20000 x 500 26, 23, 200000 x 40 34, 30; but 1000 x 130 9.8, 12.6, 4000 x 500 12, 13).
+            const uint64_t blocks = (uint64_t)ceil_div_u32(p.M / decltype(v)::value, RB) * p.nsplit;
+            const bool lin = p.nsplit > 1 && blocks > (uint64_t)std::max(ctx->num_cu, 1) &&
+                             (uint64_t)p.M * p.R * sizeof(T) >= (24u << 20);
+            if (p.ks > 1) go(v, std::integral_constant<int, 16>{}, std::false_type{});
+            else if (lin) go(v, One{}, std::true_type{});
+            else go(v, One{}, std::false_type{});
         };
         if (vec) by_ks(std::integral_constant<int, VC>{});
         else by_ks(std::integral_constant<int, 1>{});
