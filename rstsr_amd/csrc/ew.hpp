@@ -671,7 +671,9 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
     // bytes the launch moves, operands that repeat counted as nothing
     const uint64_t moved = all * ((lmask & 1 ? sizeof(typename Body::TA) : 0) + (lmask & 2 ? sizeof(typename Body::TB) : 0) +
                                   Body::OUT_SIZE);
-    const int flat_ntm = lmask != 0 && moved >= EW_NT_MOVED_MIN ? (lmask | 4) : 0;
+    bool twice = false;  // both operands in one buffer: mostly the same elements, read twice (x * x)
+    if constexpr (OPS == 3) twice = (const void*)body.a == (const void*)body.b;
+    const int flat_ntm = lmask != 0 && !twice && moved >= EW_NT_MOVED_MIN ? (lmask | 4) : 0;
 
     uint64_t inner = 1;
     for (int i = 0; i + 1 < d.nd; ++i) inner *= d.shape[i];
@@ -731,16 +733,21 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
         } else if constexpr (TILED && OPS != 0) {
             constexpr size_t ES = sizeof(typename Body::TA) > sizeof(typename Body::TB) ? sizeof(typename Body::TA)
                                                                                           : sizeof(typename Body::TB);
-            // whole lines: the output's rows along dim 0 and the staged inputs' rows along the input axis
+            // whole lines: the output's rows along dim 0 and the staged inputs' rows along the input axis; halves
+            // of 128-byte lines pass too, but for 4-byte elements, whose tiles differ (us, as whole and as cut
+            // lines: f64 [300, 400, 200] <- another order of its axes, 384 MB, 68 and 81; [10008, 2024] + its
+            // transposed like 77 and 107; f32 [16, 500, 500] 13.5 and 9.2)
+            constexpr int64_t LINE = ES > 4 ? 64 : 128;
             auto lines = [&](int k, int unit, size_t es) {
-                bool ok = dd.off[k] * (int64_t)es % 128 == 0 && dd.shape[unit] * es % 128 == 0;
+                bool ok = dd.off[k] * (int64_t)es % LINE == 0 && dd.shape[unit] * es % LINE == 0;
                 for (int i = 0; i < dd.nd; ++i)
-                    if (i != unit) ok = ok && dd.st[i][k] * (int64_t)es % 128 == 0;
+                    if (i != unit) ok = ok && dd.st[i][k] * (int64_t)es % LINE == 0;
                 return ok;
             };
             bool whole = lines(0, 0, Body::OUT_SIZE);
             if (ch.stage & 1) whole = whole && lines(1, ch.di, sizeof(typename Body::TA));
             if (ch.stage & 2) whole = whole && lines(2, ch.di, sizeof(typename Body::TB));
+            const bool far = moved >= EW_NT_MOVED_MIN;
             auto tiled = [&](auto cut_c, auto edge_c, auto slim_c) {
                 constexpr bool CUTL = decltype(cut_c)::value, EDGE = decltype(edge_c)::value;
                 // tiles (input axis x output axis): 64 x 64 for 8-byte elements, 32 x 64 for 16-byte (32 x 32 where
@@ -833,7 +840,6 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
                 static constexpr Cand CUT_BIG[] = {{3, 1}, {1, 1}};  // beside a staged operand one that is not
                 static constexpr Cand CUT16[] = {{1, 3}, {0, 3}, {2, 3}, {3, 3}};
                 constexpr int ncand = !CUTL || WIDE ? 4 : 2;
-                const bool far = moved >= EW_NT_MOVED_MIN;
                 const Cand* cands = !CUTL ? WHOLE : (WIDE ? CUT16 : (OPS == 3 && ch.stage != 3 && far ? CUT_BIG : CUT));
                 auto use = [&](int c) {
                     xmap = cands[c].xmap;
@@ -860,12 +866,14 @@ static void launch_ew(rstsr_hip_ctx* ctx, const Body& body, Dims d, EwChoice ch,
                     use(0);
                 }
             };
-            // Whole lines in tiles that end past the matrix: tiles as for whole ones (f32 [100000, 64] + its
-            // transposed like 16 us, on 64 x 128 tiles 27), unless two operands are staged.
+            // Whole lines in tiles that end past the matrix: tiles as for whole ones, unless two operands are
+            // staged. 4-byte elements only where the output axis would not fill the tiles for cut lines (f32
+            // [100000, 64] + its transposed like 16 us, 27 on 64 x 128) or the launch is large enough for hints
+            // ([8000, 4000] 68 and 109; but [64, 100000] <- its transposed like 10.6 and 8.8).
             const bool ragged = dd.shape[0] % 64 != 0 || dd.shape[ch.di] % (ES > 8 ? 32 : ES > 4 ? 64 : 128) != 0;
             using Y = std::true_type;
             using N = std::false_type;
-            if (!whole || (ragged && (ch.stage == 3 || Body::OUT_SIZE > 8))) {
+            if (!whole || (ragged && (ch.stage == 3 || Body::OUT_SIZE > 8 || (ES <= 4 && !far && dd.shape[0] > 64)))) {
                 if constexpr (ES > 8) dd.shape[0] <= 32 ? tiled(Y{}, Y{}, Y{}) : tiled(Y{}, Y{}, N{});
                 else tiled(Y{}, Y{}, N{});
             } else if (ragged) {
