@@ -111,8 +111,8 @@ struct Recip<double> {
 __device__ __forceinline__ bool subnormal(double x) { return __builtin_amdgcn_class(x, 0x90); }
 __device__ __forceinline__ bool subnormal(c128 x) { return subnormal(x.re) || subnormal(x.im); }
 
-// Complex quotients: a conj(b) / |b|^2, b scaled to parts in [1/2, 1) and below by a power of two 2^k (exact; no
-// overflow of |b|^2), which the quotient is scaled back by.
+// Complex quotients: a conj(b) / |b|^2, b scaled by a power of two 2^k so that its larger part lies in
+// [1/2, 1) (exact; no overflow of |b|^2), and the quotient scaled back.
 template <class T, class R>
 struct Scaled {
     R br, bi, d;
@@ -237,16 +237,20 @@ constexpr int TRSM_FPW = TRSM_F / TRSM_NW;   // fragments per wave
 // What bounds it: the chain over the rows (a column's x[i] needs every x before it), so all of it
 // runs in one launch and each step is kept short. A block owns 16 columns of X, which are
 // independent of all others: r / 16 blocks without any exchange. X stays in registers, its updates in
-// the matrix cores' accumulators, fragment f (rows 16 f ..) in wave f % 8. Step j: the wave that owns fragment j
-// subtracts block j - 1's share from it (four MFMAs), solves its 16 rows by substitution in the
-// accumulators' own layout and publishes x through LDS; after one barrier the waves subtract
+// the matrix cores' accumulators, fragment f (rows 16 f ..) in wave f % 8. Step j: the wave that owns
+// fragment j subtracts block j - 1's share from it (four MFMAs), solves its 16 rows by substitution in
+// the accumulators' own layout and publishes x through LDS; after one barrier the waves subtract
 // T(f, j) x from their fragments below, with the blocks of T loaded a step ahead.
 // Measured: 256 rows x 1600 columns f64 37 us; 2000 rows 0.51 ms in all, eight such launches and
 // the updates between them by the GEMM (3.5 ms with 64-row blocks, one thread per column).
+// TRSM_OCC waves per SIMD: three blocks per CU (f32), two (f64, c64), one (c128: its LDS).
 template <class T>
-__global__ void __launch_bounds__(64 * TRSM_NW, sizeof(T) == 16 ? 2 : sizeof(T) == 4 ? 6 : 4) k_trsm_block(const T* __restrict__ Tm, int64_t trs, int64_t tcs, int unit,
-                                                            int kb, T* __restrict__ X, int64_t xrs, int64_t xcs,
-                                                            int64_t r) {
+constexpr int TRSM_OCC = sizeof(T) == 16 ? 2 : sizeof(T) == 4 ? 6 : 4;
+
+template <class T>
+__global__ void __launch_bounds__(64 * TRSM_NW, TRSM_OCC<T>)
+    k_trsm_block(const T* __restrict__ Tm, int64_t trs, int64_t tcs, int unit, int kb, T* __restrict__ X, int64_t xrs,
+                 int64_t xcs, int64_t r) {
     using R = typename ElemOf<T>::R;
     using MM = Mma<R>;
     constexpr bool CX = ElemOf<T>::CX;
